@@ -340,12 +340,15 @@ int nsa_range_dq_cw(const void* q, const void* dout, const void* kc, const void*
 
 /* Backward dK/dV of the range branches (key-outer; the key-side half of
  * _range_attn_bwd_qtiled_kernel).  coff / dot: row offsets and deltas from
- * nsa_bwd_prep.  dk/dv float32 [B][Hkv][Lk][D], every key written.  The
- * window has one writer per key.  Compression splits each key's queries into
- * chunks: with dkdv_part (nullable, part_bytes >=
- * nsa_range_dkdv_partial_bytes for the same stream's device) the chunks write
- * partial rows that one more launch sums in chunk order (bit-identical run
- * to run); without it they merge with float atomics into zero-filled dk/dv. */
+ * nsa_bwd_prep.  dk/dv float32 [B][Hkv][Lk][D], every key written.
+ * Compression splits each key's queries into chunks: with dkdv_part
+ * (nullable, part_bytes >= nsa_range_dkdv_partial_bytes for the same stream's
+ * device) the chunks write partial rows that one more launch sums in chunk
+ * order (bit-identical run to run); without it they merge with float atomics
+ * into zero-filled dk/dv.  The window has one writer per key, or, where the
+ * key blocks alone would leave CUs idle and dkdv_part has room, its queries
+ * in parts that are summed the same way (nsa_range_dkdv_partial_bytes with
+ * cmp_block = the window, cmp_stride = 1; 0: not split). */
 size_t nsa_range_dkdv_partial_bytes(int mode, int B, int Hkv, int T, int Lk, int D, int cmp_block, int cmp_stride,
                                     void* stream);
 int nsa_range_dkdv(int mode, const void* q, const void* k, const void* v, const void* dout, const float* coff,

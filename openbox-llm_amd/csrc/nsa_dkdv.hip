@@ -18,9 +18,11 @@
 // serves both and the S / dP accumulators line up with the operand slots.
 // Tiles whose two queries see all 32 keys of a wave skip the per-element mask.
 //
-//   * window      : a workgroup owns 32*NW keys and walks queries [k0, k0 + 32 NW + w - 2].
-//   * compression : same, over query chunks of kCmpChunk; chunks merge with
-//                   float atomics; the key blocks of one chunk share an XCD.
+//   * window      : a workgroup owns 32*NW keys and walks queries [k0, k0 + 32 NW + w - 2], or a
+//                   part of them where the key blocks alone leave CUs idle (win_split).
+//   * compression : same, over query chunks of kCmpChunk; the key blocks of one chunk share an XCD.
+//   Parts and chunks write partial rows that k_range_dkdv_reduce sums (or, without a
+//   partial buffer, the chunks merge with float atomics and the window is not split).
 //   For 16-bit operands both run the role-split walk (kv_walk's work on two
 //   waves per 32 keys, two waves per SIMD; below).
 //   * selection   : work items (block, chunk of its CSR query list) built by
@@ -753,6 +755,26 @@ template <typename T, int D, int NTH> struct FlatReq {
   }
 };
 
+// FlatReq's tiles as a tile source of kv_walk (one head chunk; the requests
+// come in tile order).
+template <typename T, int D, int NTH> struct FlatTiles {
+  struct Info {
+    int it;
+  };
+  FlatReq<T, D, NTH> rq;
+  int rlo, rhi, key, kw, window, cl, cd, h;
+  bool key_ok;
+  __device__ __forceinline__ void prepare(int, int) {}
+  __device__ __forceinline__ void issue(KvStage<T, D>& s, int, int) { rq.request(s); }
+  __device__ __forceinline__ Info info(const KvStage<T, D>&, int ti) const { return Info{ti}; }
+  __device__ __forceinline__ VisBits vis(const Info& i, bool& mask) const {
+    const int R0 = rlo + 32 * i.it;
+    mask = flat_tile_needs_mask(kw, R0, rhi, rq.G, window, cl, cd);
+    const uint32_t bits = key_ok ? flat_rows_seeing(key, R0, rq.G, window, cl, cd) : 0u;
+    return VisBits{bits >> (8 * h)};
+  }
+};
+
 // One walk per role (the roles' registers are then never live at once).
 // Per tile: [role work before the barrier]; wait for tile it+1; barrier;
 // [role work after it]; refill the stage of tile it.  P goes through
@@ -928,129 +950,153 @@ __device__ __forceinline__ void zero_rows(float* dkrow, float* dvrow, int h) {
 }
 
 // ---------------------------------------------------------------------------
-// range dK/dV: window: ceil(Lk / (32 NW)) * B*Hkv workgroups.  Compression:
-// every (query chunk, key block) pair takes about as long as any other, so a
-// grid of them would end in a partial round of workgroups on an otherwise idle
-// GPU.  Chunks from `chs` on are split into `spl` sub-chunks and launched
-// last, where their short workgroups fill that round.  Logical workgroups
-// (placed on the XCDs by xcd_remap_split):
+// Work of a range dK/dV launch.  Window: ceil(Lk / (32 NW)) key blocks per bh,
+// the queries of each in `spl` equal parts (win_split).  Compression: every
+// (query chunk, key block) pair takes about as long as any other, so a grid
+// of them would end in a partial round of workgroups on an otherwise idle GPU.
+// Chunks from `chs` on are split into `spl` sub-chunks and launched last,
+// where their short workgroups fill that round.  Logical workgroups (placed
+// on the XCDs by xcd_remap_split):
 //   [0, nbh * big)  chunks < chs, per bh chunk-major
 //   the rest        chunks >= chs, per bh (chunk, sub-chunk)-major
 // (big / small: cmp_blocks_range over the two chunk ranges).
 // ---------------------------------------------------------------------------
-template <typename T, int D, int NW>
+struct KvRange {
+  int mode, T_, Lk, chunk, window, cl, cd, nbh, chs, spl;
+};
+struct KvWork {
+  int64_t wg;     // logical workgroup: its 32 NW rows of the partial buffer
+  int bh, k0;     // (b, hkv) and first key
+  int tlo, thi;   // its queries (tlo > thi: none)
+};
+template <int NW> __device__ __forceinline__ KvWork kv_work(const KvRange& r) {
+  KvWork x;
+  x.wg = blockIdx.x;
+  const int nkb = (r.Lk + 32 * NW - 1) / (32 * NW);
+  if (r.mode == NSA_MODE_COMPRESS) {
+    const int nch = (r.T_ + r.chunk - 1) / r.chunk;
+    const int big = cmp_blocks_range(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, 0, r.chs);
+    const int per = cmp_blocks_range(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, r.chs, nch) * r.spl;
+    x.wg = xcd_remap_split(blockIdx.x, (int64_t)big * r.nbh, (int64_t)per * r.nbh);
+    int i, ch, sub = 0, qlen = r.chunk;
+    if (x.wg < (int64_t)big * r.nbh) {
+      x.bh = (int)(x.wg / big);
+      i = (int)(x.wg % big);
+      for (ch = 0; ch < r.chs - 1; ++ch) {   // chunk ch holds the first cmp_active_blocks(.., ch) key blocks
+        const int nb = cmp_active_blocks(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, ch);
+        if (i < nb) break;
+        i -= nb;
+      }
+    } else {
+      const int64_t w2 = x.wg - (int64_t)big * r.nbh;
+      x.bh = (int)(w2 / per);
+      i = (int)(w2 % per);
+      for (ch = r.chs; ch < nch - 1; ++ch) {
+        const int nb = cmp_active_blocks(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, ch) * r.spl;
+        if (i < nb) break;
+        i -= nb;
+      }
+      const int nb = cmp_active_blocks(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, ch);
+      sub = i / nb;
+      i %= nb;
+      qlen = (r.chunk + r.spl - 1) / r.spl;
+    }
+    x.k0 = i * 32 * NW;
+    const int q0 = ch * r.chunk + sub * qlen;
+    if (q0 + qlen > ch * r.chunk + r.chunk) qlen = ch * r.chunk + r.chunk - q0;
+    x.tlo = x.k0 * r.cd + r.cl - 1;
+    x.tlo = x.tlo > q0 ? x.tlo : q0;
+    x.thi = q0 + qlen - 1;
+  } else {
+    const int sub = (int)(x.wg % r.spl);
+    const int64_t kb = x.wg / r.spl;
+    x.k0 = (int)(kb % nkb) * 32 * NW;
+    x.bh = (int)(kb / nkb);
+    const int klast = x.k0 + 32 * NW - 1 < r.Lk - 1 ? x.k0 + 32 * NW - 1 : r.Lk - 1;
+    const int win = r.window < r.T_ ? r.window : r.T_;   // a longer window sees no more
+    const int last = klast + win - 1;
+    const int len = (32 * NW + win - 1 + r.spl - 1) / r.spl;
+    x.tlo = x.k0 + sub * len;
+    x.thi = r.spl > 1 && x.tlo + len - 1 < last ? x.tlo + len - 1 : last;
+  }
+  x.thi = x.thi < r.T_ - 1 ? x.thi : r.T_ - 1;
+  return x;
+}
+
+// The single-role walk (float inputs).  FLAT: the query tiles are 32
+// consecutive rows t G + g of the group (groups of G < 16 heads), else two
+// queries x 16 heads of a head chunk.  A float tile is bound by its MFMAs
+// (32x32x2: 8192 cycles for the tile's four products at D = 64), so rows that
+// do not exist cost as much as rows that do.
+template <typename T, int D, int NW, bool FLAT>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void k_range_dkdv32(int mode, const T* __restrict__ q, const T* __restrict__ dout, const float* __restrict__ coff,
-                    const float* __restrict__ dot, const T* __restrict__ k, const T* __restrict__ v,
-                    float* __restrict__ dk, float* __restrict__ dv, float* __restrict__ part, int64_t part_half,
-                    int Hq, int Hkv, int T_, int Lk, int chunk, int window, int cl, int cd, int nbh, int chs, int spl,
-                    float sl2, float scale) {
+void k_range_dkdv32(const KvRange r, const T* __restrict__ q, const T* __restrict__ dout,
+                    const float* __restrict__ coff, const float* __restrict__ dot, const T* __restrict__ k,
+                    const T* __restrict__ v, float* __restrict__ dk, float* __restrict__ dv, float* __restrict__ part,
+                    int64_t part_half, int Hq, int Hkv, float sl2, float scale) {
   constexpr int NTH = 64 * NW;
   __shared__ __align__(16) KvStage<T, D> stg[kKvStages];
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, n = lane & 31;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: its masks branch
-  // 1-D grid over the (key block, query chunk) pairs that have work, per bh,
-  // chunk-major: the workgroups of one chunk (which stream the same queries)
-  // are consecutive, and XCD x takes a contiguous, equal share of them.  The
-  // window has one chunk and uniform work per key block.
-  const int nkb = (Lk + 32 * NW - 1) / (32 * NW);
-  int kblk, ch, bh;
-  int q0 = 0, qlen = chunk;   // compression: the workgroup's queries [q0, q0 + qlen)
-  int64_t wg = blockIdx.x;    // logical workgroup (compression: its rows of the partial buffer)
-  if (mode == NSA_MODE_COMPRESS) {
-    const int nch = (T_ + chunk - 1) / chunk;
-    const int big = cmp_blocks_range(T_, Lk, chunk, NW, cl, cd, 0, chs);
-    const int per = cmp_blocks_range(T_, Lk, chunk, NW, cl, cd, chs, nch) * spl;
-    wg = xcd_remap_split(blockIdx.x, (int64_t)big * nbh, (int64_t)per * nbh);
-    int r, sub = 0;
-    if (wg < (int64_t)big * nbh) {
-      bh = (int)(wg / big);
-      r = (int)(wg % big);
-      for (ch = 0; ch < chs - 1; ++ch) {   // chunk ch holds the first cmp_active_blocks(.., ch) key blocks
-        const int nb = cmp_active_blocks(T_, Lk, chunk, NW, cl, cd, ch);
-        if (r < nb) break;
-        r -= nb;
-      }
-    } else {
-      const int64_t w2 = wg - (int64_t)big * nbh;
-      bh = (int)(w2 / per);
-      r = (int)(w2 % per);
-      for (ch = chs; ch < nch - 1; ++ch) {
-        const int nb = cmp_active_blocks(T_, Lk, chunk, NW, cl, cd, ch) * spl;
-        if (r < nb) break;
-        r -= nb;
-      }
-      const int nb = cmp_active_blocks(T_, Lk, chunk, NW, cl, cd, ch);
-      sub = r / nb;
-      r %= nb;
-      qlen = (chunk + spl - 1) / spl;
-    }
-    kblk = r;
-    q0 = ch * chunk + sub * qlen;
-    if (q0 + qlen > ch * chunk + chunk) qlen = ch * chunk + chunk - q0;
-  } else {
-    kblk = (int)(blockIdx.x % nkb);
-    ch = 0;
-    bh = (int)(blockIdx.x / nkb);
-  }
-  const int b = bh / Hkv, hkv = bh % Hkv;
-  const int k0 = kblk * 32 * NW;
-  const int kw = k0 + 32 * w;
+  const KvWork wk = kv_work<NW>(r);
+  const int b = wk.bh / Hkv, hkv = wk.bh % Hkv;
+  const int kw = wk.k0 + 32 * w;
   const int key = kw + n;
-  const bool key_ok = key < Lk;
-  const QSide<T> x = qside<T, D>(q, dout, coff, dot, Hq, Hkv, T_, false);
-  // query range of the workgroup
-  int tlo, thi;
-  const int klast = k0 + 32 * NW - 1 < Lk - 1 ? k0 + 32 * NW - 1 : Lk - 1;
-  if (mode == NSA_MODE_WINDOW) {
-    tlo = k0;
-    thi = klast + window - 1;
-  } else {
-    tlo = k0 * cd + cl - 1;
-    thi = T_ - 1;
-    const int c0 = q0, c1 = q0 + qlen - 1;
-    tlo = tlo > c0 ? tlo : c0;
-    thi = thi < c1 ? thi : c1;
-  }
-  thi = thi < T_ - 1 ? thi : T_ - 1;
-  // compression with a partial buffer: this workgroup's 32 NW rows of it
-  // (every logical workgroup writes them, zeros when it has no query)
-  float* prow = part != nullptr && mode == NSA_MODE_COMPRESS ? part + (wg * 32 * NW + (key - k0)) * D : nullptr;
-  if (tlo > thi) {   // uniform over the workgroup
+  const bool key_ok = key < r.Lk;
+  const QSide<T> x = qside<T, D>(q, dout, coff, dot, Hq, Hkv, r.T_, false);
+  // with a partial buffer: this workgroup's 32 NW rows of it (every logical
+  // workgroup writes them, zeros when it has no query)
+  float* prow = part != nullptr ? part + (wk.wg * 32 * NW + (key - wk.k0)) * D : nullptr;
+  if (wk.tlo > wk.thi) {   // uniform over the workgroup
     if (prow != nullptr && key_ok) zero_rows<D>(prow, prow + part_half, h);
     return;
   }
   KeyAcc<T, D> acc;
-  const int64_t kvoff = (int64_t)bh * Lk * D;
-  acc.init(k + kvoff, v + kvoff, key_ok ? key : Lk - 1, h);
-  const int ntile = (thi - tlo) / 2 + 1;
-  const int wlast = kw + 31;   // last key of the wave (may pass Lk: those columns are never stored)
-  auto qsrc = [&](int i, int& tA, int& tB, int& sA, int& sB) {
-    tA = tlo + 2 * i;
-    tB = tA + 1 <= thi ? tA + 1 : -1;
-    sA = sB = 0;
-  };
-  auto vis = [&](int tA, int tB, bool& mask, bool& visA, bool& visB) {
-    const int tb = tB >= 0 ? tB : tA;
-    if (mode == NSA_MODE_WINDOW) {
-      mask = !(tA >= wlast && tb - window < kw);
-      visA = key <= tA && key > tA - window;
-      visB = key <= tb && key > tb - window;
-    } else {
-      mask = !(wlast * cd + cl - 1 <= tA);
-      visA = key * cd + cl - 1 <= tA;
-      visB = key * cd + cl - 1 <= tb;
-    }
-  };
+  const int64_t kvoff = (int64_t)wk.bh * r.Lk * D;
+  acc.init(k + kvoff, v + kvoff, key_ok ? key : r.Lk - 1, h);
   auto no_pre = [](const Frag<T>*, int) {};
   auto no_post = [](const auto&, int, int) {};
-  auto tiles = pair_tiles<T, D, NTH>(x, b, hkv, qsrc, vis);
-  kv_walk<false, 0, T, D, NTH>(acc, stg, tiles, x.NHC, ntile, no_pre, no_post, sl2, tid);
+  if constexpr (FLAT) {
+    FlatTiles<T, D, NTH> tiles;
+    tiles.rlo = wk.tlo * x.G;
+    tiles.rhi = wk.thi * x.G + x.G - 1;
+    tiles.rq.init(x, b, hkv, tiles.rlo, wk.thi, tid);
+    tiles.key = key;
+    tiles.kw = kw;
+    tiles.window = r.mode == NSA_MODE_WINDOW ? r.window : 0;
+    tiles.cl = r.cl;
+    tiles.cd = r.cd;
+    tiles.h = h;
+    tiles.key_ok = key_ok;
+    kv_walk<false, 0, T, D, NTH>(acc, stg, tiles, 1, (tiles.rhi - tiles.rlo) / 32 + 1, no_pre, no_post, sl2, tid);
+  } else {
+    const int ntile = (wk.thi - wk.tlo) / 2 + 1;
+    const int wlast = kw + 31;   // last key of the wave (may pass Lk: those columns are never stored)
+    auto qsrc = [&](int i, int& tA, int& tB, int& sA, int& sB) {
+      tA = wk.tlo + 2 * i;
+      tB = tA + 1 <= wk.thi ? tA + 1 : -1;
+      sA = sB = 0;
+    };
+    auto vis = [&](int tA, int tB, bool& mask, bool& visA, bool& visB) {
+      const int tb = tB >= 0 ? tB : tA;
+      if (r.mode == NSA_MODE_WINDOW) {
+        mask = !(tA >= wlast && tb - r.window < kw);
+        visA = key <= tA && key > tA - r.window;
+        visB = key <= tb && key > tb - r.window;
+      } else {
+        mask = !(wlast * r.cd + r.cl - 1 <= tA);
+        visA = key * r.cd + r.cl - 1 <= tA;
+        visB = key * r.cd + r.cl - 1 <= tb;
+      }
+    };
+    auto tiles = pair_tiles<T, D, NTH>(x, b, hkv, qsrc, vis);
+    kv_walk<false, 0, T, D, NTH>(acc, stg, tiles, x.NHC, ntile, no_pre, no_post, sl2, tid);
+  }
   if (key_ok) {
     if (prow != nullptr)
       acc.write(prow, prow + part_half, scale, false, h);
     else
-      acc.write(dk + kvoff + (int64_t)key * D, dv + kvoff + (int64_t)key * D, scale, mode == NSA_MODE_COMPRESS, h);
+      acc.write(dk + kvoff + (int64_t)key * D, dv + kvoff + (int64_t)key * D, scale, r.mode == NSA_MODE_COMPRESS, h);
   }
 }
 
@@ -1083,11 +1129,10 @@ __device__ __forceinline__ void store_rows(const f32x16 (&acc)[Tile32<T, D>::DT]
 // of G < 16 heads), else two queries x 16 heads of a head chunk (SplitReq).
 template <typename T, int D, int NW, bool FLAT>
 __global__ __launch_bounds__(128 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void k_range_dkdv_split(int mode, const T* __restrict__ q, const T* __restrict__ dout, const float* __restrict__ coff,
-                    const float* __restrict__ dot, const T* __restrict__ k, const T* __restrict__ v,
-                    float* __restrict__ dk, float* __restrict__ dv, float* __restrict__ part, int64_t part_half,
-                    int Hq, int Hkv, int T_, int Lk, int chunk, int window, int cl, int cd, int nbh, int chs, int spl,
-                    float sl2, float scale) {
+void k_range_dkdv_split(const KvRange r, const T* __restrict__ q, const T* __restrict__ dout,
+                        const float* __restrict__ coff, const float* __restrict__ dot, const T* __restrict__ k,
+                        const T* __restrict__ v, float* __restrict__ dk, float* __restrict__ dv,
+                        float* __restrict__ part, int64_t part_half, int Hq, int Hkv, float sl2, float scale) {
   constexpr int NTH = 128 * NW;
   __shared__ __align__(16) KvStage<T, D> stg[kSplitStages];
   __shared__ __align__(16) PTile pbuf[NW][2];
@@ -1095,81 +1140,24 @@ void k_range_dkdv_split(int mode, const T* __restrict__ q, const T* __restrict__
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool pwave = wv < NW;
   const int w = pwave ? wv : wv - NW;   // key group (wave-uniform: its masks branch)
-  // 1-D grid over the (key block, query chunk) pairs that have work, per bh,
-  // chunk-major: the workgroups of one chunk (which stream the same queries)
-  // are consecutive, and XCD x takes a contiguous, equal share of them.  The
-  // window has one chunk and uniform work per key block.
-  const int nkb = (Lk + 32 * NW - 1) / (32 * NW);
-  int kblk, ch, bh;
-  int q0 = 0, qlen = chunk;   // compression: the workgroup's queries [q0, q0 + qlen)
-  int64_t wg = blockIdx.x;    // logical workgroup (compression: its rows of the partial buffer)
-  if (mode == NSA_MODE_COMPRESS) {
-    const int nch = (T_ + chunk - 1) / chunk;
-    const int big = cmp_blocks_range(T_, Lk, chunk, NW, cl, cd, 0, chs);
-    const int per = cmp_blocks_range(T_, Lk, chunk, NW, cl, cd, chs, nch) * spl;
-    wg = xcd_remap_split(blockIdx.x, (int64_t)big * nbh, (int64_t)per * nbh);
-    int r, sub = 0;
-    if (wg < (int64_t)big * nbh) {
-      bh = (int)(wg / big);
-      r = (int)(wg % big);
-      for (ch = 0; ch < chs - 1; ++ch) {   // chunk ch holds the first cmp_active_blocks(.., ch) key blocks
-        const int nb = cmp_active_blocks(T_, Lk, chunk, NW, cl, cd, ch);
-        if (r < nb) break;
-        r -= nb;
-      }
-    } else {
-      const int64_t w2 = wg - (int64_t)big * nbh;
-      bh = (int)(w2 / per);
-      r = (int)(w2 % per);
-      for (ch = chs; ch < nch - 1; ++ch) {
-        const int nb = cmp_active_blocks(T_, Lk, chunk, NW, cl, cd, ch) * spl;
-        if (r < nb) break;
-        r -= nb;
-      }
-      const int nb = cmp_active_blocks(T_, Lk, chunk, NW, cl, cd, ch);
-      sub = r / nb;
-      r %= nb;
-      qlen = (chunk + spl - 1) / spl;
-    }
-    kblk = r;
-    q0 = ch * chunk + sub * qlen;
-    if (q0 + qlen > ch * chunk + chunk) qlen = ch * chunk + chunk - q0;
-  } else {
-    kblk = (int)(blockIdx.x % nkb);
-    ch = 0;
-    bh = (int)(blockIdx.x / nkb);
-  }
-  const int b = bh / Hkv, hkv = bh % Hkv;
-  const int k0 = kblk * 32 * NW;
-  const int kw = k0 + 32 * w;
+  const KvWork wk = kv_work<NW>(r);
+  const int b = wk.bh / Hkv, hkv = wk.bh % Hkv;
+  const int kw = wk.k0 + 32 * w;
   const int key = kw + n;
-  const bool key_ok = key < Lk;
-  const QSide<T> x = qside<T, D>(q, dout, coff, dot, Hq, Hkv, T_, false);
-  // query range of the workgroup
-  int tlo, thi;
-  const int klast = k0 + 32 * NW - 1 < Lk - 1 ? k0 + 32 * NW - 1 : Lk - 1;
-  if (mode == NSA_MODE_WINDOW) {
-    tlo = k0;
-    thi = klast + window - 1;
-  } else {
-    tlo = k0 * cd + cl - 1;
-    thi = T_ - 1;
-    const int c0 = q0, c1 = q0 + qlen - 1;
-    tlo = tlo > c0 ? tlo : c0;
-    thi = thi < c1 ? thi : c1;
-  }
-  thi = thi < T_ - 1 ? thi : T_ - 1;
-  // compression with a partial buffer: this workgroup's 32 NW rows of it
-  // (every logical workgroup writes them, zeros when it has no query)
-  float* prow = part != nullptr && mode == NSA_MODE_COMPRESS ? part + (wg * 32 * NW + (key - k0)) * D : nullptr;
+  const bool key_ok = key < r.Lk;
+  const int tlo = wk.tlo, thi = wk.thi, window = r.window, cl = r.cl, cd = r.cd;
+  const QSide<T> x = qside<T, D>(q, dout, coff, dot, Hq, Hkv, r.T_, false);
+  // with a partial buffer: this workgroup's 32 NW rows of it (every logical
+  // workgroup writes them, zeros when it has no query)
+  float* prow = part != nullptr ? part + (wk.wg * 32 * NW + (key - wk.k0)) * D : nullptr;
   if (tlo > thi) {   // uniform over the workgroup
     if (prow != nullptr && key_ok) zero_rows<D>(prow, prow + part_half, h);
     return;
   }
-  const int64_t kvoff = (int64_t)bh * Lk * D;
+  const int64_t kvoff = (int64_t)wk.bh * r.Lk * D;
   const int wlast = kw + 31;   // last key of the group (may pass Lk: those columns are never stored)
-  const int key_safe = key_ok ? key : Lk - 1;
-  const bool atomic = mode == NSA_MODE_COMPRESS && prow == nullptr;
+  const int key_safe = key_ok ? key : r.Lk - 1;
+  const bool atomic = r.mode == NSA_MODE_COMPRESS && prow == nullptr;
   // the two roles' walks over the workgroup's query tiles
   auto run = [&](auto make_rq, int total, auto vis) {
     if (pwave) {
@@ -1194,7 +1182,7 @@ void k_range_dkdv_split(int mode, const T* __restrict__ q, const T* __restrict__
       rq.init(x, b, hkv, rlo, thi, tid);
       return rq;
     };
-    const int wmode = mode == NSA_MODE_WINDOW ? window : 0;
+    const int wmode = r.mode == NSA_MODE_WINDOW ? window : 0;
     auto vis = [&](const KvStage<T, D>&, int it, bool& mask) {
       const int R0 = rlo + 32 * it;
       mask = flat_tile_needs_mask(kw, R0, rhi, G, wmode, cl, cd);
@@ -1212,7 +1200,7 @@ void k_range_dkdv_split(int mode, const T* __restrict__ q, const T* __restrict__
       const int tA = __builtin_amdgcn_readfirstlane(s.meta[0]), tB = __builtin_amdgcn_readfirstlane(s.meta[1]);
       const int tb = tB >= 0 ? tB : tA;
       VisPair v;
-      if (mode == NSA_MODE_WINDOW) {
+      if (r.mode == NSA_MODE_WINDOW) {
         mask = !(tA >= wlast && tb - window < kw);
         v.a = key <= tA && key > tA - window;
         v.b = key <= tb && key > tb - window;
@@ -1498,47 +1486,51 @@ __global__ __launch_bounds__(256) void k_sel_dkdv_reduce(const float* __restrict
   reinterpret_cast<f32x4*>(dv + orow)[c] = b;
 }
 
-// dK / dV of the pooled keys from the compression workgroups' partial rows:
-// one thread per 4 floats of a key row, summed over the key block's chunks in
-// chunk (then sub-chunk) order -- the logical workgroup numbering of
-// k_range_dkdv32 / k_range_dkdv_split -- so the result does not depend on
-// which workgroup finished first.
+// dK / dV of every key from the range workgroups' partial rows: one thread
+// per 4 floats of a key row, summed over the key block's parts (window) or
+// chunks (compression: chunk, then sub-chunk) in query order -- the logical
+// workgroup numbering of kv_work -- so the result does not depend on which
+// workgroup finished first.
 template <int D, int NW>
-__global__ __launch_bounds__(256) void k_cmp_dkdv_reduce(const float* __restrict__ part, int64_t part_half,
-                                                         float* __restrict__ dk, float* __restrict__ dv, int T_,
-                                                         int Lk, int chunk, int cl, int cd, int nbh, int chs,
-                                                         int spl) {
+__global__ __launch_bounds__(256) void k_range_dkdv_reduce(const KvRange r, const float* __restrict__ part,
+                                                           int64_t part_half, float* __restrict__ dk,
+                                                           float* __restrict__ dv) {
   constexpr int KB = 32 * NW;
   constexpr int V4 = D / 4;   // float4 per key row
   const int64_t f = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (f >= (int64_t)nbh * Lk * V4) return;
+  if (f >= (int64_t)r.nbh * r.Lk * V4) return;
   const int c = (int)(f % V4);
-  const int key = (int)((f / V4) % Lk);
-  const int bh = (int)(f / ((int64_t)V4 * Lk));
+  const int key = (int)((f / V4) % r.Lk);
+  const int bh = (int)(f / ((int64_t)V4 * r.Lk));
   const int kblk = key / KB, kk = key % KB;
-  const int nch = (T_ + chunk - 1) / chunk;
-  const int big = cmp_blocks_range(T_, Lk, chunk, NW, cl, cd, 0, chs);
-  const int per = cmp_blocks_range(T_, Lk, chunk, NW, cl, cd, chs, nch) * spl;
   f32x4 a = zero4(), b = zero4();
   auto add = [&](int64_t wgi) {
     const int64_t row = wgi * KB + kk;
     a += reinterpret_cast<const f32x4*>(part + row * D)[c];
     b += reinterpret_cast<const f32x4*>(part + part_half + row * D)[c];
   };
-  int64_t base = (int64_t)bh * big;   // chunks < chs: per bh, chunk-major
-  for (int ch = 0; ch < chs; ++ch) {
-    const int na = cmp_active_blocks(T_, Lk, chunk, NW, cl, cd, ch);
-    if (kblk < na) add(base + kblk);
-    base += na;
+  if (r.mode == NSA_MODE_WINDOW) {
+    const int64_t w0 = ((int64_t)bh * ((r.Lk + KB - 1) / KB) + kblk) * r.spl;
+    for (int i = 0; i < r.spl; ++i) add(w0 + i);
+  } else {
+    const int nch = (r.T_ + r.chunk - 1) / r.chunk;
+    const int big = cmp_blocks_range(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, 0, r.chs);
+    const int per = cmp_blocks_range(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, r.chs, nch) * r.spl;
+    int64_t base = (int64_t)bh * big;   // chunks < chs: per bh, chunk-major
+    for (int ch = 0; ch < r.chs; ++ch) {
+      const int na = cmp_active_blocks(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, ch);
+      if (kblk < na) add(base + kblk);
+      base += na;
+    }
+    base = (int64_t)big * r.nbh + (int64_t)bh * per;   // the split chunks: (chunk, sub-chunk)-major
+    for (int ch = r.chs; ch < nch; ++ch) {
+      const int na = cmp_active_blocks(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, ch);
+      if (kblk < na)
+        for (int sub = 0; sub < r.spl; ++sub) add(base + (int64_t)sub * na + kblk);
+      base += (int64_t)na * r.spl;
+    }
   }
-  base = (int64_t)big * nbh + (int64_t)bh * per;   // the split chunks: (chunk, sub-chunk)-major
-  for (int ch = chs; ch < nch; ++ch) {
-    const int na = cmp_active_blocks(T_, Lk, chunk, NW, cl, cd, ch);
-    if (kblk < na)
-      for (int sub = 0; sub < spl; ++sub) add(base + (int64_t)sub * na + kblk);
-    base += (int64_t)na * spl;
-  }
-  const int64_t orow = ((int64_t)bh * Lk + key) * D;
+  const int64_t orow = ((int64_t)bh * r.Lk + key) * D;
   reinterpret_cast<f32x4*>(dk + orow)[c] = a;
   reinterpret_cast<f32x4*>(dv + orow)[c] = b;
 }
@@ -1557,7 +1549,7 @@ using namespace nsa;
   }
 
 static constexpr int kCmpChunk = 2048;   // queries per compression dK/dV work item
-static constexpr int kCmpSplit = 4;      // sub-chunks of the chunks that end the grid
+static constexpr int kCmpSplit = 4;      // sub-chunks of the chunks that end a grid of several rounds
 
 // Device of a stream (the null stream: the current device), or -1.
 static int stream_device(hipStream_t s) {
@@ -1582,38 +1574,73 @@ static int device_cu_count(hipStream_t s) {
 }
 
 
+constexpr int kRangeNW = 2;        // key groups of 32 per range dK/dV workgroup
+constexpr int kMinPartQueries = 32;   // fewest queries of a window part or compression sub-chunk
+
 // Compression dK/dV grid: logical workgroups over (key block, query chunk),
-// the chunks from *chs on split into *spl sub-chunks while their workgroups fit
-// in one round of the resident workgroups (two per CU of the stream's device).
-static int64_t cmp_grid(int T, int Lk, int cl, int cd, int nbh, hipStream_t s, int* chs_out, int* spl_out) {
-  constexpr int NW = 2;
-  const int nch = (T + kCmpChunk - 1) / kCmpChunk;
+// the chunks from r.chs on in r.spl sub-chunks while their workgroups fit in
+// one round of the resident workgroups (two per CU of the stream's device).
+// A sequence whose chunks all fit takes as many sub-chunks as fill that
+// round.  With it, the window's parts and flat float tiles, a float32 layer
+// step at B1 T1024 Hq4 Hkv1 D64 takes 892 us instead of 3267: the compression
+// ran on 4 workgroups and the window on 16, three of four tile rows empty.
+static int64_t cmp_grid(KvRange& r, hipStream_t s) {
+  constexpr int NW = kRangeNW;
+  r.chunk = r.T_ < kCmpChunk ? r.T_ : kCmpChunk;
+  const int nch = (r.T_ + r.chunk - 1) / r.chunk;
   const int64_t slots = 2 * (int64_t)device_cu_count(s);
   int64_t tail = 0;
   int chs = nch;
   while (chs > 0) {
-    const int64_t add = (int64_t)cmp_active_blocks(T, Lk, kCmpChunk, NW, cl, cd, chs - 1) * nbh;
+    const int64_t add = (int64_t)cmp_active_blocks(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, chs - 1) * r.nbh;
     if (tail + add > slots) break;
     tail += add;
     --chs;
   }
-  const int spl = chs < nch ? kCmpSplit : 1;
-  *chs_out = chs;
-  *spl_out = spl;
-  return ((int64_t)cmp_blocks_range(T, Lk, kCmpChunk, NW, cl, cd, 0, chs) +
-          (int64_t)cmp_blocks_range(T, Lk, kCmpChunk, NW, cl, cd, chs, nch) * spl) * nbh;
+  r.chs = chs;
+  r.spl = chs < nch ? kCmpSplit : 1;
+  if (chs == 0 && tail > 0) {
+    int64_t most = slots / tail;
+    const int64_t room = (r.chunk + kMinPartQueries - 1) / kMinPartQueries;
+    if (most > room) most = room;
+    if (most > r.spl) r.spl = (int)most;
+  }
+  return ((int64_t)cmp_blocks_range(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, 0, chs) +
+          (int64_t)cmp_blocks_range(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, chs, nch) * r.spl) * r.nbh;
+}
+
+// Window dK/dV grid: one workgroup per key block, or r.spl of them while they
+// still fit in one round of the resident workgroups (a split past that only
+// adds a second round and the partial rows).
+static int64_t win_grid(KvRange& r, bool split, hipStream_t s) {
+  const int64_t g = (int64_t)((r.Lk + 32 * kRangeNW - 1) / (32 * kRangeNW)) * r.nbh;
+  r.chunk = r.T_;
+  r.chs = 0;
+  r.spl = 1;
+  if (split && g > 0) {
+    int64_t most = 2 * (int64_t)device_cu_count(s) / g;
+    const int64_t room = (32 * kRangeNW + (int64_t)(r.window < r.T_ ? r.window : r.T_) - 1) / kMinPartQueries;
+    if (most > room) most = room;
+    if (most > 1) r.spl = (int)most;
+  }
+  return g * r.spl;
+}
+
+static size_t range_part_bytes(int64_t grid, int D) {
+  return (size_t)grid * 32 * kRangeNW * (size_t)D * 2 * sizeof(float);
 }
 
 extern "C" {
 
 size_t nsa_range_dkdv_partial_bytes(int mode, int B, int Hkv, int T, int Lk, int D, int cmp_block, int cmp_stride,
                                     void* stream) {
-  if (mode != NSA_MODE_COMPRESS || B <= 0 || Hkv <= 0 || T <= 0 || Lk <= 0 || D <= 0 || cmp_block < 1 ||
-      cmp_stride < 1)
+  if ((mode != NSA_MODE_COMPRESS && mode != NSA_MODE_WINDOW) || B <= 0 || Hkv <= 0 || T <= 0 || Lk <= 0 || D <= 0 ||
+      cmp_block < 1 || cmp_stride < 1)
     return 0;
-  int chs = 0, spl = 1;
-  const int64_t grid = cmp_grid(T, Lk, cmp_block, cmp_stride, B * Hkv, (hipStream_t)stream, &chs, &spl);
-  return (size_t)grid * 64 * (size_t)D * 2 * sizeof(float);
+  KvRange r{mode, T, Lk, 0, cmp_block, cmp_block, cmp_stride, B * Hkv, 0, 1};
+  if (mode == NSA_MODE_COMPRESS) return range_part_bytes(cmp_grid(r, (hipStream_t)stream), D);
+  const int64_t grid = win_grid(r, true, (hipStream_t)stream);
+  return r.spl > 1 ? range_part_bytes(grid, D) : 0;
 }
 
 int nsa_range_dkdv(int mode, const void* q, const void* k, const void* v, const void* dout, const float* coff,
@@ -1635,17 +1662,22 @@ int nsa_range_dkdv(int mode, const void* q, const void* k, const void* v, const 
   // both walks; the role-split walk takes config 3's window / compression
   // dK/dV from 2.03 / 3.89 ms to 1.72 / 3.18 ms, and unrolled over its
   // stages to 1.61 / 3.03 ms.
-  constexpr int NW = 2;
-  const int nbh = B * Hkv;
-  int chs = 0, spl = 1;
+  constexpr int NW = kRangeNW;
+  KvRange r{mode, T, Lk, T, window, cmp_block, cmp_stride, B * Hkv, 0, 1};
   int64_t grid = 0;
-  if (T > 0 && Lk > 0)
-    grid = mode == NSA_MODE_COMPRESS ? cmp_grid(T, Lk, cmp_block, cmp_stride, nbh, s, &chs, &spl)
-                                     : (int64_t)((Lk + 32 * NW - 1) / (32 * NW)) * nbh;
-  // compression partials: the workgroups write their rows, k_cmp_dkdv_reduce
-  // sums them in a fixed order and writes every key
-  const bool partial = mode == NSA_MODE_COMPRESS && dkdv_part != nullptr && grid > 0;
-  NSA_CHECK(!partial || part_bytes >= (size_t)grid * 64 * D * 2 * sizeof(float), NSA_ERR_WORKSPACE);
+  if (T > 0 && Lk > 0) {
+    if (mode == NSA_MODE_COMPRESS) {
+      grid = cmp_grid(r, s);
+    } else {
+      grid = win_grid(r, dkdv_part != nullptr, s);
+      // a buffer without room for the parts: the window is not split
+      if (r.spl > 1 && part_bytes < range_part_bytes(grid, D)) grid = win_grid(r, false, s);
+    }
+  }
+  // partials: the workgroups write their rows, k_range_dkdv_reduce sums them
+  // in a fixed order and writes every key
+  const bool partial = dkdv_part != nullptr && grid > 0 && (mode == NSA_MODE_COMPRESS || r.spl > 1);
+  NSA_CHECK(!partial || part_bytes >= range_part_bytes(grid, D), NSA_ERR_WORKSPACE);
   if ((mode == NSA_MODE_COMPRESS && !partial) || T == 0) {
     int rc = zero_f32(dk, nel, s);
     if (rc == NSA_OK) rc = zero_f32(dv, nel, s);
@@ -1657,22 +1689,22 @@ int nsa_range_dkdv(int mode, const void* q, const void* k, const void* v, const 
   const float sl2 = scale * kLog2e;
   float* part = partial ? dkdv_part : nullptr;
   const int64_t part_half = grid * 32 * NW * D;
+  // groups of G < 16 heads: query tiles of 32 consecutive (query, head) rows
+  const bool flat = Hq / Hkv < 16;
   NSA_DISPATCH_D(D, {
     if (dtype == NSA_BF16) {
-      // groups of G < 16 heads: query tiles of 32 consecutive (query, head) rows
-      auto kern = Hq / Hkv < 16 ? k_range_dkdv_split<bf16, DD, NW, true> : k_range_dkdv_split<bf16, DD, NW, false>;
-      kern<<<(unsigned)grid, 128 * NW, 0, s>>>(mode, (const bf16*)q, (const bf16*)dout, coff, dot, (const bf16*)k,
-                                               (const bf16*)v, dk, dv, part, part_half, Hq, Hkv, T, Lk, kCmpChunk,
-                                               window, cmp_block, cmp_stride, nbh, chs, spl, sl2, scale);
-    } else
-      k_range_dkdv32<float, DD, NW><<<(unsigned)grid, 64 * NW, 0, s>>>(
-          mode, (const float*)q, (const float*)dout, coff, dot, (const float*)k, (const float*)v, dk, dv, part,
-          part_half, Hq, Hkv, T, Lk, kCmpChunk, window, cmp_block, cmp_stride, nbh, chs, spl, sl2, scale);
+      auto kern = flat ? k_range_dkdv_split<bf16, DD, NW, true> : k_range_dkdv_split<bf16, DD, NW, false>;
+      kern<<<(unsigned)grid, 128 * NW, 0, s>>>(r, (const bf16*)q, (const bf16*)dout, coff, dot, (const bf16*)k,
+                                               (const bf16*)v, dk, dv, part, part_half, Hq, Hkv, sl2, scale);
+    } else {
+      auto kern = flat ? k_range_dkdv32<float, DD, NW, true> : k_range_dkdv32<float, DD, NW, false>;
+      kern<<<(unsigned)grid, 64 * NW, 0, s>>>(r, (const float*)q, (const float*)dout, coff, dot, (const float*)k,
+                                              (const float*)v, dk, dv, part, part_half, Hq, Hkv, sl2, scale);
+    }
     if (partial) {
       if (hipGetLastError() != hipSuccess) return NSA_ERR_LAUNCH;
-      const int64_t total = (int64_t)nbh * Lk * (DD / 4);
-      k_cmp_dkdv_reduce<DD, NW><<<(unsigned)((total + 255) / 256), 256, 0, s>>>(
-          part, part_half, dk, dv, T, Lk, kCmpChunk, cmp_block, cmp_stride, nbh, chs, spl);
+      const int64_t total = (int64_t)r.nbh * Lk * (DD / 4);
+      k_range_dkdv_reduce<DD, NW><<<(unsigned)((total + 255) / 256), 256, 0, s>>>(r, part, part_half, dk, dv);
     }
   });
   return nsa_launch_status();

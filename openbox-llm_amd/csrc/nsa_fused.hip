@@ -111,9 +111,9 @@ FwdScratch carve_fwd(const Dims& m, void* base, size_t* bytes) {
 }
 
 struct BwdScratch {
-  float *dot, *rs, *coff, *dks, *dvs, *dkw, *dvw, *dkp, *dvp, *sel_part, *cmp_part;
+  float *dot, *rs, *coff, *dks, *dvs, *dkw, *dvw, *dkp, *dvp, *sel_part, *cmp_part, *win_part;
   void *dop, *kt_s, *dq_part, *sel_ws, *kt_w, *kt_c;
-  size_t sel_bytes, sel_part_bytes, cmp_part_bytes;
+  size_t sel_bytes, sel_part_bytes, cmp_part_bytes, win_part_bytes;
 };
 
 BwdScratch carve_bwd(const Dims& m, void* base, size_t* bytes, hipStream_t s) {
@@ -142,6 +142,9 @@ BwdScratch carve_bwd(const Dims& m, void* base, size_t* bytes, hipStream_t s) {
   x.dvp = (f32 && m.pooled) ? nullptr : (float*)c.take(m.kv(n) * sizeof(float));
   x.cmp_part_bytes = nsa_range_dkdv_partial_bytes(NSA_MODE_COMPRESS, m.B, m.Hkv, m.T, n, m.D, m.l, m.d, s);
   x.cmp_part = (float*)c.take(x.cmp_part_bytes);
+  // the window's dK/dV parts (0 bytes where it is not split)
+  x.win_part_bytes = nsa_range_dkdv_partial_bytes(NSA_MODE_WINDOW, m.B, m.Hkv, m.T, m.T, m.D, m.window, 1, s);
+  x.win_part = x.win_part_bytes > 0 ? (float*)c.take(x.win_part_bytes) : nullptr;
   x.kt_c = c.take((size_t)m.B * m.Hkv * m.D * nsa_padded_len(n) * m.es());
   *bytes = c.off;
   return x;
@@ -259,8 +262,8 @@ int nsa_fused_bwd(const void* dout, const void* q, const void* kc, const void* v
                        S, sel_block, kDkdvChunk, dtype, stream));
   // window and compression dK/dV
   NSA_TRY(nsa_transpose_kv(kw, w.kt_w, B * Hkv, T, D, Lpt, dtype, stream));
-  NSA_TRY(nsa_range_dkdv(NSA_MODE_WINDOW, q, kw, vw, dout, w.coff + 2 * R, w.dot + 2 * R, dkw32, dvw32, nullptr, 0, B,
-                         Hq, Hkv, T, T, D, window, 1, 1, dtype, stream));
+  NSA_TRY(nsa_range_dkdv(NSA_MODE_WINDOW, q, kw, vw, dout, w.coff + 2 * R, w.dot + 2 * R, dkw32, dvw32, w.win_part,
+                         w.win_part_bytes, B, Hq, Hkv, T, T, D, window, 1, 1, dtype, stream));
   NSA_TRY(nsa_range_dkdv(NSA_MODE_COMPRESS, q, k_cmp, v_cmp, dout, w.coff, w.dot, dkp32, dvp32, w.cmp_part,
                          w.cmp_part_bytes, B, Hq, Hkv, T, n, D, 0, cmp_block, cmp_stride, dtype, stream));
   // compression + window dQ in one launch, rows finished with the selection partials

@@ -663,9 +663,11 @@ def range_dkdv(mode, q, k, v, do, coff, dot, window=0, cmp_block=1, cmp_stride=1
     dk = torch.empty(B, Hkv, Lk, D, device=q.device, dtype=torch.float32)
     dv = torch.empty_like(dk)
     part, part_bytes = None, 0
-    if DETERMINISTIC_DKDV and mode == MODE_COMPRESS:
-        part_bytes = int(_lib().nsa_range_dkdv_partial_bytes(mode, B, Hkv, T, Lk, D, int(cmp_block),
-                                                             int(cmp_stride), _stream(q)))
+    if DETERMINISTIC_DKDV:
+        # (the window takes its window in the span's place; 0 bytes where it is not split)
+        span, step = (window, 1) if mode == MODE_WINDOW else (cmp_block, cmp_stride)
+        part_bytes = int(_lib().nsa_range_dkdv_partial_bytes(mode, B, Hkv, T, Lk, D, int(span), int(step),
+                                                             _stream(q)))
         if part_bytes > 0:
             part = torch.empty(part_bytes // 4, device=q.device, dtype=torch.float32)
     _call(_span_name("dkdv", mode), _lib().nsa_range_dkdv, mode, L.ptr(q), L.ptr(k), L.ptr(v), L.ptr(do),
