@@ -203,6 +203,9 @@ int nsa_csr_build(const int32_t* block_idx, int32_t* q_of_block, int32_t* block_
  * slot, pass), scaled, in the input dtype,
  * [B][Hkv][T][nsa_sel_partial_slots(S, block_size)][G][D] -- summed by
  * nsa_sel_dq_reduce. */
+/* nsa_sel_dkdv_chunk: the chunk that suits these sizes (fewer queries per
+ * work item where the items would leave CUs idle). */
+int nsa_sel_dkdv_chunk(int B, int Hkv, int T, int S, int block_size);
 size_t nsa_sel_dkdv_workspace(int B, int Hkv, int T, int S, int block_size, int chunk);
 size_t nsa_sel_dkdv_partial_bytes(int B, int Hkv, int T, int S, int D, int block_size, int chunk);
 int nsa_sel_dkdv(const void* q, const void* k, const void* v, const void* kt, const void* dout, const float* coff,
@@ -251,6 +254,8 @@ int nsa_sel_dkdv_noalloc(const void* q, const void* k, const void* v, const void
  * every such partial) reaches 2^15.  nsa_sel_merge and nsa_range_fwd_finish read them
  * with the inputs' dtype. */
 int nsa_sel_partial_slots(int S, int block_size);
+/* nsa_sel_fwd_chunk: the chunk that suits these sizes. */
+int nsa_sel_fwd_chunk(int B, int Hkv, int T, int S, int block_size);
 size_t nsa_sel_fwd_bo_workspace(int B, int Hkv, int T, int S, int block_size, int chunk);
 int nsa_sel_fwd_bo(const void* q, const void* k, const void* vt, const int32_t* q_of_block,
                    const int32_t* block_offsets, void* o_part, float* ml_part, void* workspace,

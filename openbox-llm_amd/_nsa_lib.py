@@ -54,6 +54,8 @@ SIGNATURES = {
                         _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "nsa_csr_workspace": (_Z, [_I, _I, _I, _I, _I]),
     "nsa_csr_build": (_I, [_P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _I, _I, _P]),
+    "nsa_sel_fwd_chunk": (_I, [_I, _I, _I, _I, _I]),
+    "nsa_sel_dkdv_chunk": (_I, [_I, _I, _I, _I, _I]),
     "nsa_sel_dkdv_workspace": (_Z, [_I, _I, _I, _I, _I, _I]),
     "nsa_sel_dkdv_partial_bytes": (_Z, [_I, _I, _I, _I, _I, _I, _I]),
     "nsa_sel_dkdv": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _Z, _P, _P, _Z,

@@ -1710,6 +1710,11 @@ int nsa_range_dkdv(int mode, const void* q, const void* k, const void* v, const 
   return nsa_launch_status();
 }
 
+int nsa_sel_dkdv_chunk(int B, int Hkv, int T, int S, int block_size) {
+  if (B <= 0 || Hkv <= 0 || T < 0 || S < 0 || block_size <= 0) return 0;
+  return sel_dkdv_chunk((int64_t)B * Hkv * T * S * sel_passes(block_size));
+}
+
 size_t nsa_sel_dkdv_workspace(int B, int Hkv, int T, int S, int block_size, int chunk) {
   if (B <= 0 || Hkv <= 0 || T < 0 || S < 0 || block_size <= 0 || chunk <= 0) return 0;
   const size_t nb = (size_t)B * Hkv * sel_csr_blocks(T, block_size);

@@ -21,9 +21,6 @@
 
 namespace {
 
-constexpr int kFwdChunk = 128;    // CSR queries per selection forward work item
-constexpr int kDkdvChunk = 512;   // CSR queries per selection dK/dV work item
-
 struct Carver {
   size_t off = 0;
   char* base = nullptr;
@@ -47,6 +44,9 @@ struct Dims {
   // float32 for float32 inputs (unrounded either way but for fp16's 11 bits)
   int o_dtype() const { return dtype == NSA_BF16 ? NSA_F16S : NSA_F32; }
   size_t o_bytes() const { return dtype == NSA_BF16 ? (size_t)rows() * (2 * D + 4) : (size_t)rows() * D * 4; }
+  // CSR queries per selection work item
+  int fwd_chunk() const { return nsa_sel_fwd_chunk(B, Hkv, T, S(), ls); }
+  int dkdv_chunk() const { return nsa_sel_dkdv_chunk(B, Hkv, T, S(), ls); }
   int64_t kv(int L) const { return (int64_t)B * Hkv * L * D; }
   bool ok() const {
     return B > 0 && Hkv > 0 && Hq % Hkv == 0 && (D == 16 || D == 32 || D == 64 || D == 128) && l >= 1 && d >= 1 &&
@@ -103,7 +103,7 @@ FwdScratch carve_fwd(const Dims& m, void* base, size_t* bytes) {
   x.vt_s = c.take((size_t)m.B * m.Hkv * m.D * nsa_padded_len(m.T) * m.es());
   x.o_part = c.take((size_t)m.rows() * ns * m.D * m.es());
   x.ml_part = (float*)c.take((size_t)m.rows() * ns * 2 * sizeof(float));
-  x.sel_bytes = nsa_sel_fwd_bo_workspace(m.B, m.Hkv, m.T, S, m.ls, kFwdChunk);
+  x.sel_bytes = nsa_sel_fwd_bo_workspace(m.B, m.Hkv, m.T, S, m.ls, m.fwd_chunk());
   x.sel_ws = c.take(x.sel_bytes);
   x.vt_w = c.take((size_t)m.B * m.Hkv * m.D * nsa_padded_len(m.T) * m.es());
   *bytes = c.off;
@@ -131,9 +131,9 @@ BwdScratch carve_bwd(const Dims& m, void* base, size_t* bytes, hipStream_t s) {
   x.dks = f32 ? nullptr : (float*)c.take(m.kv(m.T) * sizeof(float));
   x.dvs = f32 ? nullptr : (float*)c.take(m.kv(m.T) * sizeof(float));
   x.dq_part = c.take((size_t)m.rows() * ns * m.D * m.es());
-  x.sel_bytes = nsa_sel_dkdv_workspace(m.B, m.Hkv, m.T, S, m.ls, kDkdvChunk);
+  x.sel_bytes = nsa_sel_dkdv_workspace(m.B, m.Hkv, m.T, S, m.ls, m.dkdv_chunk());
   x.sel_ws = c.take(x.sel_bytes);
-  x.sel_part_bytes = nsa_sel_dkdv_partial_bytes(m.B, m.Hkv, m.T, S, m.D, m.ls, kDkdvChunk);
+  x.sel_part_bytes = nsa_sel_dkdv_partial_bytes(m.B, m.Hkv, m.T, S, m.D, m.ls, m.dkdv_chunk());
   x.sel_part = (float*)c.take(x.sel_part_bytes);
   x.kt_w = c.take((size_t)m.B * m.Hkv * m.D * nsa_padded_len(m.T) * m.es());
   x.dkw = f32 ? nullptr : (float*)c.take(m.kv(m.T) * sizeof(float));
@@ -215,7 +215,7 @@ int nsa_fused_fwd(const void* q, const void* kc, const void* vc, const void* ks,
                         S, sel_block, m.nblk(), 1, stream));
   NSA_TRY(nsa_transpose_kv(vs, w.vt_s, B * Hkv, T, D, Lpt, dtype, stream));
   NSA_TRY(nsa_sel_fwd_bo(x.qp, ks, w.vt_s, x.q_of_block, x.offsets, w.o_part, w.ml_part, w.sel_ws, w.sel_bytes, B, Hq,
-                         Hkv, T, D, S, sel_block, kFwdChunk, dtype, stream));
+                         Hkv, T, D, S, sel_block, m.fwd_chunk(), dtype, stream));
   // window, finishing the rows: selection merge and gate
   NSA_TRY(nsa_transpose_kv(vw, w.vt_w, B * Hkv, T, D, Lpt, dtype, stream));
   return nsa_range_fwd_finish(NSA_MODE_WINDOW, q, kw, w.vt_w, x.o_w, x.lse_w, B, Hq, Hkv, T, T, D, window, 1, 1,
@@ -259,7 +259,7 @@ int nsa_fused_bwd(const void* dout, const void* q, const void* kc, const void* v
   NSA_TRY(nsa_transpose_kv(ks, w.kt_s, B * Hkv, T, D, Lpt, dtype, stream));
   NSA_TRY(nsa_sel_dkdv(x.qp, ks, vs, w.kt_s, w.dop, w.coff + R, w.dot + R, x.q_of_block, 1, x.offsets, x.count,
                        dks32, dvs32, w.sel_part, w.sel_part_bytes, w.dq_part, w.sel_ws, w.sel_bytes, B, Hq, Hkv, T, D,
-                       S, sel_block, kDkdvChunk, dtype, stream));
+                       S, sel_block, m.dkdv_chunk(), dtype, stream));
   // window and compression dK/dV
   NSA_TRY(nsa_transpose_kv(kw, w.kt_w, B * Hkv, T, D, Lpt, dtype, stream));
   NSA_TRY(nsa_range_dkdv(NSA_MODE_WINDOW, q, kw, vw, dout, w.coff + 2 * R, w.dot + 2 * R, dkw32, dvw32, w.win_part,

@@ -75,6 +75,26 @@ static inline size_t sel_items_cap(int B, int Hkv, int T, int S, int block_size,
   return nb + (pairs + chunk - 1) / chunk + 1;
 }
 
+// CSR queries per selection work item: the largest power of two that still
+// gives every resident slot of the kernel an item of a sequence this short, so
+// that a few blocks' queries do not run on a few CUs.  An item costs its
+// block's keys (forward: 64 keys of K and V^T; dK/dV: also K^T and 64 float
+// rows of dK and dV written and summed again), which sets both ends.
+// Measured, us, forward at chunks 128 / the rule's and dK/dV at 512 / the
+// rule's: B1 T1301 Hq64 Hkv4 D128 163 / 103 (64); B1 T2048 Hq16 Hkv1 D128
+// 159 / 62 (32) and 442 / 93 (64); T1024 Hq4 D64 float32 106 / 33 (16) and 445
+// / 91 (32); T6011 Hq16 Hkv4 D64 dK/dV 297 / 242 (256); T32768 Hq64 Hkv4 D128
+// dK/dV 4732 (512, four and more rounds of items) against 4790 at 256.
+__host__ __device__ inline int sel_item_chunk(int64_t pairs, int64_t slots, int lo, int hi) {
+  int c = lo;
+  while (c < hi && pairs / slots >= 2 * c) c *= 2;
+  return c;
+}
+static inline int sel_fwd_chunk(int64_t pairs) { return sel_item_chunk(pairs, 1024, 16, 128); }   // one wave per SIMD
+static inline int sel_dkdv_chunk(int64_t pairs) {                                                // two workgroups per CU
+  return pairs >= 512 * 2048 ? 512 : sel_item_chunk(pairs, 512, 32, 256);
+}
+
 // Most CSR entries in one selection work item (the kernels stage an item's
 // entries in LDS); the item chunk passed to the entry points is capped here.
 constexpr int kSelItemMax = 1024;

@@ -606,6 +606,11 @@ extern "C" {
 
 int nsa_sel_partial_slots(int S, int block_size) { return S * sel_passes(block_size); }
 
+int nsa_sel_fwd_chunk(int B, int Hkv, int T, int S, int block_size) {
+  if (B <= 0 || Hkv <= 0 || T < 0 || S < 0 || block_size <= 0) return 0;
+  return sel_fwd_chunk((int64_t)B * Hkv * T * S * sel_passes(block_size));
+}
+
 size_t nsa_sel_fwd_bo_workspace(int B, int Hkv, int T, int S, int block_size, int chunk) {
   if (B <= 0 || Hkv <= 0 || T < 0 || S < 0 || block_size <= 0 || chunk <= 0) return 0;
   return sel_items_cap(B, Hkv, T, S, block_size, chunk) * sizeof(int4) + 256;

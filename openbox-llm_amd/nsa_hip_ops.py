@@ -24,9 +24,10 @@ import _nsa_lib as L
 
 MODE_WINDOW = L.MODE_WINDOW
 MODE_COMPRESS = L.MODE_COMPRESS
-SEL_DKDV_CHUNK = 512          # CSR queries per selection dK/dV work item (deterministic partials: 512 measured
-                              # 0.1 ms a c3 step and 0.09 ms a c4 layer faster than 1024)
-SEL_FWD_CHUNK = 128           # CSR queries per selection forward work item (c3: 128 measured 0.1 ms faster than 512)
+# most CSR queries per selection work item; shorter problems take fewer
+# (nsa_sel_dkdv_chunk / nsa_sel_fwd_chunk)
+SEL_DKDV_CHUNK = 512
+SEL_FWD_CHUNK = 128
 
 
 @dataclass(frozen=True)
@@ -746,16 +747,17 @@ def sel_dkdv(q, k, v, do, coff, dot, block_idx, block_size, csr=None, kt=None, w
             kt = transpose_kv(k)
         ns = int(_lib().nsa_sel_partial_slots(S, block_size))
         dq_part = torch.empty(B, Hkv, T, ns, Hq // Hkv, D, device=q.device, dtype=q.dtype)
-    ws_bytes = int(_lib().nsa_sel_dkdv_workspace(B, Hkv, T, S, block_size, SEL_DKDV_CHUNK))
+    chunk = max(2, min(SEL_DKDV_CHUNK, int(_lib().nsa_sel_dkdv_chunk(B, Hkv, T, S, block_size))))
+    ws_bytes = int(_lib().nsa_sel_dkdv_workspace(B, Hkv, T, S, block_size, chunk))
     ws = torch.empty(max(ws_bytes, 1), device=q.device, dtype=torch.uint8)
     part, part_bytes = None, 0
     if DETERMINISTIC_DKDV:
-        part_bytes = int(_lib().nsa_sel_dkdv_partial_bytes(B, Hkv, T, S, D, block_size, SEL_DKDV_CHUNK))
+        part_bytes = int(_lib().nsa_sel_dkdv_partial_bytes(B, Hkv, T, S, D, block_size, chunk))
         part = torch.empty(max(part_bytes // 4, 1), device=q.device, dtype=torch.float32)
     _call("dkdv[sel]", _lib().nsa_sel_dkdv, L.ptr(qp), L.ptr(k), L.ptr(v), L.ptr(kt), L.ptr(dop), L.ptr(coff),
           L.ptr(dot), L.ptr(q_of_block), int(want_dq), L.ptr(offsets),
           L.ptr(count), L.ptr(dk), L.ptr(dv), L.ptr(part), part_bytes, L.ptr(dq_part), L.ptr(ws), ws_bytes, B, Hq,
-          Hkv, T, D, S, block_size, SEL_DKDV_CHUNK, L.dtype_code(q), _stream(q))
+          Hkv, T, D, S, block_size, chunk, L.dtype_code(q), _stream(q))
     return dk, dv, dq_part
 
 
@@ -865,10 +867,11 @@ def sel_fwd_partials(q, k, v, block_idx, block_size, csr=None, vt=None, qp=None)
     G = Hq // Hkv
     o_part = torch.empty(B, Hkv, T, ns, G, D, device=q.device, dtype=_partial_dtype(q.dtype))
     ml_part = torch.empty(B, Hkv, T, ns, G, 2, device=q.device, dtype=torch.float32)
-    ws_bytes = int(_lib().nsa_sel_fwd_bo_workspace(B, Hkv, T, S, block_size, SEL_FWD_CHUNK))
+    chunk = max(2, min(SEL_FWD_CHUNK, int(_lib().nsa_sel_fwd_chunk(B, Hkv, T, S, block_size))))
+    ws_bytes = int(_lib().nsa_sel_fwd_bo_workspace(B, Hkv, T, S, block_size, chunk))
     ws = torch.empty(max(ws_bytes, 1), device=q.device, dtype=torch.uint8)
     _call("fwd[sel]", _lib().nsa_sel_fwd_bo, L.ptr(qp), L.ptr(k), L.ptr(vt), L.ptr(q_of_block), L.ptr(offsets),
-          L.ptr(o_part), L.ptr(ml_part), L.ptr(ws), ws_bytes, B, Hq, Hkv, T, D, S, block_size, SEL_FWD_CHUNK,
+          L.ptr(o_part), L.ptr(ml_part), L.ptr(ws), ws_bytes, B, Hq, Hkv, T, D, S, block_size, chunk,
           L.dtype_code(q), _stream(q))
     return (o_part, ml_part), csr
 
