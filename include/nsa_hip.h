@@ -376,7 +376,8 @@ int nsa_range_dkdv(int mode, const void* q, const void* k, const void* v, const 
  * (nsa_fused_ctx_bytes) is written by the forward and read by the backward
  * (pooled keys, packed q, the float32 branch outputs, their lse, the block ->
  * query CSR); scratch (nsa_fused_scratch_bytes, for the stream's device) is
- * transient and may be shared by both calls.  The backward takes the
+ * transient and may be shared by both calls (nsa_fused_fwd_scratch_bytes /
+ * nsa_fused_bwd_scratch_bytes: what one of them needs).  The backward takes the
  * forward's inputs again, dO, and writes every gradient in dtype: dq, dkc /
  * dvc (shaped like kc / vc), dks, dvs, dkw, dvw, dgate [B][Hq][T][3]; the
  * compression and selection dK/dV use the deterministic partial merge. */
@@ -384,6 +385,10 @@ size_t nsa_fused_ctx_bytes(int B, int Hq, int Hkv, int T, int D, int cmp_block, 
                            int n_sel, int window, int pooled, int dtype);
 size_t nsa_fused_scratch_bytes(int B, int Hq, int Hkv, int T, int D, int cmp_block, int cmp_stride, int sel_block,
                                int n_sel, int window, int pooled, int dtype, void* stream);
+size_t nsa_fused_fwd_scratch_bytes(int B, int Hq, int Hkv, int T, int D, int cmp_block, int cmp_stride, int sel_block,
+                                   int n_sel, int window, int pooled, int dtype);
+size_t nsa_fused_bwd_scratch_bytes(int B, int Hq, int Hkv, int T, int D, int cmp_block, int cmp_stride, int sel_block,
+                                   int n_sel, int window, int pooled, int dtype, void* stream);
 int nsa_fused_fwd(const void* q, const void* kc, const void* vc, const void* ks, const void* vs, const void* kw,
                   const void* vw, const void* gate, int32_t* block_idx, int idx_given, void* out, void* ctx,
                   size_t ctx_bytes, void* scratch, size_t scratch_bytes, int B, int Hq, int Hkv, int T, int D,

@@ -179,6 +179,25 @@ size_t nsa_fused_scratch_bytes(int B, int Hq, int Hkv, int T, int D, int cmp_blo
   return fb > bb ? fb : bb;
 }
 
+// one direction's share of it (what that call checks)
+size_t nsa_fused_fwd_scratch_bytes(int B, int Hq, int Hkv, int T, int D, int cmp_block, int cmp_stride, int sel_block,
+                                   int n_sel, int window, int pooled, int dtype) {
+  const Dims m{B, Hq, Hkv, T, D, cmp_block, cmp_stride, sel_block, n_sel, window, 0, 0, dtype, pooled};
+  if (!m.ok()) return 0;
+  size_t bytes = 0;
+  carve_fwd(m, nullptr, &bytes);
+  return bytes;
+}
+
+size_t nsa_fused_bwd_scratch_bytes(int B, int Hq, int Hkv, int T, int D, int cmp_block, int cmp_stride, int sel_block,
+                                   int n_sel, int window, int pooled, int dtype, void* stream) {
+  const Dims m{B, Hq, Hkv, T, D, cmp_block, cmp_stride, sel_block, n_sel, window, 0, 0, dtype, pooled};
+  if (!m.ok()) return 0;
+  size_t bytes = 0;
+  carve_bwd(m, nullptr, &bytes, (hipStream_t)stream);
+  return bytes;
+}
+
 int nsa_fused_fwd(const void* q, const void* kc, const void* vc, const void* ks, const void* vs, const void* kw,
                   const void* vw, const void* gate, int32_t* block_idx, int idx_given, void* out, void* ctx,
                   size_t ctx_bytes, void* scratch, size_t scratch_bytes, int B, int Hq, int Hkv, int T, int D,
@@ -187,15 +206,12 @@ int nsa_fused_fwd(const void* q, const void* kc, const void* vc, const void* ks,
   const Dims m{B, Hq, Hkv, T, D, cmp_block, cmp_stride, sel_block, n_sel, window, force_init, n_local, dtype, pooled};
   NSA_CHECK(m.ok(), dtype == NSA_F32 || dtype == NSA_BF16 ? NSA_ERR_SHAPE : NSA_ERR_DTYPE);
   NSA_CHECK(q && kc && vc && ks && vs && kw && vw && gate && block_idx && out && ctx && scratch, NSA_ERR_ARG);
-  hipStream_t s = (hipStream_t)stream;
   size_t cb = 0, sb = 0;
   carve_ctx(m, nullptr, &cb);
   NSA_CHECK(ctx_bytes >= cb, NSA_ERR_WORKSPACE);
-  NSA_CHECK(scratch_bytes >= nsa_fused_scratch_bytes(B, Hq, Hkv, T, D, cmp_block, cmp_stride, sel_block, n_sel,
-                                                     window, pooled, dtype, stream),
-            NSA_ERR_WORKSPACE);
   const Ctx x = carve_ctx(m, ctx, &cb);
   const FwdScratch w = carve_fwd(m, scratch, &sb);
+  NSA_CHECK(scratch_bytes >= sb, NSA_ERR_WORKSPACE);
   const int n = m.ncmp(), S = m.S(), Lpn = nsa_padded_len(n), Lpt = nsa_padded_len(T);
   const void* k_cmp = pooled ? kc : x.k_cmp;
   const void* v_cmp = pooled ? vc : x.v_cmp;
@@ -236,11 +252,9 @@ int nsa_fused_bwd(const void* dout, const void* q, const void* kc, const void* v
   size_t cb = 0, sb = 0;
   carve_ctx(m, nullptr, &cb);
   NSA_CHECK(ctx_bytes >= cb, NSA_ERR_WORKSPACE);
-  NSA_CHECK(scratch_bytes >= nsa_fused_scratch_bytes(B, Hq, Hkv, T, D, cmp_block, cmp_stride, sel_block, n_sel,
-                                                     window, pooled, dtype, stream),
-            NSA_ERR_WORKSPACE);
   const Ctx x = carve_ctx(m, (void*)ctx, &cb);
   const BwdScratch w = carve_bwd(m, scratch, &sb, s);
+  NSA_CHECK(scratch_bytes >= sb, NSA_ERR_WORKSPACE);
   const int n = m.ncmp(), S = m.S(), G = m.G(), Lpn = nsa_padded_len(n), Lpt = nsa_padded_len(T);
   const int64_t R = m.rows();
   const bool f32 = dtype == NSA_F32;

@@ -8,7 +8,7 @@ MI355X (drop-in for the reference module nsa_fused_kernel.py).
 * ``block_mean_pool`` (nsa_fused_kernel.py:549-554) is the HIP pooling kernel
   with its backward.
 * ``nsa_fused_forward`` (nsa_fused_kernel.py:560-573) runs the whole gated
-  three-branch layer inside one autograd boundary (``NSAFusedHIP``).
+  three-branch layer inside one autograd boundary (``nsa_hip_ops.nsa_attention``).
 * ``nsa_attention`` adds what the reference leaves to the model: block choice
   by importance + top-n on the GPU and the overlapping compression /
   selection geometry (``NSAGeometry``).
@@ -58,8 +58,7 @@ def nsa_fused_forward(q, kc, vc, ks, vs, kw, vw, gate_logits, block_idx, block_s
     """
     S = block_idx.shape[-1]
     geom = NSAGeometry.aligned(block_size, S, window)
-    out, _ = _ops.NSAFusedHIP.apply(q, kc, vc, ks, vs, kw, vw, gate_logits, block_idx, geom)
-    return out
+    return _ops.nsa_attention(q, kc, vc, ks, vs, kw, vw, gate_logits, geom, block_idx)[0]
 
 
 def nsa_attention(q, kc, vc, ks, vs, kw, vw, gate_logits, geom, block_idx=None):

@@ -1199,58 +1199,86 @@ class NSAFusedCAPI(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, kc, vc, ks, vs, kw, vw, gate, block_idx, geom, pooled=False):
-        check_qkv(q, ks, vs)
-        check_qkv(q, kw, vw)
+        _check_layer(q, kc, vc, ks, vs, kw, vw, gate, geom, pooled)
         ins = tuple(_contig(t) for t in (q, kc, vc, ks, vs, kw, vw, gate))
         q = ins[0]
         B, Hq, T, D = q.shape
         Hkv = ins[3].shape[1]
         dt = L.dtype_code(q)
+        lib = _lib()
         dims = (B, Hq, Hkv, T, D, geom.cmp_block, geom.cmp_stride, geom.sel_block, geom.n_sel, geom.window)
-        ctx_bytes = int(_lib().nsa_fused_ctx_bytes(*dims, int(pooled), dt))
-        scr_bytes = int(_lib().nsa_fused_scratch_bytes(*dims, int(pooled), dt, _stream(q)))
+        ctx_bytes = int(lib.nsa_fused_ctx_bytes(*dims, int(pooled), dt))
+        scr_bytes = int(lib.nsa_fused_fwd_scratch_bytes(*dims, int(pooled), dt))
         assert ctx_bytes > 0 and scr_bytes > 0, "nsa_fused: unsupported shape (T must reach cmp_block and sel_block)"
         saved = torch.empty(ctx_bytes, device=q.device, dtype=torch.uint8)
         scratch = torch.empty(scr_bytes, device=q.device, dtype=torch.uint8)
         S = min(geom.n_sel, T // geom.sel_block)
         given = block_idx is not None
-        idx = (block_idx.to(torch.int32).contiguous() if given
-               else torch.empty(B, Hkv, T, S, device=q.device, dtype=torch.int32))
+        if given:
+            assert block_idx.shape == (B, Hkv, T, S), "block_idx must be [B, Hkv, T, min(n_sel, T // sel_block)]"
+            idx = block_idx.to(torch.int32).contiguous()
+        else:
+            idx = torch.empty(B, Hkv, T, S, device=q.device, dtype=torch.int32)
         out = torch.empty_like(q)
-        _call("nsa_fused_fwd", _lib().nsa_fused_fwd, *map(L.ptr, ins), L.ptr(idx), int(given), L.ptr(out),
+        _call("nsa_fused_fwd", lib.nsa_fused_fwd, *map(L.ptr, ins), L.ptr(idx), int(given), L.ptr(out),
               L.ptr(saved), ctx_bytes, L.ptr(scratch), scr_bytes, *dims, int(geom.force_init), int(geom.n_local),
               int(pooled), dt, _stream(q))
-        ctx.save_for_backward(*ins, idx, saved)
-        ctx.meta = (dims, scr_bytes, int(pooled), dt)
+        # the backward reads the pooled tokens: the caller's, or the context's
+        keep = ins if pooled else (ins[0], None, None, *ins[3:])
+        ctx.save_for_backward(*keep, idx, saved)
+        ctx.meta = (dims, int(pooled), dt)
         ctx.mark_non_differentiable(idx)
         return out, idx
 
     @staticmethod
     def backward(ctx, dout, _didx):
         *ins, idx, saved = ctx.saved_tensors
-        dims, scr_bytes, pooled, dt = ctx.meta
+        dims, pooled, dt = ctx.meta
+        lib = _lib()
         dout = _contig(dout.to(ins[0].dtype))
+        stream = _stream(dout)
+        scr_bytes = int(lib.nsa_fused_bwd_scratch_bytes(*dims, pooled, dt, stream))
         scratch = torch.empty(scr_bytes, device=dout.device, dtype=torch.uint8)
-        grads = [torch.empty_like(t) for t in ins]
-        _call("nsa_fused_bwd", _lib().nsa_fused_bwd, L.ptr(dout), *map(L.ptr, ins), L.ptr(idx), L.ptr(saved),
-              saved.numel(), L.ptr(scratch), scr_bytes, *map(L.ptr, grads), *dims, pooled, dt, _stream(dout))
+        # unpooled compression keys and values are shaped like the selection's
+        grads = [torch.empty_like(ins[3] if t is None else t) for t in ins]
+        _call("nsa_fused_bwd", lib.nsa_fused_bwd, L.ptr(dout), *map(L.ptr, ins), L.ptr(idx), L.ptr(saved),
+              saved.numel(), L.ptr(scratch), scr_bytes, *map(L.ptr, grads), *dims, pooled, dt, stream)
         return (*grads, None, None, None)
 
 
-# True: a model layer (nsa_attention_layer) runs through the C entry points
+def _check_layer(q, kc, vc, ks, vs, kw, vw, gate, geom, pooled):
+    """The argument checks of ``fused_forward`` and of the calls it makes."""
+    check_qkv(q, kc, vc)
+    check_qkv(q, ks, vs)
+    check_qkv(q, kw, vw)
+    B, Hq, T, _ = q.shape
+    assert ks.shape[2] == T and kw.shape[2] == T, "selection / window keys must have the query length"
+    assert kc.shape[1] == ks.shape[1] == kw.shape[1], "the branches must share their KV heads"
+    assert kc.shape[2] == (n_cmp_tokens(T, geom.cmp_block, geom.cmp_stride) if pooled else T), \
+        "compression keys must have the query length, or be its (T - l) // d + 1 pooled tokens"
+    assert gate.shape == (B, Hq, T, 3) and gate.dtype == q.dtype, "gate logits must be [B, Hq, T, 3] in q's dtype"
+
+
+# True: the layer runs through the C entry points where they take the call
 LAYER_CAPI = True
 
 
-def nsa_attention_layer(q, kc, vc, ks, vs, kw, vw, gate_logits, geom: NSAGeometry, block_idx=None, pooled=False):
-    """``nsa_attention`` for a model layer: through the C entry points
-    (``NSAFusedCAPI``) where they take the shape, one launch sequence per
-    direction issued from C++; else (``T`` shorter than a compression or
-    selection block, per-call timing wanted, or ``LAYER_CAPI`` off) through
-    ``NSAFusedHIP``."""
+def _capi_takes(q, ks, geom, block_idx):
+    """Whether the C entry points run this call: shapes they cover (``T`` at
+    least a compression and a selection block, ``block_idx`` of the S they
+    would choose themselves) and every switch of the Python sequence (per-call
+    timing, overlap, unfused dQ, atomic merges, work item sizes) at its
+    default."""
+    if not LAYER_CAPI or _TIMER is not None or q.dim() != 4 or ks.dim() != 4:
+        return False
     T = q.shape[2]
-    if LAYER_CAPI and _TIMER is None and T >= geom.cmp_block and T >= geom.sel_block:
-        return NSAFusedCAPI.apply(q, kc, vc, ks, vs, kw, vw, gate_logits, block_idx, geom, pooled)
-    return NSAFusedHIP.apply(q, kc, vc, ks, vs, kw, vw, gate_logits, block_idx, geom, pooled)
+    if T < geom.cmp_block or T < geom.sel_block or geom.n_sel < 1 or geom.n_local < 0:
+        return False
+    if OVERLAP_SEL_BWD or SEPARATE_SEL_DQ or not (FUSE_RANGE_DQ and DETERMINISTIC_DKDV):
+        return False
+    if (SEL_DKDV_CHUNK, SEL_FWD_CHUNK) != (512, 128):
+        return False
+    return block_idx is None or block_idx.shape == (q.shape[0], ks.shape[1], T, min(geom.n_sel, T // geom.sel_block))
 
 
 def nsa_attention(q, kc, vc, ks, vs, kw, vw, gate_logits, geom: NSAGeometry, block_idx=None, pooled=False):
@@ -1260,8 +1288,17 @@ def nsa_attention(q, kc, vc, ks, vs, kw, vw, gate_logits, geom: NSAGeometry, blo
     importance and top-n (nsa_model.py:343-355) computed on the GPU.
     ``pooled=True``: ``kc``/``vc`` are pooled compression tokens.
     Returns ``(out, block_idx)``.
+
+    Runs through the C entry points (``NSAFusedCAPI``: one library call per
+    direction) where they take the call, else through ``NSAFusedHIP``: the
+    Python sequence holds the host for 461 us a step at B1 T1024 Hq4 D64
+    float32, where the GPU needs less.
     """
-    return NSAFusedHIP.apply(q, kc, vc, ks, vs, kw, vw, gate_logits, block_idx, geom, pooled)
+    fn = NSAFusedCAPI if _capi_takes(q, ks, geom, block_idx) else NSAFusedHIP
+    return fn.apply(q, kc, vc, ks, vs, kw, vw, gate_logits, block_idx, geom, pooled)
+
+
+nsa_attention_layer = nsa_attention   # the model layer's name for it
 
 
 # ---------------------------------------------------------------------------

@@ -9,7 +9,7 @@ nsa_model.py).
 * ``NSAAttention(attn_impl='fused')``: the same layer with the attention on
   the MI355X HIP kernels: compression attention over the learned pooled
   tokens, block importance + top-n, selection, sliding window and the gate
-  blend in one autograd boundary (``nsa_hip_ops.NSAFusedHIP``).  The library
+  blend in one autograd boundary (``nsa_hip_ops.nsa_attention``).  The library
   is loaded on first use and its absence raises; nothing falls back to the
   'ref' path.
 * ``FullAttention``, ``make_attention``, ``Block``, ``NSATransformer``,
