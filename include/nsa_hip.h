@@ -213,6 +213,14 @@ int nsa_sel_dkdv(const void* q, const void* k, const void* v, const void* kt, co
                  float* dk, float* dv, float* dkdv_part, size_t part_bytes, void* dq_part, void* workspace,
                  size_t workspace_bytes, int B, int Hq, int Hkv, int T, int D, int S, int block_size, int chunk,
                  int dtype, void* stream);
+/* nsa_sel_dkdv with dk / dv in out_dtype: NSA_F32, or NSA_BF16 for bf16
+ * inputs (each float32 result rounded once; needs dkdv_part). */
+int nsa_sel_dkdv_as(const void* q, const void* k, const void* v, const void* kt, const void* dout, const float* coff,
+                    const float* dot, const int32_t* q_of_block, int packed, const int32_t* block_offsets,
+                    const int32_t* pair_count, void* dk, void* dv, float* dkdv_part, size_t part_bytes, void* dq_part,
+                    void* workspace, size_t workspace_bytes, int B, int Hq, int Hkv, int T, int D, int S,
+                    int block_size, int chunk, int dtype, int out_dtype, void* stream);
+
 
 /* nsa_sel_dkdv without a workspace argument: allocates nothing (no
  * hipMalloc, no allocating library call).  No counterpart in the reference:
@@ -269,6 +277,12 @@ int nsa_sel_fwd_bo(const void* q, const void* k, const void* vt, const int32_t* 
  * or NSA_F32 unrounded. */
 int nsa_sel_merge(const int32_t* block_idx, const void* o_part, const float* ml_part, void* o, float* lse, int B,
                   int Hq, int Hkv, int T, int D, int S, int block_size, int dtype, int o_dtype, void* stream);
+/* nsa_sel_merge with either or both results of a row: o in dtype, o32
+ * unrounded (16-bit dtype only); null: not written. */
+int nsa_sel_merge_both(const int32_t* block_idx, const void* o_part, const float* ml_part, void* o, float* o32,
+                       float* lse, int B, int Hq, int Hkv, int T, int D, int S, int block_size, int dtype,
+                       void* stream);
+
 
 /* dq_out = dq_acc (float32, nullable) + sum of the dQ partials of the valid
  * slots, written in the input dtype (the dQ reduce of
@@ -359,6 +373,12 @@ size_t nsa_range_dkdv_partial_bytes(int mode, int B, int Hkv, int T, int Lk, int
 int nsa_range_dkdv(int mode, const void* q, const void* k, const void* v, const void* dout, const float* coff,
                    const float* dot, float* dk, float* dv, float* dkdv_part, size_t part_bytes, int B, int Hq,
                    int Hkv, int T, int Lk, int D, int window, int cmp_block, int cmp_stride, int dtype, void* stream);
+/* nsa_range_dkdv with dk / dv in out_dtype: NSA_F32, or NSA_BF16 for bf16
+ * inputs (each float32 result rounded once; compression then needs dkdv_part). */
+int nsa_range_dkdv_as(int mode, const void* q, const void* k, const void* v, const void* dout, const float* coff,
+                      const float* dot, void* dk, void* dv, float* dkdv_part, size_t part_bytes, int B, int Hq,
+                      int Hkv, int T, int Lk, int D, int window, int cmp_block, int cmp_stride, int dtype,
+                      int out_dtype, void* stream);
 
 /* ---- the gated three-branch layer in two calls -------------------------------
  * nsa_fused_fwd / nsa_fused_bwd replace nsa_fused_forward and its autograd

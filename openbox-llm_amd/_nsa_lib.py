@@ -60,12 +60,15 @@ SIGNATURES = {
     "nsa_sel_dkdv_partial_bytes": (_Z, [_I, _I, _I, _I, _I, _I, _I]),
     "nsa_sel_dkdv": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _Z, _P, _P, _Z,
                           _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
+    "nsa_sel_dkdv_as": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _Z, _P, _P, _Z,
+                             _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "nsa_sel_dkdv_noalloc": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P,
                                   _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "nsa_sel_partial_slots": (_I, [_I, _I]),
     "nsa_sel_fwd_bo_workspace": (_Z, [_I, _I, _I, _I, _I, _I]),
     "nsa_sel_fwd_bo": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "nsa_sel_merge": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
+    "nsa_sel_merge_both": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "nsa_sel_dq_reduce": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "nsa_range_fwd": (_I, [_I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _I, _I, _P]),
     "nsa_range_fwd_finish": (_I, [_I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I,
@@ -77,6 +80,8 @@ SIGNATURES = {
     "nsa_range_dkdv_partial_bytes": (_Z, [_I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "nsa_range_dkdv": (_I, [_I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _Z,
                             _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
+    "nsa_range_dkdv_as": (_I, [_I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _Z,
+                               _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "nsa_fused_ctx_bytes": (_Z, [_I] * 12),
     "nsa_fused_scratch_bytes": (_Z, [_I] * 12 + [_P]),
     "nsa_fused_fwd_scratch_bytes": (_Z, [_I] * 12),

@@ -1100,6 +1100,25 @@ void k_range_dkdv32(const KvRange r, const T* __restrict__ q, const T* __restric
   }
 }
 
+// four consecutive elements of a dK / dV row as float or, rounded once, bf16
+__device__ __forceinline__ void store_f32x4(float* p, const f32x4& v) { *reinterpret_cast<f32x4*>(p) = v; }
+__device__ __forceinline__ void store_f32x4(bf16* p, const f32x4& v) { store4(p, v[0], v[1], v[2], v[3]); }
+
+// accumulator columns of one key -> a bf16 row (scaled, rounded once)
+template <typename T, int D>
+__device__ __forceinline__ void store_rows16(const f32x16 (&acc)[Tile32<T, D>::DT], bf16* row, float scale, int h) {
+  using C = Tile32<T, D>;
+#pragma unroll
+  for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      const int d = 32 * dt + 8 * g4 + 4 * h;
+      if (D % 32 == 0 || d < D)
+        store4(row + d, acc[dt][4 * g4] * scale, acc[dt][4 * g4 + 1] * scale, acc[dt][4 * g4 + 2] * scale,
+               acc[dt][4 * g4 + 3] * scale);
+    }
+}
+
 // accumulator columns of one key -> a float row (scaled; atomically when
 // several workgroups add into it)
 template <typename T, int D>
@@ -1123,7 +1142,8 @@ __device__ __forceinline__ void store_rows(const f32x16 (&acc)[Tile32<T, D>::DT]
   }
 }
 
-// k_range_dkdv32 with the role-split walk: 2 NW waves, waves < NW the
+// k_range_dkdv32 with the role-split walk (dk16 / dv16, given instead of dk /
+// dv: the rows of unsplit key blocks in bf16): 2 NW waves, waves < NW the
 // P-waves of key groups 0 .. NW-1, the others their dS-waves.  FLAT: the
 // query tiles are 32 consecutive rows t G + g of the group (FlatReq, groups
 // of G < 16 heads), else two queries x 16 heads of a head chunk (SplitReq).
@@ -1132,7 +1152,8 @@ __global__ __launch_bounds__(128 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))
 void k_range_dkdv_split(const KvRange r, const T* __restrict__ q, const T* __restrict__ dout,
                         const float* __restrict__ coff, const float* __restrict__ dot, const T* __restrict__ k,
                         const T* __restrict__ v, float* __restrict__ dk, float* __restrict__ dv,
-                        float* __restrict__ part, int64_t part_half, int Hq, int Hkv, float sl2, float scale) {
+                        bf16* __restrict__ dk16, bf16* __restrict__ dv16, float* __restrict__ part,
+                        int64_t part_half, int Hq, int Hkv, float sl2, float scale) {
   constexpr int NTH = 128 * NW;
   __shared__ __align__(16) KvStage<T, D> stg[kSplitStages];
   __shared__ __align__(16) PTile pbuf[NW][2];
@@ -1164,12 +1185,18 @@ void k_range_dkdv_split(const KvRange r, const T* __restrict__ q, const T* __res
       PWave<T, D> pw;
       pw.init(k + kvoff, key_safe, h);
       walk_p<T, D, NTH>(pw, stg, pbuf[w], make_rq, total, vis, sl2, tid);
-      if (key_ok) store_rows<T, D>(pw.dv, prow ? prow + part_half : dv + kvoff + (int64_t)key * D, 1.0f, atomic, h);
+      if (key_ok && dv16 != nullptr && prow == nullptr)
+        store_rows16<T, D>(pw.dv, dv16 + kvoff + (int64_t)key * D, 1.0f, h);
+      else if (key_ok)
+        store_rows<T, D>(pw.dv, prow ? prow + part_half : dv + kvoff + (int64_t)key * D, 1.0f, atomic, h);
     } else {
       SWave<T, D> sw;
       sw.init(v + kvoff, key_safe, h);
       walk_s<T, D, NTH>(sw, stg, pbuf[w], make_rq, total, tid);
-      if (key_ok) store_rows<T, D>(sw.dk, prow ? prow : dk + kvoff + (int64_t)key * D, scale, atomic, h);
+      if (key_ok && dk16 != nullptr && prow == nullptr)
+        store_rows16<T, D>(sw.dk, dk16 + kvoff + (int64_t)key * D, scale, h);
+      else if (key_ok)
+        store_rows<T, D>(sw.dk, prow ? prow : dk + kvoff + (int64_t)key * D, scale, atomic, h);
     }
   };
   if constexpr (FLAT) {
@@ -1458,10 +1485,13 @@ void k_sel_dkdv32(const T* __restrict__ q, const T* __restrict__ dout, const flo
 // block's items in item order (the items of a block are consecutive and
 // ascend in query order), so the result does not depend on which workgroup
 // finished first.  A block no query selected gets zeros.
-template <int D>
+// The rows' loads go out kRedBatch at a time (their sums stay in item order):
+// one load per step took 33 us over 63 partial rows of 94 pooled keys.
+constexpr int kRedBatch = 8;
+template <int D, typename TO>
 __global__ __launch_bounds__(256) void k_sel_dkdv_reduce(const float* __restrict__ part, int64_t part_half,
-                                                         const int32_t* __restrict__ first, float* __restrict__ dk,
-                                                         float* __restrict__ dv, int T_, int n_blk, int L, int npass,
+                                                         const int32_t* __restrict__ first, TO* __restrict__ dk,
+                                                         TO* __restrict__ dv, int T_, int n_blk, int L, int npass,
                                                          int64_t total) {
   constexpr int V4 = D / 4;   // float4 per key row
   const int64_t f = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -1476,14 +1506,22 @@ __global__ __launch_bounds__(256) void k_sel_dkdv_reduce(const float* __restrict
   if (kSelPass * pass + kk >= L || key >= kend) return;
   const int i0 = first[e], i1 = first[e + 1];
   f32x4 a = zero4(), b = zero4();
-  for (int i = i0; i < i1; ++i) {
-    const int64_t row = ((int64_t)i * npass + pass) * kSelPass + kk;
-    a += reinterpret_cast<const f32x4*>(part + row * D)[c];
-    b += reinterpret_cast<const f32x4*>(part + part_half + row * D)[c];
+  for (int i = i0; i < i1; i += kRedBatch) {
+    f32x4 xa[kRedBatch], xb[kRedBatch];
+#pragma unroll
+    for (int u = 0; u < kRedBatch; ++u)
+      if (i + u < i1) {
+        const int64_t row = ((int64_t)(i + u) * npass + pass) * kSelPass + kk;
+        xa[u] = reinterpret_cast<const f32x4*>(part + row * D)[c];
+        xb[u] = reinterpret_cast<const f32x4*>(part + part_half + row * D)[c];
+      }
+#pragma unroll
+    for (int u = 0; u < kRedBatch; ++u)
+      if (i + u < i1) a += xa[u], b += xb[u];
   }
-  const int64_t orow = ((int64_t)bh * T_ + key) * D;
-  reinterpret_cast<f32x4*>(dk + orow)[c] = a;
-  reinterpret_cast<f32x4*>(dv + orow)[c] = b;
+  const int64_t orow = ((int64_t)bh * T_ + key) * D + 4 * c;
+  store_f32x4(dk + orow, a);
+  store_f32x4(dv + orow, b);
 }
 
 // dK / dV of every key from the range workgroups' partial rows: one thread
@@ -1491,10 +1529,10 @@ __global__ __launch_bounds__(256) void k_sel_dkdv_reduce(const float* __restrict
 // chunks (compression: chunk, then sub-chunk) in query order -- the logical
 // workgroup numbering of kv_work -- so the result does not depend on which
 // workgroup finished first.
-template <int D, int NW>
+template <int D, int NW, typename TO>
 __global__ __launch_bounds__(256) void k_range_dkdv_reduce(const KvRange r, const float* __restrict__ part,
-                                                           int64_t part_half, float* __restrict__ dk,
-                                                           float* __restrict__ dv) {
+                                                           int64_t part_half, TO* __restrict__ dk,
+                                                           TO* __restrict__ dv) {
   constexpr int KB = 32 * NW;
   constexpr int V4 = D / 4;   // float4 per key row
   const int64_t f = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -1504,40 +1542,66 @@ __global__ __launch_bounds__(256) void k_range_dkdv_reduce(const KvRange r, cons
   const int bh = (int)(f / ((int64_t)V4 * r.Lk));
   const int kblk = key / KB, kk = key % KB;
   f32x4 a = zero4(), b = zero4();
-  auto add = [&](int64_t wgi) {
-    const int64_t row = wgi * KB + kk;
-    a += reinterpret_cast<const f32x4*>(part + row * D)[c];
-    b += reinterpret_cast<const f32x4*>(part + part_half + row * D)[c];
+  // the rows of a batch of logical workgroups (-1: none), loads first
+  auto add = [&](const int64_t (&wgi)[kRedBatch]) {
+    f32x4 xa[kRedBatch], xb[kRedBatch];
+#pragma unroll
+    for (int u = 0; u < kRedBatch; ++u)
+      if (wgi[u] >= 0) {
+        const int64_t row = wgi[u] * KB + kk;
+        xa[u] = reinterpret_cast<const f32x4*>(part + row * D)[c];
+        xb[u] = reinterpret_cast<const f32x4*>(part + part_half + row * D)[c];
+      }
+#pragma unroll
+    for (int u = 0; u < kRedBatch; ++u)
+      if (wgi[u] >= 0) a += xa[u], b += xb[u];
+  };
+  // n of them, `step` apart
+  auto add_run = [&](int64_t w0, int64_t step, int n) {
+    for (int i = 0; i < n; i += kRedBatch) {
+      int64_t wgi[kRedBatch];
+#pragma unroll
+      for (int u = 0; u < kRedBatch; ++u) wgi[u] = i + u < n ? w0 + (i + u) * step : -1;
+      add(wgi);
+    }
   };
   if (r.mode == NSA_MODE_WINDOW) {
-    const int64_t w0 = ((int64_t)bh * ((r.Lk + KB - 1) / KB) + kblk) * r.spl;
-    for (int i = 0; i < r.spl; ++i) add(w0 + i);
+    add_run(((int64_t)bh * ((r.Lk + KB - 1) / KB) + kblk) * r.spl, 1, r.spl);
   } else {
     const int nch = (r.T_ + r.chunk - 1) / r.chunk;
     const int big = cmp_blocks_range(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, 0, r.chs);
     const int per = cmp_blocks_range(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, r.chs, nch) * r.spl;
     int64_t base = (int64_t)bh * big;   // chunks < chs: per bh, chunk-major
-    for (int ch = 0; ch < r.chs; ++ch) {
-      const int na = cmp_active_blocks(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, ch);
-      if (kblk < na) add(base + kblk);
-      base += na;
+    for (int c0 = 0; c0 < r.chs; c0 += kRedBatch) {
+      int64_t wgi[kRedBatch];
+#pragma unroll
+      for (int u = 0; u < kRedBatch; ++u) {
+        const int na = c0 + u < r.chs ? cmp_active_blocks(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, c0 + u) : 0;
+        wgi[u] = kblk < na ? base + kblk : -1;
+        base += na;
+      }
+      add(wgi);
     }
     base = (int64_t)big * r.nbh + (int64_t)bh * per;   // the split chunks: (chunk, sub-chunk)-major
     for (int ch = r.chs; ch < nch; ++ch) {
       const int na = cmp_active_blocks(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, ch);
-      if (kblk < na)
-        for (int sub = 0; sub < r.spl; ++sub) add(base + (int64_t)sub * na + kblk);
+      if (kblk < na) add_run(base + kblk, na, r.spl);
       base += (int64_t)na * r.spl;
     }
   }
-  const int64_t orow = ((int64_t)bh * r.Lk + key) * D;
-  reinterpret_cast<f32x4*>(dk + orow)[c] = a;
-  reinterpret_cast<f32x4*>(dv + orow)[c] = b;
+  const int64_t orow = ((int64_t)bh * r.Lk + key) * D + 4 * c;
+  store_f32x4(dk + orow, a);
+  store_f32x4(dv + orow, b);
 }
 
 }  // namespace nsa
 
 using namespace nsa;
+
+// Zeros over n elements (a multiple of 4) of a float32 or bf16 result.
+static inline int zero_out(void* x, int64_t n, int dtype, hipStream_t s) {
+  return zero_f32((float*)x, dtype == NSA_BF16 ? n / 2 : n, s);
+}
 
 #define NSA_DISPATCH_D(D_, ...)                                 \
   switch (D_) {                                                 \
@@ -1646,12 +1710,24 @@ size_t nsa_range_dkdv_partial_bytes(int mode, int B, int Hkv, int T, int Lk, int
 int nsa_range_dkdv(int mode, const void* q, const void* k, const void* v, const void* dout, const float* coff,
                    const float* dot, float* dk, float* dv, float* dkdv_part, size_t part_bytes, int B, int Hq, int Hkv,
                    int T, int Lk, int D, int window, int cmp_block, int cmp_stride, int dtype, void* stream) {
+  return nsa_range_dkdv_as(mode, q, k, v, dout, coff, dot, dk, dv, dkdv_part, part_bytes, B, Hq, Hkv, T, Lk, D, window,
+                           cmp_block, cmp_stride, dtype, NSA_F32, stream);
+}
+
+int nsa_range_dkdv_as(int mode, const void* q, const void* k, const void* v, const void* dout, const float* coff,
+                      const float* dot, void* dk, void* dv, float* dkdv_part, size_t part_bytes, int B, int Hq,
+                      int Hkv, int T, int Lk, int D, int window, int cmp_block, int cmp_stride, int dtype,
+                      int out_dtype, void* stream) {
   NSA_CHECK(mode == NSA_MODE_WINDOW || mode == NSA_MODE_COMPRESS, NSA_ERR_ARG);
   NSA_CHECK(B > 0 && Hkv > 0 && Hq % Hkv == 0 && T >= 0 && Lk >= 0, NSA_ERR_SHAPE);
   NSA_CHECK(D == 16 || D == 32 || D == 64 || D == 128, NSA_ERR_SHAPE);
   NSA_CHECK(mode == NSA_MODE_COMPRESS || (window >= 1 && Lk == T), NSA_ERR_SHAPE);
   NSA_CHECK(mode == NSA_MODE_WINDOW || (cmp_block >= 1 && cmp_stride >= 1), NSA_ERR_SHAPE);
   NSA_CHECK(dtype == NSA_F32 || dtype == NSA_BF16, NSA_ERR_DTYPE);
+  // a bf16 result has one writer per element: it needs the partial rows where
+  // several workgroups add (compression)
+  NSA_CHECK(out_dtype == NSA_F32 || (out_dtype == NSA_BF16 && dtype == NSA_BF16), NSA_ERR_DTYPE);
+  NSA_CHECK(out_dtype == NSA_F32 || mode == NSA_MODE_WINDOW || dkdv_part != nullptr, NSA_ERR_ARG);
   // the tile loads address a group's Q / dO rows with 32-bit byte offsets
   NSA_CHECK((int64_t)(Hq / Hkv) * T * D * (dtype == NSA_BF16 ? 2 : 4) < (1ll << 32), NSA_ERR_SHAPE);
   hipStream_t s = (hipStream_t)stream;
@@ -1679,8 +1755,8 @@ int nsa_range_dkdv(int mode, const void* q, const void* k, const void* v, const 
   const bool partial = dkdv_part != nullptr && grid > 0 && (mode == NSA_MODE_COMPRESS || r.spl > 1);
   NSA_CHECK(!partial || part_bytes >= range_part_bytes(grid, D), NSA_ERR_WORKSPACE);
   if ((mode == NSA_MODE_COMPRESS && !partial) || T == 0) {
-    int rc = zero_f32(dk, nel, s);
-    if (rc == NSA_OK) rc = zero_f32(dv, nel, s);
+    int rc = zero_out(dk, nel, out_dtype, s);
+    if (rc == NSA_OK) rc = zero_out(dv, nel, out_dtype, s);
     if (rc != NSA_OK) return rc;
   }
   if (grid == 0) return NSA_OK;
@@ -1691,20 +1767,28 @@ int nsa_range_dkdv(int mode, const void* q, const void* k, const void* v, const 
   const int64_t part_half = grid * 32 * NW * D;
   // groups of G < 16 heads: query tiles of 32 consecutive (query, head) rows
   const bool flat = Hq / Hkv < 16;
+  float* dk32 = out_dtype == NSA_F32 ? (float*)dk : nullptr;
+  float* dv32 = out_dtype == NSA_F32 ? (float*)dv : nullptr;
+  bf16* dk16 = out_dtype == NSA_F32 ? nullptr : (bf16*)dk;
+  bf16* dv16 = out_dtype == NSA_F32 ? nullptr : (bf16*)dv;
   NSA_DISPATCH_D(D, {
     if (dtype == NSA_BF16) {
       auto kern = flat ? k_range_dkdv_split<bf16, DD, NW, true> : k_range_dkdv_split<bf16, DD, NW, false>;
       kern<<<(unsigned)grid, 128 * NW, 0, s>>>(r, (const bf16*)q, (const bf16*)dout, coff, dot, (const bf16*)k,
-                                               (const bf16*)v, dk, dv, part, part_half, Hq, Hkv, sl2, scale);
+                                               (const bf16*)v, dk32, dv32, dk16, dv16, part, part_half, Hq, Hkv, sl2,
+                                               scale);
     } else {
       auto kern = flat ? k_range_dkdv32<float, DD, NW, true> : k_range_dkdv32<float, DD, NW, false>;
       kern<<<(unsigned)grid, 64 * NW, 0, s>>>(r, (const float*)q, (const float*)dout, coff, dot, (const float*)k,
-                                              (const float*)v, dk, dv, part, part_half, Hq, Hkv, sl2, scale);
+                                              (const float*)v, dk32, dv32, part, part_half, Hq, Hkv, sl2, scale);
     }
     if (partial) {
       if (hipGetLastError() != hipSuccess) return NSA_ERR_LAUNCH;
-      const int64_t total = (int64_t)r.nbh * Lk * (DD / 4);
-      k_range_dkdv_reduce<DD, NW><<<(unsigned)((total + 255) / 256), 256, 0, s>>>(r, part, part_half, dk, dv);
+      const unsigned rg = (unsigned)(((int64_t)r.nbh * Lk * (DD / 4) + 255) / 256);
+      if (out_dtype == NSA_F32)
+        k_range_dkdv_reduce<DD, NW, float><<<rg, 256, 0, s>>>(r, part, part_half, dk32, dv32);
+      else
+        k_range_dkdv_reduce<DD, NW, bf16><<<rg, 256, 0, s>>>(r, part, part_half, dk16, dv16);
     }
   });
   return nsa_launch_status();
@@ -1732,6 +1816,16 @@ int nsa_sel_dkdv(const void* q, const void* k, const void* v, const void* kt, co
                  float* dk, float* dv, float* dkdv_part, size_t part_bytes, void* dq_part, void* workspace,
                  size_t workspace_bytes, int B, int Hq, int Hkv, int T, int D, int S, int block_size, int chunk,
                  int dtype, void* stream) {
+  return nsa_sel_dkdv_as(q, k, v, kt, dout, coff, dot, q_of_block, packed, block_offsets, pair_count, dk, dv,
+                         dkdv_part, part_bytes, dq_part, workspace, workspace_bytes, B, Hq, Hkv, T, D, S, block_size,
+                         chunk, dtype, NSA_F32, stream);
+}
+
+int nsa_sel_dkdv_as(const void* q, const void* k, const void* v, const void* kt, const void* dout, const float* coff,
+                    const float* dot, const int32_t* q_of_block, int packed, const int32_t* block_offsets,
+                    const int32_t* pair_count, void* dk, void* dv, float* dkdv_part, size_t part_bytes, void* dq_part,
+                    void* workspace, size_t workspace_bytes, int B, int Hq, int Hkv, int T, int D, int S,
+                    int block_size, int chunk, int dtype, int out_dtype, void* stream) {
   (void)pair_count;
   NSA_CHECK(B > 0 && Hkv > 0 && Hq % Hkv == 0 && T >= 0 && S >= 0, NSA_ERR_SHAPE);
   NSA_CHECK(D == 16 || D == 32 || D == 64 || D == 128, NSA_ERR_SHAPE);
@@ -1741,6 +1835,9 @@ int nsa_sel_dkdv(const void* q, const void* k, const void* v, const void* kt, co
   NSA_CHECK(dkdv_part == nullptr || part_bytes >= nsa_sel_dkdv_partial_bytes(B, Hkv, T, S, D, block_size, chunk),
             NSA_ERR_WORKSPACE);
   NSA_CHECK(dq_part == nullptr || (packed && kt != nullptr), NSA_ERR_ARG);
+  // a bf16 result is written by the reduce of the partial rows
+  NSA_CHECK(out_dtype == NSA_F32 || (out_dtype == NSA_BF16 && dtype == NSA_BF16), NSA_ERR_DTYPE);
+  NSA_CHECK(out_dtype == NSA_F32 || dkdv_part != nullptr, NSA_ERR_ARG);
   NSA_CHECK(!packed || ((int64_t)T << sel_slot_bits(S)) < (1ll << 31), NSA_ERR_SHAPE);
   // the tile loads address a group's Q / dO rows with 32-bit byte offsets
   NSA_CHECK((int64_t)(Hq / Hkv) * T * D * (dtype == NSA_BF16 ? 2 : 4) < (1ll << 32), NSA_ERR_SHAPE);
@@ -1750,11 +1847,13 @@ int nsa_sel_dkdv(const void* q, const void* k, const void* v, const void* kt, co
   const bool empty = T == 0 || S == 0 || n_blk == 0;
   if (dkdv_part == nullptr || empty) {
     // atomics add into zeroed outputs (the partial reduce writes every key)
-    int rc = zero_f32(dk, nel, s);
-    if (rc == NSA_OK) rc = zero_f32(dv, nel, s);
+    int rc = zero_out(dk, nel, out_dtype, s);
+    if (rc == NSA_OK) rc = zero_out(dv, nel, out_dtype, s);
     if (rc != NSA_OK) return rc;
   }
   if (empty) return NSA_OK;
+  float* dk32 = out_dtype == NSA_F32 ? (float*)dk : nullptr;
+  float* dv32 = out_dtype == NSA_F32 ? (float*)dv : nullptr;
   const size_t cap = sel_items_cap(B, Hkv, T, S, block_size, chunk);
   int4* items = (int4*)workspace;
   int32_t* n_items = (int32_t*)((char*)workspace + cap * sizeof(int4));
@@ -1776,21 +1875,26 @@ int nsa_sel_dkdv(const void* q, const void* k, const void* v, const void* kt, co
       auto kern = gp ? k_sel_dkdv32<bf16, DD, true> : k_sel_dkdv32<bf16, DD, false>;
       kern<<<(unsigned)grid_cap, 128, 0, s>>>(
           (const bf16*)q, (const bf16*)dout, coff, dot, (const bf16*)k, (const bf16*)v, (const bf16*)kt, q_of_block,
-          items, n_items, dk, dv, dkdv_part, part_half, (bf16*)dq_part, Hq, Hkv, T, S, packed, n_blk, block_size,
+          items, n_items, dk32, dv32, dkdv_part, part_half, (bf16*)dq_part, Hq, Hkv, T, S, packed, n_blk, block_size,
           Lp, sl2, scale);
     } else {
       auto kern = gp ? k_sel_dkdv32<float, DD, true> : k_sel_dkdv32<float, DD, false>;
       kern<<<(unsigned)grid_cap, 128, 0, s>>>(
           (const float*)q, (const float*)dout, coff, dot, (const float*)k, (const float*)v, (const float*)kt,
-          q_of_block, items, n_items, dk, dv, dkdv_part, part_half, (float*)dq_part, Hq, Hkv, T, S, packed, n_blk,
+          q_of_block, items, n_items, dk32, dv32, dkdv_part, part_half, (float*)dq_part, Hq, Hkv, T, S, packed, n_blk,
           block_size, Lp, sl2, scale);
     }
     if (dkdv_part != nullptr) {
       if (hipGetLastError() != hipSuccess) return NSA_ERR_LAUNCH;
       const int npass = sel_passes(block_size);
       const int64_t total = (int64_t)nb * npass * kSelPass * (DD / 4);
-      k_sel_dkdv_reduce<DD><<<(unsigned)((total + 255) / 256), 256, 0, s>>>(dkdv_part, part_half, first, dk, dv, T,
-                                                                              n_blk, block_size, npass, total);
+      const unsigned rg = (unsigned)((total + 255) / 256);
+      if (out_dtype == NSA_F32)
+        k_sel_dkdv_reduce<DD, float><<<rg, 256, 0, s>>>(dkdv_part, part_half, first, dk32, dv32, T, n_blk, block_size,
+                                                        npass, total);
+      else
+        k_sel_dkdv_reduce<DD, bf16><<<rg, 256, 0, s>>>(dkdv_part, part_half, first, (bf16*)dk, (bf16*)dv, T, n_blk,
+                                                       block_size, npass, total);
     }
   });
   return nsa_launch_status();

@@ -11,7 +11,7 @@
 //              (float32), their lse, the block -> query CSR;
 //   scratch -- transient, any contents on entry: transposed K/V copies, the
 //              selection partials of the forward, then the backward's row
-//              statistics, float32 dK/dV accumulators, dQ partials and the
+//              statistics, dQ partials, pooled-key gradients and the
 //              deterministic-merge partial rows.
 #include <cstddef>
 #include <cstdint>
@@ -111,7 +111,7 @@ FwdScratch carve_fwd(const Dims& m, void* base, size_t* bytes) {
 }
 
 struct BwdScratch {
-  float *dot, *rs, *coff, *dks, *dvs, *dkw, *dvw, *dkp, *dvp, *sel_part, *cmp_part, *win_part;
+  float *dot, *rs, *coff, *dkp, *dvp, *sel_part, *cmp_part, *win_part;
   void *dop, *kt_s, *dq_part, *sel_ws, *kt_w, *kt_c;
   size_t sel_bytes, sel_part_bytes, cmp_part_bytes, win_part_bytes;
 };
@@ -122,24 +122,20 @@ BwdScratch carve_bwd(const Dims& m, void* base, size_t* bytes, hipStream_t s) {
   BwdScratch x{};
   const int n = m.ncmp(), S = m.S();
   const int ns = nsa_sel_partial_slots(S, m.ls);
-  const bool f32 = m.dtype == NSA_F32;   // float32 gradients go straight to the caller's outputs
   x.dot = (float*)c.take(3 * m.rows() * sizeof(float));
   x.rs = (float*)c.take(3 * m.rows() * sizeof(float));
   x.coff = (float*)c.take(3 * m.rows() * sizeof(float));
   x.dop = c.take((size_t)m.rows() * m.D * m.es());
   x.kt_s = c.take((size_t)m.B * m.Hkv * m.D * nsa_padded_len(m.T) * m.es());
-  x.dks = f32 ? nullptr : (float*)c.take(m.kv(m.T) * sizeof(float));
-  x.dvs = f32 ? nullptr : (float*)c.take(m.kv(m.T) * sizeof(float));
   x.dq_part = c.take((size_t)m.rows() * ns * m.D * m.es());
   x.sel_bytes = nsa_sel_dkdv_workspace(m.B, m.Hkv, m.T, S, m.ls, m.dkdv_chunk());
   x.sel_ws = c.take(x.sel_bytes);
   x.sel_part_bytes = nsa_sel_dkdv_partial_bytes(m.B, m.Hkv, m.T, S, m.D, m.ls, m.dkdv_chunk());
   x.sel_part = (float*)c.take(x.sel_part_bytes);
   x.kt_w = c.take((size_t)m.B * m.Hkv * m.D * nsa_padded_len(m.T) * m.es());
-  x.dkw = f32 ? nullptr : (float*)c.take(m.kv(m.T) * sizeof(float));
-  x.dvw = f32 ? nullptr : (float*)c.take(m.kv(m.T) * sizeof(float));
-  x.dkp = (f32 && m.pooled) ? nullptr : (float*)c.take(m.kv(n) * sizeof(float));
-  x.dvp = (f32 && m.pooled) ? nullptr : (float*)c.take(m.kv(n) * sizeof(float));
+  // the pooled keys' gradients before the pooling's backward (pooled inputs: the caller's outputs)
+  x.dkp = m.pooled ? nullptr : (float*)c.take(m.kv(n) * sizeof(float));
+  x.dvp = m.pooled ? nullptr : (float*)c.take(m.kv(n) * sizeof(float));
   x.cmp_part_bytes = nsa_range_dkdv_partial_bytes(NSA_MODE_COMPRESS, m.B, m.Hkv, m.T, n, m.D, m.l, m.d, s);
   x.cmp_part = (float*)c.take(x.cmp_part_bytes);
   // the window's dK/dV parts (0 bytes where it is not split)
@@ -257,47 +253,33 @@ int nsa_fused_bwd(const void* dout, const void* q, const void* kc, const void* v
   NSA_CHECK(scratch_bytes >= sb, NSA_ERR_WORKSPACE);
   const int n = m.ncmp(), S = m.S(), G = m.G(), Lpn = nsa_padded_len(n), Lpt = nsa_padded_len(T);
   const int64_t R = m.rows();
-  const bool f32 = dtype == NSA_F32;
   const void* k_cmp = pooled ? kc : x.k_cmp;
   const void* v_cmp = pooled ? vc : x.v_cmp;
-  float* dks32 = f32 ? (float*)dks : w.dks;
-  float* dvs32 = f32 ? (float*)dvs : w.dvs;
-  float* dkw32 = f32 ? (float*)dkw : w.dkw;
-  float* dvw32 = f32 ? (float*)dvw : w.dvw;
-  float* dkp32 = (f32 && pooled) ? (float*)dkc : w.dkp;
-  float* dvp32 = (f32 && pooled) ? (float*)dvc : w.dvp;
+  void* dkp = pooled ? dkc : (void*)w.dkp;
+  void* dvp = pooled ? dvc : (void*)w.dvp;
   // gate backward, row dots of the three branches, dO packed for the selection
   NSA_TRY(nsa_bwd_prep(dout, x.o_c, x.o_s, x.o_w, gate, dgate, x.lse_c, x.lse_s, x.lse_w, w.dot, w.rs, w.coff,
                        w.dop, G, T, R, D, 3, dtype, m.o_dtype(), dtype, stream));
   // selection dK/dV and dQ partials (block-outer, deterministic merge)
   NSA_TRY(nsa_transpose_kv(ks, w.kt_s, B * Hkv, T, D, Lpt, dtype, stream));
-  NSA_TRY(nsa_sel_dkdv(x.qp, ks, vs, w.kt_s, w.dop, w.coff + R, w.dot + R, x.q_of_block, 1, x.offsets, x.count,
-                       dks32, dvs32, w.sel_part, w.sel_part_bytes, w.dq_part, w.sel_ws, w.sel_bytes, B, Hq, Hkv, T, D,
-                       S, sel_block, m.dkdv_chunk(), dtype, stream));
+  NSA_TRY(nsa_sel_dkdv_as(x.qp, ks, vs, w.kt_s, w.dop, w.coff + R, w.dot + R, x.q_of_block, 1, x.offsets, x.count,
+                          dks, dvs, w.sel_part, w.sel_part_bytes, w.dq_part, w.sel_ws, w.sel_bytes, B, Hq, Hkv, T, D,
+                          S, sel_block, m.dkdv_chunk(), dtype, dtype, stream));
   // window and compression dK/dV
   NSA_TRY(nsa_transpose_kv(kw, w.kt_w, B * Hkv, T, D, Lpt, dtype, stream));
-  NSA_TRY(nsa_range_dkdv(NSA_MODE_WINDOW, q, kw, vw, dout, w.coff + 2 * R, w.dot + 2 * R, dkw32, dvw32, w.win_part,
-                         w.win_part_bytes, B, Hq, Hkv, T, T, D, window, 1, 1, dtype, stream));
-  NSA_TRY(nsa_range_dkdv(NSA_MODE_COMPRESS, q, k_cmp, v_cmp, dout, w.coff, w.dot, dkp32, dvp32, w.cmp_part,
-                         w.cmp_part_bytes, B, Hq, Hkv, T, n, D, 0, cmp_block, cmp_stride, dtype, stream));
+  NSA_TRY(nsa_range_dkdv_as(NSA_MODE_WINDOW, q, kw, vw, dout, w.coff + 2 * R, w.dot + 2 * R, dkw, dvw, w.win_part,
+                            w.win_part_bytes, B, Hq, Hkv, T, T, D, window, 1, 1, dtype, dtype, stream));
+  NSA_TRY(nsa_range_dkdv_as(NSA_MODE_COMPRESS, q, k_cmp, v_cmp, dout, w.coff, w.dot, dkp, dvp, w.cmp_part,
+                            w.cmp_part_bytes, B, Hq, Hkv, T, n, D, 0, cmp_block, cmp_stride, dtype,
+                            pooled ? dtype : NSA_F32, stream));
   // compression + window dQ in one launch, rows finished with the selection partials
   NSA_TRY(nsa_transpose_kv(k_cmp, w.kt_c, B * Hkv, n, D, Lpn, dtype, stream));
   NSA_TRY(nsa_range_dq_cw(q, dout, k_cmp, v_cmp, w.kt_c, x.lse_c, w.dot, w.rs, n, cmp_block, cmp_stride, kw, vw,
                           w.kt_w, x.lse_w, w.dot + 2 * R, w.rs + 2 * R, window, B, Hq, Hkv, T, D, w.dq_part, block_idx,
                           S, sel_block, dq, dtype, dtype, stream));
-  // the key / value gradients in the input dtype
   if (!pooled) {
-    NSA_TRY(nsa_pool_bwd(dkp32, NSA_F32, dkc, B, Hkv, T, D, cmp_block, cmp_stride, dtype, stream));
-    NSA_TRY(nsa_pool_bwd(dvp32, NSA_F32, dvc, B, Hkv, T, D, cmp_block, cmp_stride, dtype, stream));
-  } else if (!f32) {
-    NSA_TRY(nsa_cast_f32(dkp32, dkc, m.kv(n), dtype, stream));
-    NSA_TRY(nsa_cast_f32(dvp32, dvc, m.kv(n), dtype, stream));
-  }
-  if (!f32) {
-    NSA_TRY(nsa_cast_f32(dks32, dks, m.kv(T), dtype, stream));
-    NSA_TRY(nsa_cast_f32(dvs32, dvs, m.kv(T), dtype, stream));
-    NSA_TRY(nsa_cast_f32(dkw32, dkw, m.kv(T), dtype, stream));
-    NSA_TRY(nsa_cast_f32(dvw32, dvw, m.kv(T), dtype, stream));
+    NSA_TRY(nsa_pool_bwd(dkp, NSA_F32, dkc, B, Hkv, T, D, cmp_block, cmp_stride, dtype, stream));
+    NSA_TRY(nsa_pool_bwd(dvp, NSA_F32, dvc, B, Hkv, T, D, cmp_block, cmp_stride, dtype, stream));
   }
   return NSA_OK;
 }

@@ -530,10 +530,8 @@ __global__ __launch_bounds__(256) void k_sel_merge(const int32_t* __restrict__ i
     const float inv = Ls > 0.0f ? 1.0f / Ls : 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] *= inv;
-    if (o32 != nullptr)
-      store8(o32 + orow * D + 8 * c, acc);
-    else
-      store8(o + orow * D + 8 * c, acc);
+    if (o32 != nullptr) store8(o32 + orow * D + 8 * c, acc);
+    if (o != nullptr) store8(o + orow * D + 8 * c, acc);
     if (c == 0) lse[orow] = Ls > 0.0f ? (M + __log2f(Ls)) * kLn2 : kLseEmpty;
   }
 }
@@ -657,10 +655,19 @@ int nsa_sel_fwd_bo(const void* q, const void* k, const void* vt, const int32_t* 
 
 int nsa_sel_merge(const int32_t* block_idx, const void* o_part, const float* ml_part, void* o, float* lse, int B,
                   int Hq, int Hkv, int T, int D, int S, int block_size, int dtype, int o_dtype, void* stream) {
-  NSA_CHECK(sel_args_ok(B, Hq, Hkv, T, D, S, block_size), NSA_ERR_SHAPE);
   NSA_CHECK(dtype == NSA_F32 || dtype == NSA_BF16, NSA_ERR_DTYPE);
   NSA_CHECK(o_dtype == dtype || o_dtype == NSA_F32, NSA_ERR_DTYPE);
-  float* o32 = o_dtype == NSA_F32 && dtype != NSA_F32 ? (float*)o : nullptr;
+  const bool f32 = o_dtype == NSA_F32 && dtype != NSA_F32;
+  return nsa_sel_merge_both(block_idx, o_part, ml_part, f32 ? nullptr : o, f32 ? (float*)o : nullptr, lse, B, Hq, Hkv,
+                            T, D, S, block_size, dtype, stream);
+}
+
+int nsa_sel_merge_both(const int32_t* block_idx, const void* o_part, const float* ml_part, void* o, float* o32,
+                       float* lse, int B, int Hq, int Hkv, int T, int D, int S, int block_size, int dtype,
+                       void* stream) {
+  NSA_CHECK(sel_args_ok(B, Hq, Hkv, T, D, S, block_size), NSA_ERR_SHAPE);
+  NSA_CHECK(dtype == NSA_F32 || dtype == NSA_BF16, NSA_ERR_DTYPE);
+  NSA_CHECK(dtype == NSA_BF16 || o32 == nullptr, NSA_ERR_ARG);
   const int64_t total = (int64_t)B * Hq * T * (D / 8);
   if (total == 0) return NSA_OK;
   hipStream_t s = (hipStream_t)stream;
@@ -668,8 +675,8 @@ int nsa_sel_merge(const int32_t* block_idx, const void* o_part, const float* ml_
   NSA_DISPATCH_D(D, {
     if (dtype == NSA_BF16)
       k_sel_merge<bf16, DD><<<grid_for(total), 256, 0, s>>>(block_idx, (const f16*)o_part, (const float2*)ml_part,
-                                                            o32 ? nullptr : (bf16*)o, lse, Hq, Hkv, T, S, n_csr,
-                                                            block_size, nsub, total, o32);
+                                                            (bf16*)o, lse, Hq, Hkv, T, S, n_csr, block_size, nsub,
+                                                            total, o32);
     else
       k_sel_merge<float, DD><<<grid_for(total), 256, 0, s>>>(block_idx, (const float*)o_part,
                                                              (const float2*)ml_part, (float*)o, lse, Hq, Hkv, T, S,

@@ -715,9 +715,9 @@ def csr_device(block_idx, block_size, n_blk=None, pack_slot=False):
 
 
 def sel_dkdv(q, k, v, do, coff, dot, block_idx, block_size, csr=None, kt=None, want_dq=False, qp=None,
-             dop=None, stats_packed=False):
-    """dK, dV (float32) of the selection branch over the block -> query CSR;
-    with ``want_dq`` also the dQ partials of every (query, slot, pass) for
+             dop=None, stats_packed=False, out_dtype=torch.float32):
+    """dK, dV of the selection branch over the block -> query CSR (float32, or
+    rounded once to ``out_dtype``); with ``want_dq`` also the dQ partials of every (query, slot, pass) for
     ``sel_dq_reduce`` (the CSR must then be built with ``pack_slot``).
     ``qp`` / ``dop``: ``pack_heads`` copies of q / do (made here when not
     given).  ``coff`` / ``dot``: [B, Hq, T], or with ``stats_packed`` already
@@ -739,7 +739,8 @@ def sel_dkdv(q, k, v, do, coff, dot, block_idx, block_size, csr=None, kt=None, w
     if csr is None:
         csr = csr_device(idx, block_size, pack_slot=want_dq)
     q_of_block, offsets, _, count = csr
-    dk = torch.empty(B, Hkv, T, D, device=q.device, dtype=torch.float32)
+    dt = torch.float32 if not DETERMINISTIC_DKDV else out_dtype   # atomic merges add in float32
+    dk = torch.empty(B, Hkv, T, D, device=q.device, dtype=dt)
     dv = torch.empty_like(dk)
     dq_part = None
     if want_dq:
@@ -754,10 +755,12 @@ def sel_dkdv(q, k, v, do, coff, dot, block_idx, block_size, csr=None, kt=None, w
     if DETERMINISTIC_DKDV:
         part_bytes = int(_lib().nsa_sel_dkdv_partial_bytes(B, Hkv, T, S, D, block_size, chunk))
         part = torch.empty(max(part_bytes // 4, 1), device=q.device, dtype=torch.float32)
-    _call("dkdv[sel]", _lib().nsa_sel_dkdv, L.ptr(qp), L.ptr(k), L.ptr(v), L.ptr(kt), L.ptr(dop), L.ptr(coff),
+    _call("dkdv[sel]", _lib().nsa_sel_dkdv_as, L.ptr(qp), L.ptr(k), L.ptr(v), L.ptr(kt), L.ptr(dop), L.ptr(coff),
           L.ptr(dot), L.ptr(q_of_block), int(want_dq), L.ptr(offsets),
           L.ptr(count), L.ptr(dk), L.ptr(dv), L.ptr(part), part_bytes, L.ptr(dq_part), L.ptr(ws), ws_bytes, B, Hq,
-          Hkv, T, D, S, block_size, chunk, L.dtype_code(q), _stream(q))
+          Hkv, T, D, S, block_size, chunk, L.dtype_code(q), L.dtype_code(dk), _stream(q))
+    if dt != out_dtype:
+        dk, dv = cast_f32(dk, out_dtype), cast_f32(dv, out_dtype)
     return dk, dv, dq_part
 
 
@@ -784,19 +787,21 @@ def sel_dq_reduce(block_idx, dq_part, dq_acc, block_size, dtype):
     return out if dtype == out.dtype else out.to(dtype)
 
 
-def sel_fwd_fsa(q, k, v, block_idx, block_size, csr=None, vt=None, qp=None, o_f32=False):
+def sel_fwd_fsa(q, k, v, block_idx, block_size, csr=None, vt=None, qp=None, o_f32=False, o_both=False):
     """Block-outer selection forward -> (o, lse[f32], csr); ``csr`` is the
     packed block -> query CSR (built here when not given), ``qp`` the
     ``pack_heads`` copy of q (made here when not given).  ``o_f32``: o in
-    float32 (unrounded), else in q's dtype."""
+    float32 (unrounded), else in q's dtype; ``o_both``: the pair (o in q's
+    dtype, o in float32)."""
     parts, csr = sel_fwd_partials(q, k, v, block_idx, block_size, csr, vt, qp)
-    o, lse = sel_merge(block_idx, parts, q.shape, k.shape[1], block_size, o_f32=o_f32)
+    o, lse = sel_merge(block_idx, parts, q.shape, k.shape[1], block_size, o_f32=o_f32, o_both=o_both)
     return o, lse, csr
 
 
-def sel_merge(block_idx, parts, q_shape, Hkv, block_size, o_f32=False):
+def sel_merge(block_idx, parts, q_shape, Hkv, block_size, o_f32=False, o_both=False):
     """The selection output and lse of every row from the partials of
-    ``sel_fwd_partials`` (o in the inputs' dtype, or float32 unrounded)."""
+    ``sel_fwd_partials`` (o in the inputs' dtype, or float32 unrounded; with
+    ``o_both`` the pair, which is one tensor for float32 inputs)."""
     o_part, ml_part = parts
     B, Hq, T, D = q_shape
     idx = block_idx.to(torch.int32).contiguous()
@@ -807,12 +812,16 @@ def sel_merge(block_idx, parts, q_shape, Hkv, block_size, o_f32=False):
             or ml_part.dtype != torch.float32 or not ml_part.is_contiguous():
         raise ValueError("o_part / ml_part must hold the [B, Hkv, T, slots, G] partials of block_idx")
     dt = _partial_input_dtype(o_part)
-    o = torch.empty(q_shape, device=o_part.device, dtype=torch.float32 if o_f32 else dt)
+    want32 = dt != torch.float32 and (o_f32 or o_both)
+    o = torch.empty(q_shape, device=o_part.device, dtype=dt) if o_both or not want32 else None
+    o32 = torch.empty(q_shape, device=o_part.device, dtype=torch.float32) if want32 else None
     lse = torch.empty(B, Hq, T, device=o_part.device, dtype=torch.float32)
-    _call("nsa_sel_merge", _lib().nsa_sel_merge, L.ptr(idx), L.ptr(o_part), L.ptr(ml_part), L.ptr(o), L.ptr(lse), B,
-          Hq, Hkv, T, D, idx.shape[-1], block_size, L.NSA_BF16 if dt == torch.bfloat16 else L.NSA_F32,
-          L.dtype_code(o), _stream(o_part))
-    return o, lse
+    _call("nsa_sel_merge", _lib().nsa_sel_merge_both, L.ptr(idx), L.ptr(o_part), L.ptr(ml_part), L.ptr(o), L.ptr(o32),
+          L.ptr(lse), B, Hq, Hkv, T, D, idx.shape[-1], block_size, L.NSA_BF16 if dt == torch.bfloat16 else L.NSA_F32,
+          _stream(o_part))
+    if o_both:
+        return (o, o if o32 is None else o32), lse
+    return o if o32 is None else o32, lse
 
 
 def _partial_dtype(dtype):
@@ -895,8 +904,7 @@ class SelectionAttnHIP(torch.autograd.Function):
         # and dK (the same choice as the fused layer's branch outputs)
         # the packed Q copy both block-outer kernels read, made once
         qp = pack_heads(q, k.shape[1])
-        o32, lse, csr = sel_fwd_fsa(q, k, v, idx, block_size, qp=qp, o_f32=q.dtype != torch.float32)
-        o = cast_f32(o32, q.dtype)
+        (o, o32), lse, csr = sel_fwd_fsa(q, k, v, idx, block_size, qp=qp, o_both=True)
         ctx.save_for_backward(q, k, v, idx, o32, lse, qp, *csr)
         ctx.block_size = block_size
         return o
@@ -936,11 +944,8 @@ def selection_backward_fsa(q, k, v, block_idx, block_size, do, o, lse, csr=None,
     idx = block_idx.to(torch.int32).contiguous()
     dot, coff, dop = delta_of(do, o, lse, pack_hkv=k.shape[1])
     dk, dv, dq_part = sel_dkdv(q, k, v, do, coff, dot, idx, block_size, csr=csr, want_dq=True, qp=qp, dop=dop,
-                               stats_packed=True)
-    dq = sel_dq_reduce(idx, dq_part, None, block_size, q.dtype)
-    if grads_f32:
-        return dq, dk, dv
-    return dq, cast_f32(dk, k.dtype), cast_f32(dv, v.dtype)
+                               stats_packed=True, out_dtype=torch.float32 if grads_f32 else k.dtype)
+    return sel_dq_reduce(idx, dq_part, None, block_size, q.dtype), dk, dv
 
 
 class RangeAttnHIP(torch.autograd.Function):
