@@ -508,6 +508,14 @@ int nsa_decode_append(void* kc, void* vc, void* ks, void* vs, void* kw, void* vw
                       const void* kc_new, const void* vc_new, const void* ks_new, const void* vs_new,
                       const void* kw_new, const void* vw_new, const int32_t* lens_in, int32_t* lens_out, int B,
                       int Hkv, int D, int Tcap, int Ncap, int cmp_block, int cmp_stride, int dtype, void* stream);
+/* nsa_decode_append, then nsa_decode_fwd over the new lengths (lens_out). */
+int nsa_decode_step(void* kc, void* vc, void* ks, void* vs, void* kw, void* vw, void* k_cmp, void* v_cmp,
+                    const void* kc_new, const void* vc_new, const void* ks_new, const void* vs_new, const void* kw_new,
+                    const void* vw_new, const int32_t* lens_in, int32_t* lens_out, const void* q, const void* gate,
+                    void* out, int32_t* block_idx, void* workspace, size_t workspace_bytes, int B, int Hq, int Hkv,
+                    int D, int Tcap, int Ncap, int cmp_block, int cmp_stride, int sel_block, int n_sel, int window,
+                    int force_init, int n_local, int dtype, void* stream);
+
 
 #ifdef __cplusplus
 }

@@ -98,6 +98,7 @@ SIGNATURES = {
     "nsa_decode_workspace": (_Z, [_I] * 11),
     "nsa_decode_fwd": (_I, [_P] * 15 + [_Z] + [_I] * 14 + [_P]),
     "nsa_decode_append": (_I, [_P] * 16 + [_I] * 8 + [_P]),
+    "nsa_decode_step": (_I, [_P] * 21 + [_Z] + [_I] * 14 + [_P]),
 }
 
 _lib = None

@@ -134,6 +134,11 @@ class NSADecodeCache:
                                self.geom, workspace=self._workspace(q.shape[1], q.shape[2]), **kw)
 
     def step(self, q, gate, new_rows, **kw):
-        """``append(*new_rows)`` then ``attend(q, gate)``."""
-        self.append(*new_rows)
-        return self.attend(q, gate, **kw)
+        """``append(*new_rows)`` then ``attend(q, gate)``: one library call,
+        unless a compressor pools in between or an extra is asked for."""
+        if self.compressor is not None or kw or _ops._TIMER is not None:
+            self.append(*new_rows)
+            return self.attend(q, gate, **kw)
+        self.lens, out, idx = _ops.decode_step(self.caches(), self.k_cmp, self.v_cmp, new_rows, self.lens, q, gate,
+                                               self.geom, self._workspace(q.shape[1], q.shape[2]))
+        return out, idx

@@ -1471,3 +1471,39 @@ def decode_append(kc, vc, ks, vs, kw, vw, k_cmp, v_cmp, new_rows, lens, geom: NS
           *map(L.ptr, rows), L.ptr(lens), L.ptr(lens_out), B, Hkv, D, Tcap, k_cmp.shape[2], geom.cmp_block,
           geom.cmp_stride, L.dtype_code(kc), _stream(kc))
     return lens_out
+
+
+def decode_step(caches, k_cmp, v_cmp, new_rows, lens, q, gate, geom: NSAGeometry, workspace):
+    """``decode_append`` of ``new_rows``, then ``decode_fwd`` at the new
+    lengths, in one library call -> (new lens, out, block_idx).  ``caches``:
+    kc vc ks vs kw vw; ``workspace``: ``decode_workspace_bytes`` of these
+    sizes.  At one sequence the step's kernels take less than two calls hold
+    the host."""
+    kc = caches[0]
+    B, Hkv, Tcap, D = kc.shape
+    dt = kc.dtype
+    for x in (*caches, k_cmp, v_cmp):
+        assert x.is_contiguous() and x.dtype == dt, "decode_step: caches must be contiguous, one dtype"
+    for x in caches:
+        assert x.shape == kc.shape
+    if any(x.data_ptr() % 16 for x in (*caches, k_cmp, v_cmp)) or workspace.data_ptr() % 256:
+        lens = decode_append(*caches, k_cmp, v_cmp, new_rows, lens, geom)   # (the forward copies such a cache)
+        return (lens, *decode_fwd(q, k_cmp, v_cmp, *caches[2:], gate, lens, geom, workspace=workspace))
+    Ncap = k_cmp.shape[2]
+    assert k_cmp.shape == (B, Hkv, Ncap, D) and v_cmp.shape == k_cmp.shape, "decode: pooled caches [B, Hkv, Ncap, D]"
+    rows = [_contig(r) for r in new_rows]
+    assert len(rows) == 6 and all(r.shape == (B, Hkv, D) and r.dtype == dt for r in rows)
+    assert lens.dtype == torch.int32 and lens.shape == (B,) and lens.is_contiguous() and lens.is_cuda
+    assert q.dim() == 3 and q.is_cuda and q.shape[0] == B and q.shape[2] == D, "decode: q must be [B, Hq, D] on the GPU"
+    Hq = q.shape[1]
+    assert Hq % Hkv == 0, "GQA needs n_q_heads divisible by n_kv_heads"
+    assert gate.shape == (B, Hq, 3) and gate.dtype == dt and q.dtype == dt, "decode: q and gate in the caches' dtype"
+    q, gate = _contig(q), _contig(gate)
+    out = torch.empty_like(q)
+    idx = torch.empty(B, Hkv, geom.n_sel, device=q.device, dtype=torch.int32)
+    lens_out = torch.empty_like(lens)
+    ptrs = [t.data_ptr() for t in (*caches, k_cmp, v_cmp, *rows, lens, lens_out, q, gate, out, idx, workspace)]
+    _call("nsa_decode_step", _lib().nsa_decode_step, *ptrs, workspace.numel() * workspace.element_size(), B, Hq, Hkv,
+          D, Tcap, Ncap, geom.cmp_block, geom.cmp_stride, geom.sel_block, geom.n_sel, geom.window,
+          int(geom.force_init), geom.n_local, L.dtype_code(q), _stream(q))
+    return lens_out, out, idx
