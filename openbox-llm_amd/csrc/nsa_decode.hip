@@ -374,22 +374,27 @@ __device__ __forceinline__ void dec_head_lse2(const DecGeom& g, const float* __r
   }
 }
 
-// p_cmp of pooled tokens i4 .. i4 + 3 of one (b, hkv) summed over the group's
-// heads (each head's four scores in one 16-byte load; heads 0-7, then 8-15,
-// of each 16-head chunk, as the prefill importance kernel sums them)
-__device__ __forceinline__ void dec_token_sums4(const DecGeom& g, const float* __restrict__ s_cmp, int bh, int i4,
-                                                const float* lse2, float sl2, float (&v)[4]) {
-  const float* sc = s_cmp + (int64_t)bh * g.G * g.NcapP;
+// The scores of W consecutive pooled tokens (from i) for the 16 heads of the
+// chunk c0 (one 4 W byte load per head; inside the row pitch, past nvis the
+// values are never used).
+template <int W> struct DecScores {
+  typedef float vec __attribute__((ext_vector_type(W)));
+  vec x[16];
+  __device__ __forceinline__ void load(const DecGeom& g, const float* __restrict__ s_cmp, int bh, int c0, int i) {
+    const float* sc = s_cmp + (int64_t)bh * g.G * g.NcapP;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = 0.0f;
-  for (int c0 = 0; c0 < g.G; c0 += 16) {
-    f32x4 x[16];
+    for (int j = 0; j < 16; ++j) {
+      if (c0 + j < g.G)
+        x[j] = *reinterpret_cast<const vec*>(sc + (int64_t)(c0 + j) * g.NcapP + i);
+      else
+        x[j] = 0.0f;
+    }
+  }
+  // p_cmp summed over the chunk's heads (heads 0-7, then 8-15, as the prefill
+  // importance kernel sums them), added to v for chunks after the first
+  __device__ __forceinline__ void add(const DecGeom& g, int c0, const float* lse2, float sl2, float (&v)[W]) const {
 #pragma unroll
-    for (int j = 0; j < 16; ++j)   // past nvis (inside the row pitch) the values are never used
-      x[j] = c0 + j < g.G ? *reinterpret_cast<const f32x4*>(sc + (int64_t)(c0 + j) * g.NcapP + i4)
-                          : (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < W; ++e) {
       float half[2];
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
@@ -403,6 +408,19 @@ __device__ __forceinline__ void dec_token_sums4(const DecGeom& g, const float* _
       }
       v[e] = c0 == 0 ? half[0] + half[1] : v[e] + (half[0] + half[1]);
     }
+  }
+};
+
+// p_cmp of pooled tokens i4 .. i4 + 3 of one (b, hkv) summed over the group's
+// heads
+__device__ __forceinline__ void dec_token_sums4(const DecGeom& g, const float* __restrict__ s_cmp, int bh, int i4,
+                                                const float* lse2, float sl2, float (&v)[4]) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = 0.0f;
+  for (int c0 = 0; c0 < g.G; c0 += 16) {
+    DecScores<4> x;
+    x.load(g, s_cmp, bh, c0, i4);
+    x.add(g, c0, lse2, sl2, v);
   }
 }
 
@@ -438,10 +456,12 @@ __global__ __launch_bounds__(256) void k_dec_toksum(const DecArgs<T> a, int nch)
 // tokens ascending, weighted by overlap / cd.  Its key is (order key of the
 // score: +inf forced, -FLT_MAX incomplete) << 32 | ~j, unique, so the top S
 // keys are the highest scores with ties to the lower block.  They are found
-// by radix selection (eight 8-bit digits from the top: a histogram of the
-// keys that match the digits fixed so far, and the digit at which the count
-// from the top reaches the picks still needed), gathered, and sorted
-// descending across the lanes of one wave.  FUSE: the workgroup forms the
+// by radix selection (8-bit digits from the top: a histogram of the keys that
+// match the digits fixed so far, and the digit at which the count from the
+// top reaches the picks still needed) until the bucket at that digit is picked
+// whole or holds at most 64 keys, and ranked by one wave: the count of keys
+// above each takes S steps of a few instructions, a bitonic sort 21 exchanges.
+// Bound by its chain of latencies (one CU per (b, hkv)): PH_TOPN.  FUSE: the workgroup forms the
 // token sums itself (k_dec_toksum's arithmetic, so the same bits) instead of
 // reading them, one launch and one round trip less when the pooled sequence
 // is short.
@@ -454,25 +474,35 @@ __global__ __launch_bounds__(kDecTopnThreads) void k_dec_topn(const int32_t* __r
                                                              const float* __restrict__ s_cmp, float sl2) {
   __shared__ uint32_t hist[2][256];
   __shared__ uint64_t ctl_prefix;
-  __shared__ int ctl_need;
-  __shared__ uint64_t picked[kDecMaxSel];
-  __shared__ int npicked;
+  __shared__ int ctl_need, ctl_left;
+  __shared__ uint64_t picked[kDecMaxSel], match[kWave];
+  __shared__ int npicked, nmatch;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int bh = blockIdx.x, b = bh / g.Hkv;
   const DecLen L = dec_len(lens[b], g);
   int32_t* orow = idx + (int64_t)bh * g.n_sel;
   extern __shared__ __align__(16) float tk[];   // token sums [NcapP] (FUSE: then lse2 [G])
   if (tid < 256) hist[0][tid] = 0;
-  if (tid == 0) npicked = 0;
+  if (tid == 0) npicked = nmatch = 0;
   if constexpr (FUSE) {
+    // the host fuses pooled sequences of at most 2 kDecTopnThreads tokens: two
+    // a thread, their first 16 heads' scores requested before the length and
+    // the heads' sums are known, so that one latency covers all three
     float* lse2 = tk + g.NcapP;
+    const int i2 = 2 * tid;
+    DecScores<2> x;
+    if (i2 < g.NcapP) x.load(g, s_cmp, bh, 0, i2);
     if (L.nvis > 0) {   // uniform
       if (tid < 256) dec_head_lse2(g, p1_ml, bh, dec_cmp_splits(L, g), lse2, tid);
       __syncthreads();
-      for (int i4 = 4 * tid; i4 < L.nvis; i4 += 4 * kDecTopnThreads) {
-        float v[4];
-        dec_token_sums4(g, s_cmp, bh, i4, lse2, sl2, v);
-        *reinterpret_cast<f32x4*>(tk + i4) = (f32x4){v[0], v[1], v[2], v[3]};   // inside the row pitch
+      if (i2 < L.nvis) {
+        float v[2] = {0.0f, 0.0f};
+        x.add(g, 0, lse2, sl2, v);
+        for (int c0 = 16; c0 < g.G; c0 += 16) {
+          x.load(g, s_cmp, bh, c0, i2);
+          x.add(g, c0, lse2, sl2, v);
+        }
+        *reinterpret_cast<float2*>(tk + i2) = make_float2(v[0], v[1]);   // inside the row pitch
       }
     }
   } else {
@@ -508,8 +538,8 @@ __global__ __launch_bounds__(kDecTopnThreads) void k_dec_topn(const int32_t* __r
   const int S = L.S;
   if (S > 0) {   // uniform: every thread of the workgroup sees the same L
     uint64_t prefix = 0, mask = 0;
-    int need = S;
-    for (int p = 0; p < 8; ++p) {
+    int need = S, left = L.ncand;   // picks among the keys that match the prefix, and how many those are
+    for (int p = 0; p < 8 && need < left && left > kWave; ++p) {
       const int shift = 56 - 8 * p;
       uint32_t* h = hist[p & 1];
       if (tid < 256) hist[(p + 1) & 1][tid] = 0;   // the other buffer: last read before the previous barrier
@@ -534,8 +564,8 @@ __global__ __launch_bounds__(kDecTopnThreads) void k_dec_topn(const int32_t* __r
         for (int i = 0; i < 4; ++i) {
           if (run < (uint32_t)need && run + c[i] >= (uint32_t)need) {
             ctl_prefix = prefix | ((uint64_t)(255 - 4 * lane - i) << shift);
-            // the whole bucket is picked: the remaining digits can stay 0
-            ctl_need = run + c[i] == (uint32_t)need ? 0 : need - (int)run;
+            ctl_need = need - (int)run;
+            ctl_left = (int)c[i];
           }
           run += c[i];
         }
@@ -543,27 +573,42 @@ __global__ __launch_bounds__(kDecTopnThreads) void k_dec_topn(const int32_t* __r
       __syncthreads();
       prefix = ctl_prefix;
       need = ctl_need;
+      left = ctl_left;
       mask |= (uint64_t)255 << shift;
-      if (need == 0) break;
     }
-    // exactly S keys are >= prefix (the S-th highest key, or the lowest
-    // possible key of a bucket that is picked whole)
+    // The picks are the S - need keys above the matching ones and the highest
+    // `need` of those: all of them, or the first of at most 64 (a key is
+    // unique, so a bucket cannot stay larger to the last digit), which one
+    // wave ranks by counting the keys above each.
 #pragma unroll
-    for (int k = 0; k < kDecKeysPerThread; ++k)
-      if (key[k] != 0 && key[k] >= prefix) picked[atomicAdd(&npicked, 1)] = key[k];
+    for (int k = 0; k < kDecKeysPerThread; ++k) {
+      if (key[k] == 0) continue;
+      const uint64_t m = key[k] & mask;
+      if (m > prefix || (m == prefix && need == left))
+        picked[atomicAdd(&npicked, 1)] = key[k];
+      else if (m == prefix)
+        match[atomicAdd(&nmatch, 1)] = key[k];
+    }
     __syncthreads();
     if (w == 0) {
-      uint64_t x = lane < S ? picked[lane] : 0;
-      // bitonic sort, descending across the 64 lanes
-      for (int k = 2; k <= kWave; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-          const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)x, j, kWave);
-          const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(x >> 32), j, kWave);
-          const uint64_t y = ((uint64_t)hi << 32) | lo;
-          const bool desc = (lane & k) == 0, low = (lane & j) == 0;
-          x = (low == desc) ? (y > x ? y : x) : (y < x ? y : x);
+      auto above = [&](uint64_t x, int n) {   // how many of lanes 0 .. n - 1 hold a higher key
+        int r = 0;
+        for (int i = 0; i < n; ++i) {
+          const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, i);
+          const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), i);
+          r += (((uint64_t)hi << 32) | lo) > x;
         }
-      if (lane < S) orow[lane] = (int32_t)(0xFFFFFFFFu - (uint32_t)x);
+        return r;
+      };
+      if (need < left) {
+        const uint64_t x = lane < left ? match[lane] : 0;
+        const int r = above(x, left);
+        if (lane < left && r < need) picked[S - need + r] = x;
+        wave_fence();
+      }
+      const uint64_t x = lane < S ? picked[lane] : 0;
+      const int r = above(x, S);
+      if (lane < S) orow[r] = (int32_t)(0xFFFFFFFFu - (uint32_t)x);
     }
   }
   for (int s = S + tid; s < g.n_sel; s += kDecTopnThreads) orow[s] = -1;
