@@ -20,6 +20,7 @@
 // line up with the next contraction's operand slots (nsa_tile32.h).
 #include "nsa_items.h"
 #include "nsa_launch.h"
+#include "nsa_slots.h"
 #include "nsa_tile32.h"
 
 namespace nsa {
@@ -215,7 +216,7 @@ __device__ __forceinline__ void finish_rows(const FwdExtras<T, TO>& f, const f32
   __syncthreads();
   constexpr int CPR = D / 8, RPI = 64 / CPR;   // 8-element chunks per row, rows per pass
   const int c8 = lane % CPR, rsub = lane / CPR;
-  const int nsub = sel_passes(f.sel_L), NS = f.S * nsub, n_csr = sel_csr_blocks(T_, f.sel_L);
+  const int nsub = sel_passes(f.sel_L), n_csr = sel_csr_blocks(T_, f.sel_L);
   const int G = mp.G;
   const int64_t bh = (int64_t)mp.b * Hkv + mp.hkv;
   for (int r0 = 0; r0 < 32; r0 += RPI) {
@@ -239,47 +240,9 @@ __device__ __forceinline__ void finish_rows(const FwdExtras<T, TO>& f, const f32
       for (int i = 0; i < 4; ++i) ow[i] = a[i], ow[4 + i] = b2[i];
       store_branch8<TO, CPR, kWholeLines<D>>(o + orow * D + 8 * c8, ow, f.o_scale + orow, c8 == 0);
     }
-    // selection: merge the slot partials (running maximum over batches of 16)
-    const int64_t qs = bh * T_ + t;
-    const int32_t* irow = f.idx + qs * f.S;
-    float acc_s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float M = -__builtin_inff(), Ls = 0.0f;
-    for (int s0 = 0; s0 < NS; s0 += 16) {
-      Raw8<PartT<T>> x[16];
-      float2 ml[16];
-      int jv[16];
-#pragma unroll
-      for (int k2 = 0; k2 < 16; ++k2) {
-        const int sl = s0 + k2 < NS ? s0 + k2 : NS - 1;
-        const int64_t pr = (qs * NS + sl) * G + gl;
-        jv[k2] = irow[sl / nsub];
-        ml[k2] = f.ml[pr];
-        x[k2].load_nt(f.opart + pr * D + 8 * c8);
-      }
-      bool ok[16];
-      float bm = M;
-#pragma unroll
-      for (int k2 = 0; k2 < 16; ++k2) {
-        ok[k2] = s0 + k2 < NS && sel_slot_valid(jv[k2], n_csr, f.sel_L, t) && ml[k2].y > 0.0f;
-        bm = ok[k2] ? fmaxf(bm, ml[k2].x) : bm;
-      }
-      if (bm == -__builtin_inff()) continue;   // nothing valid yet
-      const float rs = M == -__builtin_inff() ? 0.0f : fast_exp2(M - bm);
-      Ls *= rs;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc_s[i] *= rs;
-#pragma unroll
-      for (int k2 = 0; k2 < 16; ++k2) {
-        // the partial is unnormalised; a slot that does not count was maybe
-        // never written, so nothing of it (not even 0 x its l) is used
-        const float wk = ok[k2] ? fast_exp2(ml[k2].x - bm) : 0.0f;
-        x[k2].keep_if(ok[k2]);
-        Ls += ok[k2] ? wk * ml[k2].y : 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc_s[i] += wk * x[k2].get(i);
-      }
-      M = bm;
-    }
+    // selection: merge the slot partials
+    float acc_s[8], M, Ls;
+    merge_slots<PartT<T>, D>(f.opart, f.ml, f.idx, bh * T_ + t, t, gl, G, f.S, nsub, n_csr, f.sel_L, c8, acc_s, M, Ls);
     const float inv_s = Ls > 0.0f ? 1.0f / Ls : 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc_s[i] *= inv_s;
@@ -743,7 +706,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __syncthreads();
     constexpr int CPR = D / 8, RPI = 64 / CPR;   // 8-element chunks per row, rows per pass
     const int c8 = lane % CPR, rsub = lane / CPR;
-    const int nsub = sel_passes(sel_L), NS = S * nsub, n_csr = sel_csr_blocks(T_, sel_L);
+    const int nsub = sel_passes(sel_L), n_csr = sel_csr_blocks(T_, sel_L);
     const int G = mp.G;
     for (int r0 = 0; r0 < 32; r0 += RPI) {
       const int r = r0 + rsub;
@@ -764,24 +727,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] += u[i];
       }
-      const int64_t qrow_sel = (int64_t)bh * T_ + t;
-      const int32_t* irow = sel_idx + qrow_sel * S;
-      for (int s0 = 0; s0 < NS; s0 += 16) {
-        Raw8<T> x[16];
-        int jv[16];
-#pragma unroll
-        for (int k2 = 0; k2 < 16; ++k2) {
-          const int sl = s0 + k2 < NS ? s0 + k2 : NS - 1;
-          jv[k2] = irow[sl / nsub];
-          x[k2].load_nt(sel_part + ((qrow_sel * NS + sl) * G + gl) * D + 8 * c8);
-        }
-#pragma unroll
-        for (int k2 = 0; k2 < 16; ++k2) {
-          x[k2].keep_if(s0 + k2 < NS && sel_slot_valid(jv[k2], n_csr, sel_L, t));
-#pragma unroll
-          for (int i = 0; i < 8; ++i) v[i] += x[k2].get(i);
-        }
-      }
+      add_slots<T, D>(sel_part, sel_idx, (int64_t)bh * T_ + t, t, gl, G, S, nsub, n_csr, sel_L, c8, lane, v);
       if (dq_out32 != nullptr)
         store8(dq_out32 + orow * D + 8 * c8, v);
       else

@@ -14,6 +14,7 @@
 // k_sel_dq_reduce sums the dQ partials written by the dK/dV kernel.
 #include "nsa_items.h"
 #include "nsa_launch.h"
+#include "nsa_slots.h"
 #include "nsa_tile32.h"
 
 namespace nsa {
@@ -462,23 +463,21 @@ static inline int grid_for(int64_t n) {
 }
 
 // Both reductions below take one thread per 8 elements of a row, rows ordered
-// (b, hkv, t, g) so that a wave reads contiguous partial rows.  Every slot's
-// partial is loaded -- the buffers hold all NS slots of a row, and a slot
-// without a pair was never written -- kSlotBatch at a time, with all loads of
-// a batch issued together and none of their addresses depending on the block
-// indices; a slot that does not count is then replaced by zeros (bit for bit)
-// and weight 0, so whatever an unwritten slot holds never reaches a result.
-constexpr int kSlotBatch = 16;
+// (b, hkv, t, g) so that a wave reads contiguous partial rows (nsa_slots.h).
+// Every slot's partial is loaded -- the buffers hold all NS slots of a row,
+// and a slot without a pair was never written -- 16 at a time, with all loads
+// of a batch issued together and none of their addresses depending on the
+// block indices.
 
 // o[row] = sum_slots exp2(m - M) O_slot / sum exp2(m - M) l over the valid
 // slots, lse = (M + log2 L) ln 2, with a running maximum M across batches.
 template <typename T, int D>
-__global__ __launch_bounds__(256) void k_sel_merge(const int32_t* __restrict__ idx, const PartT<T>* __restrict__ opart,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 ? 3 : 2))) void k_sel_merge(const int32_t* __restrict__ idx, const PartT<T>* __restrict__ opart,
                                                    const float2* __restrict__ mlpart, T* __restrict__ o,
                                                    float* __restrict__ lse, int Hq, int Hkv, int T_, int S, int n_csr,
                                                    int L, int nsub, int64_t total, float* __restrict__ o32) {
   constexpr int NC = D / 8;
-  const int G = Hq / Hkv, NS = S * nsub;
+  const int G = Hq / Hkv;
   for (int64_t e = blockIdx.x * 256ll + threadIdx.x; e < total; e += (int64_t)gridDim.x * 256) {
     const int c = (int)(e % NC);
     int64_t r = e / NC;
@@ -486,46 +485,8 @@ __global__ __launch_bounds__(256) void k_sel_merge(const int32_t* __restrict__ i
     r /= G;
     const int t = (int)(r % T_);
     const int64_t bh = r / T_;
-    const int32_t* irow = idx + (bh * T_ + t) * S;
-    const int64_t pbase = (bh * T_ + t) * NS;
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float M = kNegInfS, Ls = 0.0f;
-    for (int s0 = 0; s0 < NS; s0 += kSlotBatch) {
-      float2 ml[kSlotBatch];
-      Raw8<PartT<T>> x[kSlotBatch];
-      bool ok[kSlotBatch];
-      int jv[kSlotBatch];
-#pragma unroll
-      for (int k = 0; k < kSlotBatch; ++k) {
-        const int sl = s0 + k < NS ? s0 + k : NS - 1;
-        const int64_t pr = (pbase + sl) * G + g;
-        jv[k] = irow[sl / nsub];
-        ml[k] = mlpart[pr];
-        x[k].load(opart + pr * D + 8 * c);
-      }
-      float bm = M;
-#pragma unroll
-      for (int k = 0; k < kSlotBatch; ++k) {
-        ok[k] = (s0 + k < NS) && sel_slot_valid(jv[k], n_csr, L, t) && ml[k].y > 0.0f;
-        bm = ok[k] ? fmaxf(bm, ml[k].x) : bm;
-      }
-      if (bm == kNegInfS) continue;   // nothing valid yet
-      const float rs = M == kNegInfS ? 0.0f : fast_exp2(M - bm);
-      Ls *= rs;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc[i] *= rs;
-#pragma unroll
-      for (int k = 0; k < kSlotBatch; ++k) {
-        // the partial is unnormalised; a slot that does not count was maybe
-        // never written, so nothing of it (not even 0 x its l) is used
-        const float wk = ok[k] ? fast_exp2(ml[k].x - bm) : 0.0f;
-        x[k].keep_if(ok[k]);
-        Ls += ok[k] ? wk * ml[k].y : 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] += wk * x[k].get(i);
-      }
-      M = bm;
-    }
+    float acc[8], M, Ls;
+    merge_slots<PartT<T>, D>(opart, mlpart, idx, bh * T_ + t, t, g, G, S, nsub, n_csr, L, c, acc, M, Ls);
     const int64_t orow = (((bh / Hkv) * Hq + (bh % Hkv) * G + g) * T_ + t);
     const float inv = Ls > 0.0f ? 1.0f / Ls : 0.0f;
 #pragma unroll
@@ -544,7 +505,7 @@ __global__ __launch_bounds__(256) void k_sel_dq_reduce(const int32_t* __restrict
                                                        int Hq, int Hkv, int T_, int S, int n_csr, int L, int nsub,
                                                        int64_t total) {
   constexpr int NC = D / 8;
-  const int G = Hq / Hkv, NS = S * nsub;
+  const int G = Hq / Hkv;
   for (int64_t e = blockIdx.x * 256ll + threadIdx.x; e < total; e += (int64_t)gridDim.x * 256) {
     const int c = (int)(e % NC);
     int64_t r = e / NC;
@@ -552,8 +513,6 @@ __global__ __launch_bounds__(256) void k_sel_dq_reduce(const int32_t* __restrict
     r /= G;
     const int t = (int)(r % T_);
     const int64_t bh = r / T_;
-    const int32_t* irow = idx + (bh * T_ + t) * S;
-    const int64_t pbase = (bh * T_ + t) * NS;
     const int64_t orow = (((bh / Hkv) * Hq + (bh % Hkv) * G + g) * T_ + t);
     float acc[8];
     if (dq_acc != nullptr) {
@@ -562,22 +521,7 @@ __global__ __launch_bounds__(256) void k_sel_dq_reduce(const int32_t* __restrict
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
     }
-    for (int s0 = 0; s0 < NS; s0 += kSlotBatch) {
-      Raw8<T> x[kSlotBatch];
-      int jv[kSlotBatch];
-#pragma unroll
-      for (int k = 0; k < kSlotBatch; ++k) {
-        const int sl = s0 + k < NS ? s0 + k : NS - 1;
-        jv[k] = irow[sl / nsub];
-        x[k].load(dqpart + ((pbase + sl) * G + g) * D + 8 * c);
-      }
-#pragma unroll
-      for (int k = 0; k < kSlotBatch; ++k) {
-        x[k].keep_if((s0 + k < NS) && sel_slot_valid(jv[k], n_csr, L, t));
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] += x[k].get(i);
-      }
-    }
+    add_slots<T, D>(dqpart, idx, bh * T_ + t, t, g, G, S, nsub, n_csr, L, c, threadIdx.x & 63, acc);
     store8(dq_out + orow * D + 8 * c, acc);
   }
 }
