@@ -1,9 +1,10 @@
 // The gated three-branch layer behind two C entry points (nsa_fused_fwd /
 // nsa_fused_bwd): the launch sequence of the Python autograd boundary
 // (nsa_hip_ops.fused_forward / fused_backward) for callers without Python.
-// Host code only: every launch goes through the library's own entry points,
-// in the same order and with the same arguments, so the results are the
-// Python path's bit for bit.
+// Host code only: every launch is one of the library's own entry points', with
+// the same arguments (the transposed copies, and the two poolings, of a
+// direction in one launch each), so the results are the Python path's bit for
+// bit.
 //
 // Two caller buffers, carved by the same plan on both calls:
 //   ctx     -- written by the forward, read by the backward (what autograd
@@ -212,11 +213,17 @@ int nsa_fused_fwd(const void* q, const void* kc, const void* vc, const void* ks,
   const void* k_cmp = pooled ? kc : x.k_cmp;
   const void* v_cmp = pooled ? vc : x.v_cmp;
   if (!pooled) {
-    NSA_TRY(nsa_pool_fwd(kc, x.k_cmp, B, Hkv, T, D, cmp_block, cmp_stride, dtype, stream));
-    NSA_TRY(nsa_pool_fwd(vc, x.v_cmp, B, Hkv, T, D, cmp_block, cmp_stride, dtype, stream));
+    const void* src[2] = {kc, vc};
+    void* dst[2] = {x.k_cmp, x.v_cmp};
+    NSA_TRY(nsa_pool_fwd_set(src, dst, 2, B, Hkv, T, D, cmp_block, cmp_stride, dtype, stream));
+  }
+  {
+    const void* src[3] = {v_cmp, vs, vw};
+    void* dst[3] = {w.vt_c, w.vt_s, w.vt_w};
+    const int len[3] = {n, T, T}, pad[3] = {Lpn, Lpt, Lpt};
+    NSA_TRY(nsa_transpose_kv_set(src, dst, len, pad, 3, B * Hkv, D, dtype, stream));
   }
   // compression (its forward also writes the packed q of the selection kernels)
-  NSA_TRY(nsa_transpose_kv(v_cmp, w.vt_c, B * Hkv, n, D, Lpn, dtype, stream));
   NSA_TRY(nsa_range_fwd(NSA_MODE_COMPRESS, q, k_cmp, w.vt_c, x.o_c, x.lse_c, B, Hq, Hkv, T, n, D, 0, cmp_block,
                         cmp_stride, x.qp, dtype, m.o_dtype(), stream));
   if (!idx_given)
@@ -225,11 +232,9 @@ int nsa_fused_fwd(const void* q, const void* kc, const void* vc, const void* ks,
   // selection partials over the block -> query CSR
   NSA_TRY(nsa_csr_build(block_idx, x.q_of_block, x.offsets, x.pair_bh, x.count, w.csr_ws, w.csr_bytes, B, Hkv, T,
                         S, sel_block, m.nblk(), 1, stream));
-  NSA_TRY(nsa_transpose_kv(vs, w.vt_s, B * Hkv, T, D, Lpt, dtype, stream));
   NSA_TRY(nsa_sel_fwd_bo(x.qp, ks, w.vt_s, x.q_of_block, x.offsets, w.o_part, w.ml_part, w.sel_ws, w.sel_bytes, B, Hq,
                          Hkv, T, D, S, sel_block, m.fwd_chunk(), dtype, stream));
   // window, finishing the rows: selection merge and gate
-  NSA_TRY(nsa_transpose_kv(vw, w.vt_w, B * Hkv, T, D, Lpt, dtype, stream));
   return nsa_range_fwd_finish(NSA_MODE_WINDOW, q, kw, w.vt_w, x.o_w, x.lse_w, B, Hq, Hkv, T, T, D, window, 1, 1,
                               w.o_part, w.ml_part, block_idx, S, sel_block, x.o_s, x.lse_s, x.o_c, gate, out, dtype,
                               m.o_dtype(), dtype, stream);
@@ -260,26 +265,30 @@ int nsa_fused_bwd(const void* dout, const void* q, const void* kc, const void* v
   // gate backward, row dots of the three branches, dO packed for the selection
   NSA_TRY(nsa_bwd_prep(dout, x.o_c, x.o_s, x.o_w, gate, dgate, x.lse_c, x.lse_s, x.lse_w, w.dot, w.rs, w.coff,
                        w.dop, G, T, R, D, 3, dtype, m.o_dtype(), dtype, stream));
+  {
+    const void* src[3] = {ks, kw, k_cmp};
+    void* dst[3] = {w.kt_s, w.kt_w, w.kt_c};
+    const int len[3] = {T, T, n}, pad[3] = {Lpt, Lpt, Lpn};
+    NSA_TRY(nsa_transpose_kv_set(src, dst, len, pad, 3, B * Hkv, D, dtype, stream));
+  }
   // selection dK/dV and dQ partials (block-outer, deterministic merge)
-  NSA_TRY(nsa_transpose_kv(ks, w.kt_s, B * Hkv, T, D, Lpt, dtype, stream));
   NSA_TRY(nsa_sel_dkdv_as(x.qp, ks, vs, w.kt_s, w.dop, w.coff + R, w.dot + R, x.q_of_block, 1, x.offsets, x.count,
                           dks, dvs, w.sel_part, w.sel_part_bytes, w.dq_part, w.sel_ws, w.sel_bytes, B, Hq, Hkv, T, D,
                           S, sel_block, m.dkdv_chunk(), dtype, dtype, stream));
   // window and compression dK/dV
-  NSA_TRY(nsa_transpose_kv(kw, w.kt_w, B * Hkv, T, D, Lpt, dtype, stream));
   NSA_TRY(nsa_range_dkdv_as(NSA_MODE_WINDOW, q, kw, vw, dout, w.coff + 2 * R, w.dot + 2 * R, dkw, dvw, w.win_part,
                             w.win_part_bytes, B, Hq, Hkv, T, T, D, window, 1, 1, dtype, dtype, stream));
   NSA_TRY(nsa_range_dkdv_as(NSA_MODE_COMPRESS, q, k_cmp, v_cmp, dout, w.coff, w.dot, dkp, dvp, w.cmp_part,
                             w.cmp_part_bytes, B, Hq, Hkv, T, n, D, 0, cmp_block, cmp_stride, dtype,
                             pooled ? dtype : NSA_F32, stream));
   // compression + window dQ in one launch, rows finished with the selection partials
-  NSA_TRY(nsa_transpose_kv(k_cmp, w.kt_c, B * Hkv, n, D, Lpn, dtype, stream));
   NSA_TRY(nsa_range_dq_cw(q, dout, k_cmp, v_cmp, w.kt_c, x.lse_c, w.dot, w.rs, n, cmp_block, cmp_stride, kw, vw,
                           w.kt_w, x.lse_w, w.dot + 2 * R, w.rs + 2 * R, window, B, Hq, Hkv, T, D, w.dq_part, block_idx,
                           S, sel_block, dq, dtype, dtype, stream));
   if (!pooled) {
-    NSA_TRY(nsa_pool_bwd(dkp, NSA_F32, dkc, B, Hkv, T, D, cmp_block, cmp_stride, dtype, stream));
-    NSA_TRY(nsa_pool_bwd(dvp, NSA_F32, dvc, B, Hkv, T, D, cmp_block, cmp_stride, dtype, stream));
+    const void* src[2] = {dkp, dvp};
+    void* dst[2] = {dkc, dvc};
+    NSA_TRY(nsa_pool_bwd_set(src, NSA_F32, dst, 2, B, Hkv, T, D, cmp_block, cmp_stride, dtype, stream));
   }
   return NSA_OK;
 }

@@ -16,3 +16,13 @@ static inline int nsa_launch_status() {
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? NSA_OK : NSA_ERR_LAUNCH;
 }
+
+// Several tensors in one launch (nsa_prep.hip; the C entry points nsa_transpose_kv,
+// nsa_pool_fwd and nsa_pool_bwd are their sets of one): up to three transposed
+// copies [BH][L][D] -> [BH][D][Lp], up to two poolings of one shape.
+int nsa_transpose_kv_set(const void* const* x, void* const* xt, const int* L, const int* Lp, int n, int BH, int D,
+                         int dtype, void* stream);
+int nsa_pool_fwd_set(const void* const* x, void* const* out, int m, int B, int H, int T, int D, int l, int d,
+                     int dtype, void* stream);
+int nsa_pool_bwd_set(const void* const* dpool, int dpool_dtype, void* const* dx, int m, int B, int H, int T, int D,
+                     int l, int d, int dtype, void* stream);

@@ -40,19 +40,29 @@ __global__ __launch_bounds__(256) void k_transpose_kv(const T* __restrict__ x, T
   }
 }
 
+// Up to three copies of one launch (blockIdx.z: BH slices of each).  One copy
+// of a short sequence is a launch of 4 us, whatever it moves: the layer's
+// three per direction go out together.
+template <typename T> struct TransposeSet {
+  const T* x[3];
+  T* xt[3];
+  int L[3], Lp[3];
+};
 // D % 8 == 0, Lp % 8 == 0, 16-byte aligned rows: 8-element global accesses.
 // A lane moves 8 consecutive d of one key in, 8 consecutive keys of one d out
 // (8 lanes cover a 64-element row piece).  The LDS row pitch (66 bf16 /
 // 65 float) puts the 8 keys x 8 d read by a wave's lanes on distinct banks.
 template <typename T>
-__global__ __launch_bounds__(256) void k_transpose_kv8(const T* __restrict__ x, T* __restrict__ xt,
-                                                       int L, int D, int Lp) {
+__global__ __launch_bounds__(256) void k_transpose_kv8(const TransposeSet<T> ts, int BH, int D) {
   constexpr int P = sizeof(T) == 2 ? 66 : 65;
   __shared__ T tile[64 * P];
-  const int bh = blockIdx.z;
+  const int which = blockIdx.z / BH, bh = blockIdx.z % BH;
+  const int L = which == 0 ? ts.L[0] : which == 1 ? ts.L[1] : ts.L[2];
+  const int Lp = which == 0 ? ts.Lp[0] : which == 1 ? ts.Lp[1] : ts.Lp[2];
   const int l0 = blockIdx.x * 64, d0 = blockIdx.y * 64;
-  const T* xb = x + (int64_t)bh * L * D;
-  T* yb = xt + (int64_t)bh * D * Lp;
+  if (l0 >= Lp) return;   // uniform: the grid covers the longest
+  const T* xb = (which == 0 ? ts.x[0] : which == 1 ? ts.x[1] : ts.x[2]) + (int64_t)bh * L * D;
+  T* yb = (which == 0 ? ts.xt[0] : which == 1 ? ts.xt[1] : ts.xt[2]) + (int64_t)bh * D * Lp;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int c = threadIdx.x + 256 * i, r = c >> 3, cc = (c & 7) * 8;   // r: key, cc: first d
@@ -102,10 +112,15 @@ __global__ __launch_bounds__(256) void k_pool_fwd(const T* __restrict__ x, T* __
 }
 
 // D % 8 == 0, 16-byte aligned rows: a lane sums 8 consecutive d (same order of
-// additions as k_pool_fwd)
+// additions as k_pool_fwd).  Few lanes sum a short sequence: the rows' latency
+// is what it waits for, so 16 are in flight.  blockIdx.y = 1: a second tensor
+// of the same shape (keys and values in one launch).
 template <typename T>
-__global__ __launch_bounds__(256) void k_pool_fwd8(const T* __restrict__ x, T* __restrict__ out,
-                                                   int BH, int L, int D, int n, int pl, int pd) {
+__global__ __launch_bounds__(256) void k_pool_fwd8(const T* __restrict__ x0, T* __restrict__ out0,
+                                                   const T* __restrict__ x1, T* __restrict__ out1, int BH, int L,
+                                                   int D, int n, int pl, int pd) {
+  const T* x = blockIdx.y == 0 ? x0 : x1;
+  T* out = blockIdx.y == 0 ? out0 : out1;
   const int dc = D / 8;
   const int64_t total = (int64_t)BH * n * dc;
   const float inv = 1.0f / (float)pl;
@@ -118,12 +133,16 @@ __global__ __launch_bounds__(256) void k_pool_fwd8(const T* __restrict__ x, T* _
     float s[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) s[j] = 0.0f;
-#pragma unroll 8
-    for (int k = 0; k < pl; ++k) {
-      Frag<T> f;
-      f.load(src + (int64_t)k * D);
+    for (int k0 = 0; k0 < pl; k0 += 16) {
+      Frag<T> f[16];   // (left to itself the compiler waits for each row)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s[j] += to_f32(f.elem(j));
+      for (int u = 0; u < 16; ++u) f[u].load(src + (int64_t)(k0 + u < pl ? k0 + u : pl - 1) * D);
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        if (k0 + u < pl) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) s[j] += to_f32(f[u].elem(j));
+        }
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) s[j] *= inv;
@@ -154,10 +173,13 @@ __global__ __launch_bounds__(256) void k_pool_bwd(const TI* __restrict__ dp, TO*
 }
 
 // D % 8 == 0, 16-byte aligned rows: a lane writes 8 consecutive d (same order
-// of additions as k_pool_bwd)
+// of additions as k_pool_bwd).  blockIdx.y = 1: a second tensor.
 template <typename TI, typename TO>
-__global__ __launch_bounds__(256) void k_pool_bwd8(const TI* __restrict__ dp, TO* __restrict__ dx,
-                                                   int BH, int L, int D, int n, int pl, int pd) {
+__global__ __launch_bounds__(256) void k_pool_bwd8(const TI* __restrict__ dp0, TO* __restrict__ dx0,
+                                                   const TI* __restrict__ dp1, TO* __restrict__ dx1, int BH, int L,
+                                                   int D, int n, int pl, int pd) {
+  const TI* dp = blockIdx.y == 0 ? dp0 : dp1;
+  TO* dx = blockIdx.y == 0 ? dx0 : dx1;
   const int dc = D / 8;
   const int64_t total = (int64_t)BH * L * dc;
   const float inv = 1.0f / (float)pl;
@@ -210,13 +232,17 @@ __global__ __launch_bounds__(256) void k_wpool_fwd8(const T* __restrict__ x, con
     float s[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) s[j] = 0.0f;
-#pragma unroll 8
-    for (int k = 0; k < pl; ++k) {
-      Frag<T> f;
-      f.load(src + (int64_t)k * D);
-      const float wk = w[k];
+    for (int k0 = 0; k0 < pl; k0 += 16) {
+      Frag<T> f[16];   // 16 rows in flight, as k_pool_fwd8
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s[j] += wk * to_f32(f.elem(j));
+      for (int u = 0; u < 16; ++u) f[u].load(src + (int64_t)(k0 + u < pl ? k0 + u : pl - 1) * D);
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        if (k0 + u < pl) {
+          const float wk = w[k0 + u];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) s[j] += wk * to_f32(f[u].elem(j));
+        }
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) s[j] += cv[8 * c + j];
@@ -743,89 +769,127 @@ static int head_segs(HeadSegs& sg, void* const* bufs, const float* const* biases
 
 using namespace nsa;
 
-extern "C" {
-
-int nsa_transpose_kv(const void* x, void* xt, int BH, int L, int D, int Lp, int dtype, void* stream) {
-  NSA_CHECK(BH > 0 && L >= 0 && D > 0 && Lp >= L, NSA_ERR_SHAPE);
+int nsa_transpose_kv_set(const void* const* x, void* const* xt, const int* L, const int* Lp, int n, int BH, int D,
+                         int dtype, void* stream) {
+  NSA_CHECK(n >= 1 && n <= 3 && BH > 0 && D > 0, NSA_ERR_SHAPE);
   NSA_CHECK(dtype == NSA_F32 || dtype == NSA_BF16, NSA_ERR_DTYPE);
-  if (L == 0 && Lp == 0) return NSA_OK;
-  dim3 grid((Lp + 63) / 64, (D + 63) / 64, BH);
-  hipStream_t s = (hipStream_t)stream;
-  const bool vec = D % 8 == 0 && Lp % 8 == 0 && aligned16(x) && aligned16(xt);
-  if (dtype == NSA_BF16) {
-    if (vec)
-      k_transpose_kv8<bf16><<<grid, 256, 0, s>>>((const bf16*)x, (bf16*)xt, L, D, Lp);
-    else
-      k_transpose_kv<bf16><<<grid, 256, 0, s>>>((const bf16*)x, (bf16*)xt, L, D, Lp);
-  } else {
-    if (vec)
-      k_transpose_kv8<float><<<grid, 256, 0, s>>>((const float*)x, (float*)xt, L, D, Lp);
-    else
-      k_transpose_kv<float><<<grid, 256, 0, s>>>((const float*)x, (float*)xt, L, D, Lp);
+  if (n > 1 && (int64_t)n * BH > 65535) {   // grid z
+    for (int i = 0; i < n; ++i) {
+      const int rc = nsa_transpose_kv_set(x + i, xt + i, L + i, Lp + i, 1, BH, D, dtype, stream);
+      if (rc != NSA_OK) return rc;
+    }
+    return NSA_OK;
   }
+  hipStream_t s = (hipStream_t)stream;
+  bool vec = D % 8 == 0;
+  int longest = 0;
+  for (int i = 0; i < n; ++i) {
+    NSA_CHECK(L[i] >= 0 && Lp[i] >= L[i], NSA_ERR_SHAPE);
+    vec = vec && Lp[i] % 8 == 0 && aligned16(x[i]) && aligned16(xt[i]);
+    longest = Lp[i] > longest ? Lp[i] : longest;
+  }
+  if (longest == 0) return NSA_OK;
+  auto go = [&](auto tag) {
+    using T = decltype(tag);
+    if (vec) {
+      TransposeSet<T> ts;
+      for (int i = 0; i < 3; ++i) {
+        const int k = i < n ? i : 0;
+        ts.x[i] = (const T*)x[k], ts.xt[i] = (T*)xt[k], ts.L[i] = L[k], ts.Lp[i] = Lp[k];
+      }
+      k_transpose_kv8<T><<<dim3((longest + 63) / 64, (D + 63) / 64, n * BH), 256, 0, s>>>(ts, BH, D);
+      return;
+    }
+    for (int i = 0; i < n; ++i)
+      if (Lp[i] > 0)
+        k_transpose_kv<T><<<dim3((Lp[i] + 63) / 64, (D + 63) / 64, BH), 256, 0, s>>>((const T*)x[i], (T*)xt[i], L[i],
+                                                                                     D, Lp[i]);
+  };
+  if (dtype == NSA_BF16)
+    go(bf16{});
+  else
+    go(float{});
   return nsa_launch_status();
 }
 
-int nsa_pool_fwd(const void* x, void* out, int B, int H, int T, int D, int l, int d, int dtype,
-                 void* stream) {
-  NSA_CHECK(B > 0 && H > 0 && T >= 0 && D > 0 && l > 0 && d > 0, NSA_ERR_SHAPE);
+int nsa_pool_fwd_set(const void* const* x, void* const* out, int m, int B, int H, int T, int D, int l, int d,
+                     int dtype, void* stream) {
+  NSA_CHECK(m >= 1 && m <= 2 && B > 0 && H > 0 && T >= 0 && D > 0 && l > 0 && d > 0, NSA_ERR_SHAPE);
   NSA_CHECK(dtype == NSA_F32 || dtype == NSA_BF16, NSA_ERR_DTYPE);
   const int n = T >= l ? (T - l) / d + 1 : 0;
   const int64_t total = (int64_t)B * H * n * D;
   if (total == 0) return NSA_OK;
   hipStream_t s = (hipStream_t)stream;
-  if (D % 8 == 0 && aligned16(x) && aligned16(out)) {
-    const int g = grid_for(total / 8);
-    if (dtype == NSA_BF16)
-      k_pool_fwd8<bf16><<<g, 256, 0, s>>>((const bf16*)x, (bf16*)out, B * H, T, D, n, l, d);
-    else
-      k_pool_fwd8<float><<<g, 256, 0, s>>>((const float*)x, (float*)out, B * H, T, D, n, l, d);
-  } else if (dtype == NSA_BF16) {
-    k_pool_fwd<bf16><<<grid_for(total), 256, 0, s>>>((const bf16*)x, (bf16*)out, B * H, T, D, n, l, d);
-  } else {
-    k_pool_fwd<float><<<grid_for(total), 256, 0, s>>>((const float*)x, (float*)out, B * H, T, D, n, l, d);
-  }
+  const bool vec = D % 8 == 0 && aligned16(x[0]) && aligned16(out[0]) && aligned16(x[m - 1]) && aligned16(out[m - 1]);
+  auto go = [&](auto tag) {
+    using E = decltype(tag);
+    if (vec) {
+      k_pool_fwd8<E><<<dim3(grid_for(total / 8), m), 256, 0, s>>>((const E*)x[0], (E*)out[0], (const E*)x[m - 1],
+                                                                  (E*)out[m - 1], B * H, T, D, n, l, d);
+      return;
+    }
+    for (int i = 0; i < m; ++i)
+      k_pool_fwd<E><<<grid_for(total), 256, 0, s>>>((const E*)x[i], (E*)out[i], B * H, T, D, n, l, d);
+  };
+  if (dtype == NSA_BF16)
+    go(bf16{});
+  else
+    go(float{});
   return nsa_launch_status();
 }
 
-// dpool_dtype: dtype of the pooled-gradient input (fp32 accumulators or the model dtype)
-int nsa_pool_bwd(const void* dpool, int dpool_dtype, void* dx, int B, int H, int T, int D, int l, int d,
-                 int dtype, void* stream) {
-  NSA_CHECK(B > 0 && H > 0 && T >= 0 && D > 0 && l > 0 && d > 0, NSA_ERR_SHAPE);
+int nsa_pool_bwd_set(const void* const* dpool, int dpool_dtype, void* const* dx, int m, int B, int H, int T, int D,
+                     int l, int d, int dtype, void* stream) {
+  NSA_CHECK(m >= 1 && m <= 2 && B > 0 && H > 0 && T >= 0 && D > 0 && l > 0 && d > 0, NSA_ERR_SHAPE);
   NSA_CHECK((dtype == NSA_F32 || dtype == NSA_BF16) && (dpool_dtype == NSA_F32 || dpool_dtype == NSA_BF16),
             NSA_ERR_DTYPE);
   const int n = T >= l ? (T - l) / d + 1 : 0;
   const int64_t total = (int64_t)B * H * T * D;
   if (total == 0) return NSA_OK;
   hipStream_t s = (hipStream_t)stream;
-  if (D % 8 == 0 && aligned16(dpool) && aligned16(dx)) {
-    const int g = grid_for(total / 8);
-    if (dpool_dtype == NSA_F32) {
-      if (dtype == NSA_BF16)
-        k_pool_bwd8<float, bf16><<<g, 256, 0, s>>>((const float*)dpool, (bf16*)dx, B * H, T, D, n, l, d);
-      else
-        k_pool_bwd8<float, float><<<g, 256, 0, s>>>((const float*)dpool, (float*)dx, B * H, T, D, n, l, d);
-    } else {
-      if (dtype == NSA_BF16)
-        k_pool_bwd8<bf16, bf16><<<g, 256, 0, s>>>((const bf16*)dpool, (bf16*)dx, B * H, T, D, n, l, d);
-      else
-        k_pool_bwd8<bf16, float><<<g, 256, 0, s>>>((const bf16*)dpool, (float*)dx, B * H, T, D, n, l, d);
+  const bool vec =
+      D % 8 == 0 && aligned16(dpool[0]) && aligned16(dx[0]) && aligned16(dpool[m - 1]) && aligned16(dx[m - 1]);
+  auto go = [&](auto in, auto outt) {
+    using TI = decltype(in);
+    using TO = decltype(outt);
+    if (vec) {
+      k_pool_bwd8<TI, TO><<<dim3(grid_for(total / 8), m), 256, 0, s>>>((const TI*)dpool[0], (TO*)dx[0],
+                                                                       (const TI*)dpool[m - 1], (TO*)dx[m - 1], B * H,
+                                                                       T, D, n, l, d);
+      return;
     }
-    return nsa_launch_status();
-  }
-  const int grid = grid_for(total);
+    for (int i = 0; i < m; ++i)
+      k_pool_bwd<TI, TO><<<grid_for(total), 256, 0, s>>>((const TI*)dpool[i], (TO*)dx[i], B * H, T, D, n, l, d);
+  };
   if (dpool_dtype == NSA_F32) {
     if (dtype == NSA_BF16)
-      k_pool_bwd<float, bf16><<<grid, 256, 0, s>>>((const float*)dpool, (bf16*)dx, B * H, T, D, n, l, d);
+      go(float{}, bf16{});
     else
-      k_pool_bwd<float, float><<<grid, 256, 0, s>>>((const float*)dpool, (float*)dx, B * H, T, D, n, l, d);
+      go(float{}, float{});
   } else {
     if (dtype == NSA_BF16)
-      k_pool_bwd<bf16, bf16><<<grid, 256, 0, s>>>((const bf16*)dpool, (bf16*)dx, B * H, T, D, n, l, d);
+      go(bf16{}, bf16{});
     else
-      k_pool_bwd<bf16, float><<<grid, 256, 0, s>>>((const bf16*)dpool, (float*)dx, B * H, T, D, n, l, d);
+      go(bf16{}, float{});
   }
   return nsa_launch_status();
+}
+
+extern "C" {
+
+int nsa_transpose_kv(const void* x, void* xt, int BH, int L, int D, int Lp, int dtype, void* stream) {
+  return nsa_transpose_kv_set(&x, &xt, &L, &Lp, 1, BH, D, dtype, stream);
+}
+
+int nsa_pool_fwd(const void* x, void* out, int B, int H, int T, int D, int l, int d, int dtype,
+                 void* stream) {
+  return nsa_pool_fwd_set(&x, &out, 1, B, H, T, D, l, d, dtype, stream);
+}
+
+// dpool_dtype: dtype of the pooled-gradient input (fp32 accumulators or the model dtype)
+int nsa_pool_bwd(const void* dpool, int dpool_dtype, void* dx, int B, int H, int T, int D, int l, int d,
+                 int dtype, void* stream) {
+  return nsa_pool_bwd_set(&dpool, dpool_dtype, &dx, 1, B, H, T, D, l, d, dtype, stream);
 }
 
 int nsa_wpool_fwd(const void* x, const float* w, const float* cvec, float* out, int B, int H, int T, int D, int l,
