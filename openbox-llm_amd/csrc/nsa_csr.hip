@@ -6,17 +6,16 @@
 // reference's stable argsort.  Two builds give the same arrays:
 //
 //  * counting (LDS for 3 n_blk + 64 S ints): one wave per chunk of 64 queries of
-//    one (b, hkv) counts its pairs per block in LDS; an exclusive scan over the
-//    counts in (key, chunk) order gives every chunk's first slot in every
-//    list; the wave then places its pairs, a pair's rank in its list within
-//    the chunk being the number of earlier queries of the chunk on its block
-//    (a 64-bit query mask per block).  Deterministic, no atomics outside LDS,
-//    no memsets.
+//    one (b, hkv) counts its pairs per block in LDS; k_csr_scan turns the
+//    counts into every chunk's first slot within every list, and the lists'
+//    totals; the wave then adds the lists' starts (its own scan of the
+//    totals) and places its pairs, a pair's rank in its list within the chunk
+//    being the number of earlier queries of the chunk on its block (a 64-bit
+//    query mask per block).  Deterministic, no atomics outside LDS, no memsets.
 //  * sort (otherwise): a stable LSD radix sort of (key, value) with a
 //    sentinel key for the non-causal slots; offsets are lower bounds of the
 //    keys in the sorted keys.
 #include <rocprim/device/device_radix_sort.hpp>
-#include <rocprim/device/device_scan.hpp>
 
 #include "nsa_launch.h"
 #include "nsa_items.h"
@@ -108,29 +107,11 @@ __device__ __forceinline__ void csr_chunk_loads(const int32_t* __restrict__ idx,
   }
 }
 
-// LDS per-list counters of one chunk: 16 loads a lane in flight per batch
-__device__ __forceinline__ void csr_lds_rows(int* __restrict__ dst, const int32_t* __restrict__ src, int n_blk,
-                                             int nchunk, int lane) {
-  for (int b0 = 0; b0 < n_blk; b0 += 16 * 64) {
-    int v[16];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int j = b0 + k * 64 + lane;
-      v[k] = j < n_blk ? src[(int64_t)j * nchunk] : 0;
-    }
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int j = b0 + k * 64 + lane;
-      if (j < n_blk) dst[j] = v[k];
-    }
-  }
-}
-
 __device__ __forceinline__ bool csr_causal(int j, int t, int n_blk, int L) {
   return j >= 0 && j < n_blk && (int64_t)j * L <= t;
 }
 
-// counts[(bh n_blk + j) nchunk + c] = pairs of chunk c of bh on block j
+// counts[(bh nchunk + c) n_blk + j] = pairs of chunk c of bh on block j
 __global__ __launch_bounds__(64) void k_csr_count(const int32_t* __restrict__ idx, int32_t* __restrict__ counts,
                                                   int T, int S, int n_blk, int L, int nchunk) {
   extern __shared__ int cnt[];
@@ -144,8 +125,95 @@ __global__ __launch_bounds__(64) void k_csr_count(const int32_t* __restrict__ id
     if (csr_causal(j, t0 + i / S, n_blk, L)) atomicAdd(&cnt[j], 1);
   });
   __syncthreads();
-  int32_t* out = counts + (int64_t)bh * n_blk * nchunk + c;
-  for (int j = lane; j < n_blk; j += 64) out[(int64_t)j * nchunk] = cnt[j];
+  int32_t* out = counts + ((int64_t)bh * nchunk + c) * n_blk;
+  for (int j = lane; j < n_blk; j += 64) out[j] = cnt[j];
+}
+
+// pos = the exclusive scan of every list's counts over its chunks, and the
+// lists' totals (64 lists a workgroup, one a lane; each of the 16 waves sums,
+// then scans, a sixteenth of the chunks).  The chunk-major counts keep every
+// access of the three kernels on consecutive addresses.  List-major, with a
+// library scan of all counts and a launch for the offsets, the build took 85
+// us at 4 x 512 lists x 512 chunks and 330 us at 2 x 2048 x 2048; 41 and 160 now
+// (without pair_bh, whose scattered stores were half of the placing).
+__global__ __launch_bounds__(1024) void k_csr_scan(const int32_t* __restrict__ counts, int32_t* __restrict__ pos,
+                                                   int32_t* __restrict__ totals, int n_blk, int nchunk) {
+  __shared__ int part[16][64];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int bh = blockIdx.y, j = blockIdx.x * 64 + lane;
+  const bool ok = j < n_blk;
+  const int cw = (nchunk + 15) / 16;
+  const int c0 = w * cw, c1 = c0 + cw < nchunk ? c0 + cw : nchunk;
+  const int64_t row0 = (int64_t)bh * nchunk * n_blk + j;
+  int v[16];
+  auto load = [&](int c) {
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = ok && c + u < c1 ? counts[row0 + (int64_t)(c + u) * n_blk] : 0;
+  };
+  int sum = 0;
+  for (int c = c0; c < c1; c += 16) {
+    load(c);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) sum += v[u];
+  }
+  part[w][lane] = sum;
+  __syncthreads();
+  int pre = 0;
+  for (int i = 0; i < w; ++i) pre += part[i][lane];
+  for (int c = c0; c < c1; c += 16) {
+    if (cw > 16) load(c);   // (up to 16 chunks a wave are still in registers)
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      if (ok && c + u < c1) pos[row0 + (int64_t)(c + u) * n_blk] = pre;
+      pre += v[u];
+    }
+  }
+  if (w == 15 && ok) totals[(int64_t)bh * n_blk + j] = pre;   // the last wave ends at the list's total
+}
+
+// Exclusive prefix of x over the wave, and its sum
+__device__ __forceinline__ int csr_wave_scan(int x, int lane, int& sum) {
+  int incl = x;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int y = __shfl_up(incl, off, 64);
+    incl += lane >= off ? y : 0;
+  }
+  sum = __builtin_amdgcn_readlane(incl, 63);
+  return incl - x;
+}
+
+// Lists past which the starts take a launch of their own (each wave of
+// k_csr_place would scan all totals: 151 us instead of 111 + 5 at 4096 lists,
+// 27 either way at 2048).
+constexpr int kCsrOwnScan = 2048;
+// totals -> starts, in place, N lists; totals[N] = their sum
+__global__ __launch_bounds__(1024) void k_csr_base(int32_t* __restrict__ totals, int N) {
+  __shared__ int part[16];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  int carry = 0;
+  for (int i0 = 0; i0 < N; i0 += 4096) {
+    int v[4], mine = 0, sum;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      v[u] = i0 + 4 * tid + u < N ? totals[i0 + 4 * tid + u] : 0;
+      mine += v[u];
+    }
+    int ex = carry + csr_wave_scan(mine, lane, sum);
+    __syncthreads();   // part's last readers are done
+    if (lane == 0) part[w] = sum;
+    __syncthreads();
+    for (int i = 0; i < 16; ++i) {
+      ex += i < w ? part[i] : 0;
+      carry += part[i];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (i0 + 4 * tid + u < N) totals[i0 + 4 * tid + u] = ex;
+      ex += v[u];
+    }
+  }
+  if (tid == 0) totals[N] = carry;
 }
 
 // LDS of the place kernel, in ints: list slots run[n_blk], query masks
@@ -155,18 +223,23 @@ __host__ __device__ inline int64_t csr_place_lds_ints(int n_blk, int S) {
   return r + 2 * (int64_t)n_blk + (int64_t)kCsrChunkQ * S + 2;
 }
 
-// pos = exclusive scan of counts: the chunk's first slot in each list.  Lane
-// q takes query t0 + q: its S indices are staged in LDS and its bit set in the
+// The chunk's first slot in each list is the list's start + pos; the starts of
+// bh's lists are the sum of all totals before bh and a scan of its own (or,
+// with own_scan = 0, read from k_csr_base's).  The first chunk's wave writes
+// bh's row of offsets (the last bh's also *count).  Lane q takes query t0 + q: its S indices are staged in LDS and its bit set in the
 // 64-bit query mask of each of its blocks.  A pair of query q on block j then
 // lands at run[j] + popcount(mask[j] & bits below q): the pairs of block j
 // from earlier queries of the chunk come first.  A row holding one block
 // twice (an atomicOr that finds its bit already set) makes the chunk take the
 // exact walk instead: pairs in input order, 64 a slice, each slot its list's
 // running slot plus the earlier lanes of the slice on the same block (ballot
-// per distinct block of the slice).
+// per distinct block of the slice).  The entries past the last pair are -1.
 __global__ __launch_bounds__(64) void k_csr_place(const int32_t* __restrict__ idx, const int32_t* __restrict__ pos,
+                                                  const int32_t* __restrict__ totals, int own_scan,
+                                                  int32_t* __restrict__ offsets, int32_t* __restrict__ count,
                                                   int32_t* __restrict__ q_of_block, int32_t* __restrict__ pair_bh,
-                                                  int T, int S, int n_blk, int L, int nchunk, int pack_slot) {
+                                                  int T, int S, int n_blk, int L, int nchunk, int pack_slot,
+                                                  int64_t cap) {
   extern __shared__ int run[];
   uint64_t* mask = (uint64_t*)(run + (((int64_t)n_blk + 1) & ~(int64_t)1));
   int* stage = (int*)(mask + n_blk);
@@ -179,7 +252,53 @@ __global__ __launch_bounds__(64) void k_csr_place(const int32_t* __restrict__ id
   const int sbits = sel_slot_bits(S);
   for (int j = lane; j < n_blk; j += 64) mask[j] = 0;
   if (lane == 0) *dup = 0;
-  csr_lds_rows(run, pos + (int64_t)bh * n_blk * nchunk + c, n_blk, nchunk, lane);
+  const int32_t* prow = pos + ((int64_t)bh * nchunk + c) * n_blk;
+  const int nbh = gridDim.y, N = nbh * n_blk, l0 = bh * n_blk;
+  int32_t* orow = offsets + (int64_t)bh * (n_blk + 1);
+  int total;   // pairs of all lists
+  if (own_scan) {
+    int before = 0, rest = 0;   // pairs of the lists before bh's, and of the others
+    for (int i0 = 0; i0 < N; i0 += 16 * 64) {
+      int v[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) v[u] = i0 + 64 * u + lane < N ? totals[i0 + 64 * u + lane] : 0;
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        before += i0 + 64 * u + lane < l0 ? v[u] : 0;
+        rest += i0 + 64 * u + lane < l0 ? 0 : v[u];
+      }
+    }
+    int start, sum;
+    csr_wave_scan(before, lane, start);
+    csr_wave_scan(rest, lane, sum);
+    total = start + sum;
+    for (int j0 = 0; j0 < n_blk; j0 += 64) {
+      const int j = j0 + lane;
+      const int v = j < n_blk ? totals[l0 + j] : 0;
+      const int p = j < n_blk ? prow[j] : 0;
+      const int ex = start + csr_wave_scan(v, lane, sum);
+      if (j < n_blk) {
+        run[j] = ex + p;
+        if (c == 0) orow[j] = ex;
+      }
+      start += sum;
+    }
+    if (c == 0 && lane == 0) orow[n_blk] = start;
+  } else {
+    total = totals[N];
+    for (int j = lane; j < n_blk; j += 64) {
+      const int ex = totals[l0 + j];
+      run[j] = ex + prow[j];
+      if (c == 0) orow[j] = ex;
+    }
+    if (c == 0 && lane == 0) orow[n_blk] = totals[l0 + n_blk];   // the next list's start, or the sum
+  }
+  if (c == 0 && bh == nbh - 1 && lane == 0) *count = total;
+  for (int64_t e = total + ((int64_t)bh * gridDim.x + c) * 64 + lane; e < cap;
+       e += (int64_t)gridDim.x * gridDim.y * 64) {
+    q_of_block[e] = -1;
+    if (pair_bh) pair_bh[e] = -1;
+  }
   csr_chunk_loads(idx, e0, ne, lane, [&](int i, int j) { stage[i] = j; });
   __syncthreads();
   const int t = t0 + lane;
@@ -238,33 +357,19 @@ __global__ __launch_bounds__(64) void k_csr_place(const int32_t* __restrict__ id
   }
 }
 
-// offsets[bh][j] = first slot of list (bh, j) (j = n_blk: the end of bh's
-// lists), *count = number of pairs, tails of q_of_block / pair_bh = -1
-__global__ __launch_bounds__(256) void k_csr_finish(const int32_t* __restrict__ counts,
-                                                    const int32_t* __restrict__ pos, int64_t M, int nbh, int n_blk,
-                                                    int nchunk, int32_t* __restrict__ offsets,
-                                                    int32_t* __restrict__ count, int32_t* __restrict__ q_of_block,
-                                                    int32_t* __restrict__ pair_bh, int64_t cap) {
-  const int32_t total = M > 0 ? pos[M - 1] + counts[M - 1] : 0;
-  const int64_t noff = (int64_t)nbh * (n_blk + 1);
+// no block or no query: every list empty, every entry unused
+__global__ __launch_bounds__(256) void k_csr_empty(int64_t noff, int32_t* __restrict__ offsets,
+                                                   int32_t* __restrict__ count, int32_t* __restrict__ q_of_block,
+                                                   int32_t* __restrict__ pair_bh, int64_t cap) {
   const int64_t n = noff > cap ? noff : cap;
   for (int64_t e = blockIdx.x * 256ll + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
-    if (e < noff) {
-      const int bh = (int)(e / (n_blk + 1)), j = (int)(e % (n_blk + 1));
-      const int64_t k = (int64_t)bh * n_blk + j;   // j == n_blk: the next bh's first list
-      offsets[e] = (M > 0 && k < (int64_t)nbh * n_blk) ? pos[k * nchunk] : total;
-    }
-    if (e >= total && e < cap) {
+    if (e < noff) offsets[e] = 0;
+    if (e < cap) {
       q_of_block[e] = -1;
       if (pair_bh) pair_bh[e] = -1;
     }
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) *count = total;
-}
-
-static inline hipError_t csr_scan(void* temp, size_t& bytes, const int32_t* in, int32_t* out, int64_t M,
-                                  hipStream_t s) {
-  return rocprim::exclusive_scan(temp, bytes, in, out, (int32_t)0, (size_t)M, rocprim::plus<int32_t>(), s);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;
 }
 
 // ---- layout of the workspace -----------------------------------------------------
@@ -274,6 +379,7 @@ struct CsrLayout {
   int nchunk;
   int64_t M;               // counting: nbh * n_blk * nchunk
   size_t keys_in, vals_in, keys_out, temp, temp_bytes, total;
+  size_t totals;   // counting
   int end_bit;
 };
 
@@ -288,14 +394,13 @@ static CsrLayout csr_layout(int B, int Hkv, int T, int S, int n_blk) {
                (int64_t)B * Hkv <= 65535;   // grid y: B*Hkv
   c.end_bit = 0;
   if (c.counting) {
-    // keys_in: counts [M], vals_in: pos [M], temp: the scan's storage
-    c.temp_bytes = 0;
-    (void)csr_scan(nullptr, c.temp_bytes, nullptr, nullptr, c.M, (hipStream_t)0);
+    // keys_in: counts [M], vals_in: pos [M], then the lists' totals
     c.keys_in = 0;
     c.vals_in = c.keys_in + align256(c.M * sizeof(int32_t));
-    c.keys_out = c.vals_in + align256(c.M * sizeof(int32_t));
-    c.temp = c.keys_out;
-    c.total = c.temp + align256(c.temp_bytes) + 256;
+    c.totals = c.vals_in + align256(c.M * sizeof(int32_t));
+    c.total = c.totals + align256(((size_t)B * Hkv * n_blk + 1) * sizeof(int32_t)) + 256;
+    c.keys_out = c.temp = c.total;
+    c.temp_bytes = 0;
     return c;
   }
   const uint64_t sentinel = (uint64_t)B * Hkv * n_blk;
@@ -346,25 +451,27 @@ int nsa_csr_build(const int32_t* block_idx, int32_t* q_of_block, int32_t* block_
   uint32_t* kout = (uint32_t*)(ws + c.keys_out);
   void* temp = ws + c.temp;
   if (c.counting) {
-    const size_t lds_count = (size_t)(n_blk > 0 ? n_blk : 1) * sizeof(int);
+    if (c.M == 0) {
+      const int64_t noff = (int64_t)nbh * (n_blk + 1);
+      k_csr_empty<<<grid_for(noff > c.n ? noff : c.n), 256, 0, s>>>(noff, block_offsets, pair_count, q_of_block,
+                                                                    pair_bh, c.n);
+      return nsa_launch_status();
+    }
+    const size_t lds_count = (size_t)n_blk * sizeof(int);
     const size_t lds = (size_t)csr_place_lds_ints(n_blk, S) * sizeof(int);
     int32_t* counts = (int32_t*)(ws + c.keys_in);
     int32_t* pos = (int32_t*)(ws + c.vals_in);
-    if (c.M > 0) {
-      const dim3 grid((unsigned)c.nchunk, (unsigned)nbh);
-      k_csr_count<<<grid, 64, lds_count, s>>>(block_idx, counts, T, S, n_blk, block_size, c.nchunk);
-      if (hipGetLastError() != hipSuccess) return NSA_ERR_LAUNCH;
-      size_t tb = c.temp_bytes;
-      if (csr_scan(temp, tb, counts, pos, c.M, s) != hipSuccess) return NSA_ERR_LAUNCH;
-      k_csr_place<<<grid, 64, lds, s>>>(block_idx, pos, q_of_block, pair_bh, T, S, n_blk, block_size, c.nchunk,
-                                        pack_slot);
-      if (hipGetLastError() != hipSuccess) return NSA_ERR_LAUNCH;
-    }
-    const int64_t nfin = std::max<int64_t>((int64_t)nbh * (n_blk + 1), c.n);
-    k_csr_finish<<<grid_for(nfin), 256, 0, s>>>(counts, pos, c.M, nbh, n_blk, c.nchunk, block_offsets, pair_count,
-                                                 q_of_block, pair_bh, c.n);
-    if (hipGetLastError() != hipSuccess) return NSA_ERR_LAUNCH;
-    return NSA_OK;
+    int32_t* totals = (int32_t*)(ws + c.totals);
+    const int lists = nbh * n_blk;
+    const bool own_scan = lists <= kCsrOwnScan;
+    const dim3 grid((unsigned)c.nchunk, (unsigned)nbh);
+    k_csr_count<<<grid, 64, lds_count, s>>>(block_idx, counts, T, S, n_blk, block_size, c.nchunk);
+    k_csr_scan<<<dim3((unsigned)((n_blk + 63) / 64), (unsigned)nbh), 1024, 0, s>>>(counts, pos, totals, n_blk,
+                                                                                  c.nchunk);
+    if (!own_scan) k_csr_base<<<1, 1024, 0, s>>>(totals, lists);
+    k_csr_place<<<grid, 64, lds, s>>>(block_idx, pos, totals, own_scan, block_offsets, pair_count, q_of_block, pair_bh,
+                                      T, S, n_blk, block_size, c.nchunk, pack_slot, c.n);
+    return nsa_launch_status();
   }
   if (c.n > 0) {
     k_csr_keys<<<grid_for(c.n), 256, 0, s>>>(block_idx, kin, vin, c.n, T, S, n_blk, block_size,

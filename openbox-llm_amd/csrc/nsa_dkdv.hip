@@ -1859,7 +1859,7 @@ int nsa_sel_dkdv_as(const void* q, const void* k, const void* v, const void* kt,
   int32_t* n_items = (int32_t*)((char*)workspace + cap * sizeof(int4));
   int32_t* first = (int32_t*)((char*)workspace + cap * sizeof(int4) + 256);
   const int nb = B * Hkv * n_blk;
-  k_sel_items<<<1, 1024, 0, s>>>(block_offsets, nb, n_blk, chunk, items, n_items, first);
+  k_sel_items<<<sel_items_grid(nb), 256, 0, s>>>(block_offsets, nb, n_blk, chunk, items, n_items, first);
   if (hipGetLastError() != hipSuccess) return NSA_ERR_LAUNCH;
   const int64_t part_half = (int64_t)cap * sel_passes(block_size) * kSelPass * D;
   // one workgroup per resident slot (two per CU); next_item hands out the rest

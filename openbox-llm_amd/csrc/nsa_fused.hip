@@ -61,7 +61,7 @@ struct Ctx {
   void *k_cmp, *v_cmp, *qp;
   void *o_c, *o_s, *o_w;
   float *lse_c, *lse_s, *lse_w;
-  int32_t *q_of_block, *offsets, *pair_bh, *count;
+  int32_t *q_of_block, *offsets, *count;
 };
 
 Ctx carve_ctx(const Dims& m, void* base, size_t* bytes) {
@@ -80,7 +80,6 @@ Ctx carve_ctx(const Dims& m, void* base, size_t* bytes) {
   const size_t cap = (size_t)m.B * m.Hkv * m.T * m.S();
   x.q_of_block = (int32_t*)c.take(cap * sizeof(int32_t));
   x.offsets = (int32_t*)c.take((size_t)m.B * m.Hkv * (m.nblk() + 1) * sizeof(int32_t));
-  x.pair_bh = (int32_t*)c.take(cap * sizeof(int32_t));
   x.count = (int32_t*)c.take(sizeof(int32_t));
   *bytes = c.off;
   return x;
@@ -230,7 +229,7 @@ int nsa_fused_fwd(const void* q, const void* kc, const void* vc, const void* ks,
     NSA_TRY(nsa_importance_topn(q, k_cmp, x.lse_c, block_idx, nullptr, B, Hq, Hkv, T, n, D, cmp_block, cmp_stride,
                                 sel_block, n_sel, force_init, n_local, dtype, stream));
   // selection partials over the block -> query CSR
-  NSA_TRY(nsa_csr_build(block_idx, x.q_of_block, x.offsets, x.pair_bh, x.count, w.csr_ws, w.csr_bytes, B, Hkv, T,
+  NSA_TRY(nsa_csr_build(block_idx, x.q_of_block, x.offsets, nullptr, x.count, w.csr_ws, w.csr_bytes, B, Hkv, T,
                         S, sel_block, m.nblk(), 1, stream));
   NSA_TRY(nsa_sel_fwd_bo(x.qp, ks, w.vt_s, x.q_of_block, x.offsets, w.o_part, w.ml_part, w.sel_ws, w.sel_bytes, B, Hq,
                          Hkv, T, D, S, sel_block, m.fwd_chunk(), dtype, stream));

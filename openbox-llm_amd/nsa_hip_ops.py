@@ -686,7 +686,7 @@ def sel_dq(q, k, v, kt, do, block_idx, block_size, lse, dot, rowscale, dq, accum
                               T, D, S, block_size, L.dtype_code(q), _stream(q))
 
 
-def csr_device(block_idx, block_size, n_blk=None, pack_slot=False):
+def csr_device(block_idx, block_size, n_blk=None, pack_slot=False, want_bh=True):
     """Block -> query CSR on the GPU without a host sync.
 
     ``n_blk`` defaults to ``ceil(T / block_size)`` (the trailing partial block
@@ -694,7 +694,9 @@ def csr_device(block_idx, block_size, n_blk=None, pack_slot=False):
     ``T // block_size`` (nsa_fsa.py:36).  ``pack_slot``: q_of_block holds
     ``(t << ceil(log2 S)) | s`` (query and slot of the pair).  Returns (q_of_block [cap],
     block_offsets [B,Hkv,n_blk+1], pair_bh [cap], pair_count [1]) int32;
-    entries past pair_count are unused.
+    entries past pair_count are unused.  ``want_bh=False``: pair_bh (which the
+    selection kernels do not read) is None; its scattered stores are half of
+    the placing.
     """
     idx = block_idx.to(torch.int32).contiguous()
     B, Hkv, T, S = idx.shape
@@ -703,7 +705,7 @@ def csr_device(block_idx, block_size, n_blk=None, pack_slot=False):
     cap = B * Hkv * T * S
     dev = idx.device
     q_of_block = torch.empty(max(cap, 1), device=dev, dtype=torch.int32)
-    pair_bh = torch.empty(max(cap, 1), device=dev, dtype=torch.int32)
+    pair_bh = torch.empty(max(cap, 1), device=dev, dtype=torch.int32) if want_bh else None
     offsets = torch.empty(B, Hkv, n_blk + 1, device=dev, dtype=torch.int32)
     count = torch.empty(1, device=dev, dtype=torch.int32)
     ws_bytes = int(_lib().nsa_csr_workspace(B, Hkv, T, S, n_blk))
@@ -737,7 +739,7 @@ def sel_dkdv(q, k, v, do, coff, dot, block_idx, block_size, csr=None, kt=None, w
     idx = block_idx.to(torch.int32).contiguous()
     S = idx.shape[-1]
     if csr is None:
-        csr = csr_device(idx, block_size, pack_slot=want_dq)
+        csr = csr_device(idx, block_size, pack_slot=want_dq, want_bh=False)
     q_of_block, offsets, _, count = csr
     dt = torch.float32 if not DETERMINISTIC_DKDV else out_dtype   # atomic merges add in float32
     dk = torch.empty(B, Hkv, T, D, device=q.device, dtype=dt)
@@ -904,7 +906,8 @@ class SelectionAttnHIP(torch.autograd.Function):
         # and dK (the same choice as the fused layer's branch outputs)
         # the packed Q copy both block-outer kernels read, made once
         qp = pack_heads(q, k.shape[1])
-        (o, o32), lse, csr = sel_fwd_fsa(q, k, v, idx, block_size, qp=qp, o_both=True)
+        csr = csr_device(idx, block_size, pack_slot=True, want_bh=False)
+        (o, o32), lse, _ = sel_fwd_fsa(q, k, v, idx, block_size, csr=csr, qp=qp, o_both=True)
         ctx.save_for_backward(q, k, v, idx, o32, lse, qp, *csr)
         ctx.block_size = block_size
         return o
