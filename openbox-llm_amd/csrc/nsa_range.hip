@@ -107,21 +107,23 @@ __device__ __forceinline__ FullSpan full_span(int mode, int tw0, int qpw, int T_
 // the rows (t, g) of one (b, hkv) are numbered t G + g, a workgroup owns 128
 // consecutive ones and a wave 32 (row n: rw0 + n), so only the sequence's last
 // tile has empty rows where a head chunk would leave 16 - G of every 16 empty.
+// With RG < 4 the workgroup's four waves are RG row groups (this wave's: rg)
+// and 4 / RG key parts, and the workgroup owns RG / 4 of those rows.
 // qpb / qpw count the queries the workgroup's / wave's rows touch; a wave past
 // the last row gets tw0 = T (no valid row).
 struct RangeRows {
   int tb0, qpb, tw0, qpw, rw0;
 };
-template <bool FLAT, int NT>
-__device__ __forceinline__ bool range_rows(RangeRows& r, int qt, int w, int G, int T_) {
+template <bool FLAT, int NT, int RG>
+__device__ __forceinline__ bool range_rows(RangeRows& r, int qt, int rg, int G, int T_) {
   if constexpr (FLAT) {
     static_assert(NT == 1, "flat rows: one 32-row tile per wave");
     const int nrow = T_ * G;
-    const int rb0 = qt * 128;
+    const int rb0 = qt * 32 * RG;
     if (rb0 >= nrow) return false;
     r.tb0 = rb0 / G;
-    r.qpb = (rb0 + 127 < nrow ? rb0 + 127 : nrow - 1) / G - r.tb0 + 1;
-    r.rw0 = rb0 + 32 * w;
+    r.qpb = (rb0 + 32 * RG - 1 < nrow ? rb0 + 32 * RG - 1 : nrow - 1) / G - r.tb0 + 1;
+    r.rw0 = rb0 + 32 * rg;
     if (r.rw0 < nrow) {
       r.tw0 = r.rw0 / G;
       r.qpw = (r.rw0 + 31 < nrow ? r.rw0 + 31 : nrow - 1) / G - r.tw0 + 1;
@@ -130,10 +132,10 @@ __device__ __forceinline__ bool range_rows(RangeRows& r, int qt, int w, int G, i
       r.qpw = 1;
     }
   } else {
-    r.tb0 = qt * 8 * NT;
+    r.tb0 = qt * 2 * NT * RG;
     if (r.tb0 >= T_) return false;
-    r.qpb = 8 * NT;
-    r.tw0 = r.tb0 + w * 2 * NT;
+    r.qpb = 2 * NT * RG;
+    r.tw0 = r.tb0 + rg * 2 * NT;
     r.qpw = 2 * NT;
     r.rw0 = 0;
   }
@@ -152,9 +154,50 @@ __device__ __forceinline__ void range_row(const RangeRows& r, const RangeMap& mp
   }
 }
 // query tiles of a range launch per (b, hkv, head chunk)
-__host__ __device__ inline int range_qtiles(bool flat, int T, int G, int NT) {
-  return flat ? (T * G + 127) / 128 : (T + 8 * NT - 1) / (8 * NT);
+__host__ __device__ inline int range_qtiles(bool flat, int T, int G, int NT, int RG) {
+  return flat ? (T * G + 32 * RG - 1) / (32 * RG) : (T + 2 * NT * RG - 1) / (2 * NT * RG);
 }
+
+// Key parts (KP = 2 or 4): launches of few workgroups, where one more partial
+// round of them, or CUs without any, costs more than the merge.  The waves of
+// a row group take the workgroup's key tiles in turn -- KP tiles a step, one
+// per part, two steps in LDS (for KP = 2 the same bytes as four single tiles)
+// -- and their accumulators are merged in LDS afterwards, in part order.
+// KP tiles from step s on: request(i, slot) for tiles i = s KP .. (a tile past
+// the last repeats it), body(tile, slot) for this wave's tile.
+template <int KP, int LT, typename Req, typename Body>
+__device__ __forceinline__ void key_pipeline_parts(int ntile, int kp, Req request, Body body) {
+  static_assert(KP * LT < 64, "in-flight operations exceed the vmcnt range");
+  const int nstep = (ntile + KP - 1) / KP;
+  auto req = [&](int s) {
+#pragma unroll
+    for (int p = 0; p < KP; ++p) {
+      const int i = s * KP + p;
+      request(i < ntile ? i : ntile - 1, (s & 1) * KP + p);
+    }
+  };
+  if (nstep > 0) req(0);
+  for (int s = 0; s < nstep; ++s) {
+    vm_wait<0>();
+    __syncthreads();   // step s is in LDS, step s - 1 retired by every wave
+    if (s + 1 < nstep) req(s + 1);
+    const int i = s * KP + kp;
+    if (i < ntile) body(i, (s & 1) * KP + kp);
+  }
+}
+// LDS bytes of the parts' exchange: the parts after the first, DT accumulator
+// tiles and two row statistics a lane
+template <int D, int KP> constexpr int parts_bytes() {
+  return (KP - 1) * (4 / KP) * 64 * (16 * ((D + 31) / 32) + 2) * (int)sizeof(float);
+}
+// Parts 1 .. KP - 1 of a row group hand v(0) .. v(n - 1) to part 0 through
+// LDS: put by kp > 0, then (after a barrier) part 0 reads part p's element e
+// at get(p, e).
+struct PartsLds {
+  float* base;
+  int n, rg, RG, lane;
+  __device__ __forceinline__ float* at(int p, int e) const { return base + (((p - 1) * RG + rg) * n + e) * 64 + lane; }
+};
 
 // ---------------------------------------------------------------------------
 // forward
@@ -170,6 +213,18 @@ __host__ __device__ inline int range_qtiles(bool flat, int T, int G, int NT) {
 // float when the caller keeps them unrounded for the backward's row dots, or
 // f16 for the NSA_F16S form (fp16 rows, a float32 scale per row after them:
 // o_scale, o_sel_scale, o_cmp_scale).
+template <typename T, int D, int KP> constexpr int range_fwd_lds() {
+  const int stages = (KP == 1 ? 4 : 2 * KP) * (Tile32<T, D>::ROW_ELEMS + Tile32<T, D>::COL_ELEMS) * (int)sizeof(T);
+  const int fin = 4 / KP * 32 * (D + 4) * (int)sizeof(float);
+  const int ex = parts_bytes<D, KP>();
+  return stages > fin ? (stages > ex ? stages : ex) : (fin > ex ? fin : ex);
+}
+template <typename T, int D, int KP> constexpr int range_dq_lds() {
+  const int stages = (KP == 1 ? 3 : 2 * KP) * (2 * Tile32<T, D>::ROW_ELEMS + Tile32<T, D>::COL_ELEMS) * (int)sizeof(T);
+  const int fin = 4 / KP * 32 * (D + 4) * (int)sizeof(float);
+  const int ex = parts_bytes<D, KP>();
+  return stages > fin ? (stages > ex ? stages : ex) : (fin > ex ? fin : ex);
+}
 template <typename T, typename TO> struct FwdExtras {
   T* q_packed;             // [B][Hkv][T][G][D] (nullable)
   const PartT<T>* opart;   // [B][Hkv][T][NS][G][D] unnormalised block-local outputs O_j = sum p v
@@ -190,36 +245,40 @@ template <typename T, typename TO> struct FwdExtras {
 // The wave's own output rows (this branch, unnormalised acc with the row
 // statistics l_, m_) go through LDS so that every row is handled in 8-element
 // chunks: lane (row sub-index, chunk) per pass.
-template <typename T, typename TO, int D, bool FLAT>
+// KP key parts: w is the wave's row group, whose accumulators part 0 holds; its
+// rows are finished by the group's KP waves in turn.
+template <typename T, typename TO, int D, bool FLAT, int KP>
 __device__ __forceinline__ void finish_rows(const FwdExtras<T, TO>& f, const f32x16 (&acc)[Tile32<T, D>::DT][1],
                                             float l_row, float m_row, bool any_key, bool rok, int64_t row, TO* o,
-                                            float* lse, char* smem, int w, int lane, const RangeRows& rr,
-                                            const RangeMap& mp, int Hq, int Hkv, int T_) {
+                                            float* lse, char* smem, int w, int kp, int lane,
+                                            const RangeRows& rr, const RangeMap& mp, int Hq, int Hkv, int T_) {
   using C = Tile32<T, D>;
   constexpr int FIN_PITCH = D + 4;
   const int h = lane >> 5, n = lane & 31;
   const float lt = l_row + __shfl_xor(l_row, 32, kWave);
   const float inv = any_key ? 1.0f / lt : 0.0f;
-  if (rok && h == 0) lse[row] = any_key ? (m_row + __log2f(lt)) * kLn2 : kLseEmpty;
+  if (kp == 0 && rok && h == 0) lse[row] = any_key ? (m_row + __log2f(lt)) * kLn2 : kLseEmpty;
   __syncthreads();   // the key stages are free
   float* fin = reinterpret_cast<float*>(smem) + w * 32 * FIN_PITCH;
+  if (kp == 0) {
 #pragma unroll
-  for (int dt = 0; dt < C::DT; ++dt)
+    for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      const int d = 32 * dt + 8 * g4 + 4 * h;
-      if (D % 32 == 0 || d < D)
-        *reinterpret_cast<f32x4*>(fin + n * FIN_PITCH + d) =
-            (f32x4){acc[dt][0][4 * g4], acc[dt][0][4 * g4 + 1], acc[dt][0][4 * g4 + 2], acc[dt][0][4 * g4 + 3]} *
-            inv;
-    }
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const int d = 32 * dt + 8 * g4 + 4 * h;
+        if (D % 32 == 0 || d < D)
+          *reinterpret_cast<f32x4*>(fin + n * FIN_PITCH + d) =
+              (f32x4){acc[dt][0][4 * g4], acc[dt][0][4 * g4 + 1], acc[dt][0][4 * g4 + 2], acc[dt][0][4 * g4 + 3]} *
+              inv;
+      }
+  }
   __syncthreads();
   constexpr int CPR = D / 8, RPI = 64 / CPR;   // 8-element chunks per row, rows per pass
   const int c8 = lane % CPR, rsub = lane / CPR;
   const int nsub = sel_passes(f.sel_L), n_csr = sel_csr_blocks(T_, f.sel_L);
   const int G = mp.G;
   const int64_t bh = (int64_t)mp.b * Hkv + mp.hkv;
-  for (int r0 = 0; r0 < 32; r0 += RPI) {
+  for (int r0 = kp * RPI; r0 < 32; r0 += KP * RPI) {
     const int r = r0 + rsub;
     int t, gl;   // query and head within the group
     range_row<FLAT>(rr, mp, 0, r, t, gl);
@@ -373,23 +432,24 @@ __device__ __forceinline__ void fwd_tile(f32x16 (&acc)[DT][NT], float (&m_)[NT],
   }
 }
 
-template <typename T, int D, int NT, typename TO, bool FLAT>
+// KP: key parts (key_pipeline_parts), 1 where the grid fills its rounds.
+template <typename T, int D, int NT, typename TO, bool FLAT, int KP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_range_fwd32(int mode, const T* __restrict__ q, const T* __restrict__ k,
                                                      const T* __restrict__ vt, TO* __restrict__ o,
                                                      float* __restrict__ lse, int Hq, int Hkv, int T_, int Lk,
                                                      int Lp, int nqt, int window, int cl, int cd, float sl2,
                                                      const FwdExtras<T, TO> fin_args) {
   using C = Tile32<T, D>;
-  constexpr int NST = 4;   // key tiles in flight + 1
-  // one LDS buffer: the key stages during the walk, then (finishing rows)
-  // each wave's float output tile [32][D + 4]
-  constexpr int FIN_PITCH = D + 4;
-  constexpr int STAGE_BYTES = NST * (C::ROW_ELEMS + C::COL_ELEMS) * (int)sizeof(T);
-  constexpr int FIN_BYTES = 4 * 32 * FIN_PITCH * (int)sizeof(float);
-  __shared__ __align__(16) char smem[STAGE_BYTES > FIN_BYTES ? STAGE_BYTES : FIN_BYTES];
+  constexpr int NST = KP == 1 ? 4 : 2 * KP;   // key tiles in LDS
+  constexpr int RG = 4 / KP;
+  // one LDS buffer: the key stages during the walk, then the parts' exchange,
+  // then (finishing rows) each row group's float output tile [32][D + 4]
+  __shared__ __align__(16) char smem[range_fwd_lds<T, D, KP>()];
   T (*sK)[C::ROW_ELEMS] = reinterpret_cast<T (*)[C::ROW_ELEMS]>(smem);
   T (*sV)[C::COL_ELEMS] = reinterpret_cast<T (*)[C::COL_ELEMS]>(smem + NST * C::ROW_ELEMS * sizeof(T));
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, n = lane & 31;
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, n = lane & 31;
+  const int wv = KP == 1 ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);   // parts branch on it
+  const int w = wv % RG, kp = wv / RG;   // row group and key part
   // window: neighbouring query tiles (which share keys) on one XCD;
   // compression: every tile reads the same small key set and the work grows
   // with t, so tiles go out round-robin, longest first, to balance the XCDs
@@ -398,7 +458,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (mode == NSA_MODE_COMPRESS) qt = nqt - 1 - qt;   // long rows first
   const RangeMap mp = range_map(wg / nqt, Hq, Hkv);
   RangeRows rr;
-  if (!range_rows<FLAT, NT>(rr, qt, w, mp.G, T_)) return;
+  if (!range_rows<FLAT, NT, RG>(rr, qt, w, mp.G, T_)) return;
   const int tw0 = rr.tw0;
   const RangeSpan sp = range_span(mode, rr.tb0, rr.qpb, tw0, rr.qpw, T_, Lk, window, cl, cd);
   const FullSpan fs = full_span(mode, tw0, rr.qpw, T_, Lk, window, cl, cd);
@@ -421,7 +481,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     visible_range(mode, t < T_ ? t : T_ - 1, Lk, window, cl, cd, lo[nt], hi[nt]);
 #pragma unroll
     for (int s = 0; s < C::KS; ++s) qf[nt][s].load(q + srow * D + 16 * s + 8 * h);
-    if (fin_args.q_packed != nullptr && rok[nt]) {
+    if (fin_args.q_packed != nullptr && rok[nt] && kp == 0) {
       T* dst = fin_args.q_packed + (((int64_t)bh * T_ + t) * mp.G + g) * D;
 #pragma unroll
       for (int s = 0; s < C::KS; ++s) qf[nt][s].store(dst + 16 * s + 8 * h);
@@ -450,27 +510,61 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   kdma.init(tid);
   vdma.init(tid, Lp);
   constexpr int LT = decltype(kdma)::NL + decltype(vdma)::NL;
-  // unrolled over the stages (immediate stage addresses): 1-2% faster here;
-  // the dQ and the top-n walk measured no gain from it
-  key_pipeline_st<NST, LT>(ntile, [&](int i, auto st) {
-    kdma.request(sK[decltype(st)::value], kbase, kt0 + 32 * i, Lk, tid);
-    vdma.request(sV[decltype(st)::value], vtbase, kt0 + 32 * i, tid);
-  }, [&](int it, auto st) {
+  // every wave takes every tile of the workgroup range (its part's, with KP >
+  // 1; the waves' own ranges differ by at most a few queries); tiles inside the
+  // wave's fully visible span skip the per-element mask
+  auto tile = [&](int it, int slot) {
     const int kb = kt0 + 32 * it;
-    // every wave takes every tile of the workgroup range (the waves' own ranges
-    // differ by at most a few queries); tiles inside the wave's fully visible
-    // span skip the per-element mask
     const bool mask = !(kb >= fs.lo && kb + 31 <= fs.hi);
-    fwd_tile<T, D, NT>(acc, m_, l_, qf, sK[decltype(st)::value], sV[decltype(st)::value], kb, mask, lo, hi, sl2, n,
-                       h, mode == NSA_MODE_WINDOW);
-  });
+    fwd_tile<T, D, NT>(acc, m_, l_, qf, sK[slot], sV[slot], kb, mask, lo, hi, sl2, n, h, mode == NSA_MODE_WINDOW);
+  };
+  auto request = [&](int i, int slot) {
+    kdma.request(sK[slot], kbase, kt0 + 32 * i, Lk, tid);
+    vdma.request(sV[slot], vtbase, kt0 + 32 * i, tid);
+  };
+  if constexpr (KP == 1) {
+    // unrolled over the stages (immediate stage addresses): 1-2% faster here;
+    // the dQ and the top-n walk measured no gain from it
+    key_pipeline_st<NST, LT>(ntile, [&](int i, auto st) { request(i, decltype(st)::value); },
+                             [&](int it, auto st) { tile(it, decltype(st)::value); });
+  } else {
+    key_pipeline_parts<KP, LT>(ntile, kp, request, tile);
+    static_assert(KP == 1 || NT == 1, "one 32-row tile per wave is merged");
+    // merge the parts: part 0 rescales to the common maximum
+    const PartsLds px{reinterpret_cast<float*>(smem), 16 * C::DT + 2, w, RG, lane};
+    __syncthreads();   // the key stages are free
+    if (kp > 0) {
+      *px.at(kp, 0) = m_[0];
+      *px.at(kp, 1) = l_[0];
+#pragma unroll
+      for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) *px.at(kp, 2 + 16 * dt + e) = acc[dt][0][e];
+    }
+    __syncthreads();
+    if (kp == 0) {
+#pragma unroll
+      for (int p = 1; p < KP; ++p) {
+        const float mo = *px.at(p, 0);
+        const float mn = fmaxf(m_[0], mo);
+        const float a = fast_exp2(m_[0] - mn), b = fast_exp2(mo - mn);
+        l_[0] = l_[0] * a + *px.at(p, 1) * b;
+        m_[0] = mn;
+#pragma unroll
+        for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[dt][0][e] = acc[dt][0][e] * a + *px.at(p, 2 + 16 * dt + e) * b;
+      }
+    }
+  }
 
   if (fin_args.opart != nullptr) {
     static_assert(NT == 1, "one 32-row tile per wave is staged");
-    finish_rows<T, TO, D, FLAT>(fin_args, acc, l_[0], m_[0], lo[0] <= hi[0], rok[0], row[0], o, lse, smem, w,
-                                lane, rr, mp, Hq, Hkv, T_);
+    finish_rows<T, TO, D, FLAT, KP>(fin_args, acc, l_[0], m_[0], lo[0] <= hi[0], rok[0], row[0], o, lse, smem, w, kp,
+                                    lane, rr, mp, Hq, Hkv, T_);
     return;
   }
+  if (kp > 0) return;
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const float lt = l_[nt] + __shfl_xor(l_[nt], 32, kWave);
@@ -579,7 +673,7 @@ __device__ __forceinline__ void dq_tile(f32x16 (&acc)[DT][NT], const Frag<T> (&q
       for (int nt = 0; nt < NT; ++nt) mma32(acc[dt][nt], ka[dt][s], dsf[nt][s]);
 }
 
-template <typename T, int D, int NT, bool FLAT>
+template <typename T, int D, int NT, bool FLAT, int KP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_range_dq32(int mode, const T* __restrict__ q, const T* __restrict__ k,
                                                     const T* __restrict__ v, const T* __restrict__ kt,
                                                     const T* __restrict__ dout, const float* __restrict__ lse,
@@ -591,23 +685,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                                                     T* __restrict__ dq_out, float* __restrict__ dq_out32, int S,
                                                     int sel_L, DqWindow<T> w2) {
   using C = Tile32<T, D>;
-  constexpr int NST = 3;   // key tiles in flight + 1
-  // one LDS buffer: the key stages during the walk, then (finishing rows)
-  // each wave's float dQ tile [32][D + 4]
+  constexpr int NST = KP == 1 ? 3 : 2 * KP;   // key tiles in LDS
+  constexpr int RG = 4 / KP;
+  // one LDS buffer: the key stages during the walk, then the parts' exchange,
+  // then (finishing rows) each row group's float dQ tile [32][D + 4]
   constexpr int FIN_PITCH = D + 4;
-  constexpr int STAGE_BYTES = NST * (2 * C::ROW_ELEMS + C::COL_ELEMS) * (int)sizeof(T);
-  constexpr int FIN_BYTES = 4 * 32 * FIN_PITCH * (int)sizeof(float);
-  __shared__ __align__(16) char smem[STAGE_BYTES > FIN_BYTES ? STAGE_BYTES : FIN_BYTES];
+  __shared__ __align__(16) char smem[range_dq_lds<T, D, KP>()];
   T (*sK)[C::ROW_ELEMS] = reinterpret_cast<T (*)[C::ROW_ELEMS]>(smem);
   T (*sV)[C::ROW_ELEMS] = reinterpret_cast<T (*)[C::ROW_ELEMS]>(smem + NST * C::ROW_ELEMS * sizeof(T));
   T (*sKt)[C::COL_ELEMS] = reinterpret_cast<T (*)[C::COL_ELEMS]>(smem + 2 * NST * C::ROW_ELEMS * sizeof(T));
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, n = lane & 31;
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, n = lane & 31;
+  const int wv = KP == 1 ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);   // parts branch on it
+  const int w = wv % RG, kp = wv / RG;   // row group and key part
   const int64_t wg = mode == NSA_MODE_COMPRESS ? (int64_t)blockIdx.x : xcd_remap(blockIdx.x, gridDim.x);
   int qt = (int)(wg % nqt);
   if (mode == NSA_MODE_COMPRESS) qt = nqt - 1 - qt;   // long rows first, round-robin (as the forward)
   const RangeMap mp = range_map(wg / nqt, Hq, Hkv);
   RangeRows rr;
-  if (!range_rows<FLAT, NT>(rr, qt, w, mp.G, T_)) return;
+  if (!range_rows<FLAT, NT, RG>(rr, qt, w, mp.G, T_)) return;
   const int tw0 = rr.tw0;
   const int bh = mp.b * Hkv + mp.hkv;
 
@@ -668,21 +763,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     ColTileDma<T, D, 256> ktdma;
     ktdma.init(tid, Lp_);
     constexpr int LT = 2 * decltype(rdma)::NL + decltype(ktdma)::NL;
-    key_pipeline<NST, LT>(ntile, [&](int i) {
-      rdma.request(sK[i % NST], kbase, kt0 + 32 * i, Lk_, tid);
-      rdma.request(sV[i % NST], vbase, kt0 + 32 * i, Lk_, tid);
-      ktdma.request(sKt[i % NST], ktbase, kt0 + 32 * i, tid);
-    }, [&](int it) {
+    auto request = [&](int i, int slot) {
+      rdma.request(sK[slot], kbase, kt0 + 32 * i, Lk_, tid);
+      rdma.request(sV[slot], vbase, kt0 + 32 * i, Lk_, tid);
+      ktdma.request(sKt[slot], ktbase, kt0 + 32 * i, tid);
+    };
+    auto tile = [&](int it, int slot) {
       const int kb = kt0 + 32 * it;
       const bool mask = !(kb >= fs.lo && kb + 31 <= fs.hi);
-      dq_tile<T, D, NT>(acc, qf, df, sK[it % NST], sV[it % NST], sKt[it % NST], kb, mask, lo, hi, c, dlt, sl2, n,
-                        h);
-    });
+      dq_tile<T, D, NT>(acc, qf, df, sK[slot], sV[slot], sKt[slot], kb, mask, lo, hi, c, dlt, sl2, n, h);
+    };
+    if constexpr (KP == 1)
+      key_pipeline<NST, LT>(ntile, [&](int i) { request(i, i % NST); }, [&](int it) { tile(it, it % NST); });
+    else
+      key_pipeline_parts<KP, LT>(ntile, kp, request, tile);
   };
   walk(mode, k, v, kt, lse, dot, rowscale, Lk, Lp);
   if (w2.k != nullptr) {
     __syncthreads();   // every wave is done with the first walk's stages
     walk(NSA_MODE_WINDOW, w2.k, w2.v, w2.kt, w2.lse, w2.dot, w2.rowscale, T_, w2.Lp);
+  }
+
+  if constexpr (KP > 1) {
+    static_assert(KP == 1 || NT == 1, "one 32-row tile per wave is merged");
+    const PartsLds px{reinterpret_cast<float*>(smem), 16 * C::DT, w, RG, lane};
+    __syncthreads();   // the key stages are free
+    if (kp > 0) {
+#pragma unroll
+      for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) *px.at(kp, 16 * dt + e) = acc[dt][0][e];
+    }
+    __syncthreads();
+    if (kp == 0) {
+#pragma unroll
+      for (int p = 1; p < KP; ++p)
+#pragma unroll
+        for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[dt][0][e] += *px.at(p, 16 * dt + e);
+    }
   }
 
   if (sel_part != nullptr) {
@@ -693,22 +813,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     static_assert(NT == 1, "one 32-row tile per wave is staged");
     __syncthreads();   // the key stages are free
     float* fin = reinterpret_cast<float*>(smem) + w * 32 * FIN_PITCH;
+    if (kp == 0) {
 #pragma unroll
-    for (int dt = 0; dt < C::DT; ++dt)
+      for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const int d = 32 * dt + 8 * g4 + 4 * h;
-        if (D % 32 == 0 || d < D)
-          *reinterpret_cast<f32x4*>(fin + n * FIN_PITCH + d) =
-              (f32x4){acc[dt][0][4 * g4], acc[dt][0][4 * g4 + 1], acc[dt][0][4 * g4 + 2], acc[dt][0][4 * g4 + 3]} *
-              scale;
-      }
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const int d = 32 * dt + 8 * g4 + 4 * h;
+          if (D % 32 == 0 || d < D)
+            *reinterpret_cast<f32x4*>(fin + n * FIN_PITCH + d) =
+                (f32x4){acc[dt][0][4 * g4], acc[dt][0][4 * g4 + 1], acc[dt][0][4 * g4 + 2], acc[dt][0][4 * g4 + 3]} *
+                scale;
+        }
+    }
     __syncthreads();
     constexpr int CPR = D / 8, RPI = 64 / CPR;   // 8-element chunks per row, rows per pass
     const int c8 = lane % CPR, rsub = lane / CPR;
     const int nsub = sel_passes(sel_L), n_csr = sel_csr_blocks(T_, sel_L);
     const int G = mp.G;
-    for (int r0 = 0; r0 < 32; r0 += RPI) {
+    for (int r0 = kp * RPI; r0 < 32; r0 += KP * RPI) {   // a row group's KP waves in turn
       const int r = r0 + rsub;
       int t, gl;   // query and head within the group
       range_row<FLAT>(rr, mp, 0, r, t, gl);
@@ -735,6 +857,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     return;
   }
+  if (kp > 0) return;
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     if (!rok[nt]) continue;
@@ -782,6 +905,36 @@ extern "C" {
 
 }  // extern "C"
 
+// Key parts of a launch: g1 workgroups of four row groups, lds[i] bytes of LDS
+// for KP = 1, 2, 4 (0: not built), at most `tiles` key tiles a workgroup.  KP
+// parts make KP times the workgroups of 1 / KP the walk; with s of them
+// resident the launch takes ceil(g1 KP / s) / KP of a whole walk.  Parts are
+// taken where that is at most `worth` of one part's and every part has two
+// tiles or more.  Measured, us of window and compression together, one part
+// -> parts: float32 T1024 Hq4 D64 (32 workgroups a branch) forward 82 -> 40 (4
+// for the window), dQ 82 -> 50 (2); bf16 windows of 1.3 and 1.5 rounds of 512
+// workgroups, where two parts take 0.75 of the rounds: forward T1301 Hq64 D128
+// 160 -> 142, T6011 Hq16 D64 99 -> 98, but the latter's dQ 74 -> 77.  So the
+// forward takes parts at 0.8 and the dQ, whose parts also sum dQ, at 0.7.
+static int key_parts(int64_t g1, const int (&lds)[3], int tiles, double worth) {
+  int best = 1;
+  double cost = 0.0;
+  for (int i = 0; i < 3; ++i) {
+    const int kp = 1 << i;
+    if (lds[i] == 0 || (kp > 1 && tiles < 2 * kp)) continue;
+    int per = 160 * 1024 / lds[i];   // workgroups per CU: by LDS, and two by registers
+    per = per > 2 ? 2 : per;
+    if (per < 1) continue;
+    const int64_t s = 256 * (int64_t)per;
+    const double c = (double)((g1 * kp + s - 1) / s) / kp;
+    if (kp == 1 || c <= worth * cost) {
+      best = kp;
+      cost = c;
+    }
+  }
+  return best;
+}
+
 template <typename E, typename TO>
 static int range_fwd_launch(int mode, const void* q, const void* k, const void* vt, void* o, float* lse, int B,
                             int Hq, int Hkv, int T, int Lk, int D, int window, int cmp_block, int cmp_stride,
@@ -792,11 +945,20 @@ static int range_fwd_launch(int mode, const void* q, const void* k, const void* 
   constexpr int NT = RangeNT<E>::fwd;
   const bool flat = Hq / Hkv < 16;   // flat rows: no empty head slots
   NSA_CHECK((int64_t)T * (Hq / Hkv) < (1ll << 31), NSA_ERR_SHAPE);
-  const int nqt = range_qtiles(flat, T, Hq / Hkv, NT);
-  const int64_t grid = (int64_t)B * Hkv * NHC * nqt;
-  NSA_CHECK(grid < (1ll << 31), NSA_ERR_SHAPE);
+  const int tiles = mode == NSA_MODE_WINDOW ? ((window < T ? window : T) + 31) / 32 + 1 : (Lk + 31) / 32;
   NSA_DISPATCH_D(D, {
-    auto kern = flat ? k_range_fwd32<E, DD, NT, TO, true> : k_range_fwd32<E, DD, NT, TO, false>;
+    constexpr int l1 = range_fwd_lds<E, DD, 1>();
+    constexpr int l2 = range_fwd_lds<E, DD, 2>();
+    constexpr int l4 = range_fwd_lds<E, DD, 4>() <= 160 * 1024 ? range_fwd_lds<E, DD, 4>() : 0;
+    const int lds[3] = {l1, l2, l4};
+    const int kp = key_parts((int64_t)B * Hkv * NHC * range_qtiles(flat, T, Hq / Hkv, NT, 4), lds, tiles, 0.8);
+    const int nqt = range_qtiles(flat, T, Hq / Hkv, NT, 4 / kp);
+    const int64_t grid = (int64_t)B * Hkv * NHC * nqt;
+    NSA_CHECK(grid < (1ll << 31), NSA_ERR_SHAPE);
+    auto kern = flat ? k_range_fwd32<E, DD, NT, TO, true, 1> : k_range_fwd32<E, DD, NT, TO, false, 1>;
+    if (kp == 2) kern = flat ? k_range_fwd32<E, DD, NT, TO, true, 2> : k_range_fwd32<E, DD, NT, TO, false, 2>;
+    if constexpr (l4 > 0)
+      if (kp == 4) kern = flat ? k_range_fwd32<E, DD, NT, TO, true, 4> : k_range_fwd32<E, DD, NT, TO, false, 4>;
     kern<<<(unsigned)grid, 256, 0, s>>>(mode, (const E*)q, (const E*)k, (const E*)vt, (TO*)o, lse, Hq, Hkv, T, Lk,
                                         Lp, nqt, window, cmp_block, cmp_stride, sl2, fin);
   });
@@ -816,11 +978,22 @@ static int range_dq_launch(int mode, const void* q, const void* k, const void* v
   constexpr int NT = RangeNT<E>::dq;
   const bool flat = Hq / Hkv < 16;   // flat rows: no empty head slots
   NSA_CHECK((int64_t)T * (Hq / Hkv) < (1ll << 31), NSA_ERR_SHAPE);
-  const int nqt = range_qtiles(flat, T, Hq / Hkv, NT);
-  const int64_t grid = (int64_t)B * Hkv * NHC * nqt;
-  NSA_CHECK(grid < (1ll << 31), NSA_ERR_SHAPE);
+  int tiles = mode == NSA_MODE_WINDOW ? ((window < T ? window : T) + 31) / 32 + 1 : (Lk + 31) / 32;
+  if (w2.k != nullptr) tiles += ((window < T ? window : T) + 31) / 32 + 1;
   NSA_DISPATCH_D(D, {
-    auto kern = flat ? k_range_dq32<E, DD, NT, true> : k_range_dq32<E, DD, NT, false>;
+    constexpr int l1 = range_dq_lds<E, DD, 1>();
+    constexpr int l2 = range_dq_lds<E, DD, 2>() <= 160 * 1024 ? range_dq_lds<E, DD, 2>() : 0;
+    constexpr int l4 = range_dq_lds<E, DD, 4>() <= 160 * 1024 ? range_dq_lds<E, DD, 4>() : 0;
+    const int lds[3] = {l1, l2, l4};
+    const int kp = key_parts((int64_t)B * Hkv * NHC * range_qtiles(flat, T, Hq / Hkv, NT, 4), lds, tiles, 0.7);
+    const int nqt = range_qtiles(flat, T, Hq / Hkv, NT, 4 / kp);
+    const int64_t grid = (int64_t)B * Hkv * NHC * nqt;
+    NSA_CHECK(grid < (1ll << 31), NSA_ERR_SHAPE);
+    auto kern = flat ? k_range_dq32<E, DD, NT, true, 1> : k_range_dq32<E, DD, NT, false, 1>;
+    if constexpr (l2 > 0)
+      if (kp == 2) kern = flat ? k_range_dq32<E, DD, NT, true, 2> : k_range_dq32<E, DD, NT, false, 2>;
+    if constexpr (l4 > 0)
+      if (kp == 4) kern = flat ? k_range_dq32<E, DD, NT, true, 4> : k_range_dq32<E, DD, NT, false, 4>;
     kern<<<(unsigned)grid, 256, 0, s>>>(mode, (const E*)q, (const E*)k, (const E*)v, (const E*)kt, (const E*)dout,
                                         lse, dot, rowscale, dq, accumulate, Hq, Hkv, T, Lk, Lp, nqt, window,
                                         cmp_block, cmp_stride, sl2, scale, (const E*)sel_part, sel_idx,
