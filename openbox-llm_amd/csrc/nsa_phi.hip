@@ -252,12 +252,17 @@ __global__ __launch_bounds__(256) void k_phi_fold8(const TI* __restrict__ dspan,
 // (group ncg1, dout's channels), and one of `nsplit` token ranges (grid.y),
 // whose sums it writes as float partials.  Both operands are token-major in
 // memory; each 32-token chunk is staged in LDS transposed, token-contiguous
-// rows of which a lane reads 8.  Span g's element k is x[bh][(i d) D + k]
-// (rows i d .. i d + l - 1 are contiguous): the spans are read in place.  bf16:
-// dpre / silu(pre) enter as bf16 hi + lo (two MFMAs, about 16 significant
-// bits), the span / dout operand is exact; float: float MFMAs.  The bias sums
-// run per thread in token order beside the staging and are combined in thread
-// order; k_phi_wgrad_reduce adds the token ranges in order, so every gradient
+// rows of which a lane reads 8.  A thread holds a pair of columns over 8
+// tokens of each operand, loaded one chunk ahead (a wave reads whole row
+// segments; the loads are unconditional, so none waits for another) and
+// written as whole 16-byte runs: what bounds the kernel is the staging, not the
+// MFMAs.  M 8188, H 128, lD 4096: 70 us; with 2-byte transposed stores (8 lanes
+// on a bank) and loads waited for at once it took 153.  Span g's element k is
+// x[bh][(i d) D + k] (rows i d .. i d + l - 1 are contiguous): the spans are
+// read in place.  bf16: dpre / silu(pre) enter as bf16 hi + lo (two MFMAs,
+// about 16 significant bits), the span / dout operand is exact; float: float
+// MFMAs.  The bias sums run per thread in token order beside the staging and
+// are combined in run order; k_phi_wgrad_reduce adds the token ranges in order, so every gradient
 // is the same bits on every run.
 constexpr int kWgCols = 128;   // output columns per workgroup
 constexpr int kWgTok = 32;     // tokens per staged chunk
@@ -271,15 +276,15 @@ __global__ __launch_bounds__(256) void k_phi_wgrad(const T* __restrict__ x, cons
   constexpr int MT = H / 32;
   constexpr int NA = sizeof(T) == 2 ? 2 : 1;           // hi (+ lo) rows of the A operand
   constexpr int P = kWgTok + 16 / (int)sizeof(T);      // row pitch (16-byte rows, skewed banks)
-  constexpr int A4 = H / 4;                            // float4 per token of dpre / pre
-  constexpr int EPC = 16 / (int)sizeof(T);             // elements per 16-byte load of x / dout
-  constexpr int BC = kWgCols / EPC;                    // loads per token of the column group
-  static_assert(256 % A4 == 0 && kWgTok * A4 % 256 == 0 && 256 % BC == 0 && kWgTok * BC % 256 == 0,
-                "fixed thread -> column slots");
+  constexpr int RUN = 8;                               // tokens per staged run
+  constexpr int NRUN = kWgTok / RUN;
+  constexpr int AP = H / 2;                            // column pairs of the A operand
+  static_assert(NRUN * 64 == 256 && 2 * 64 == kWgCols && AP <= 64, "one (run, column pair) per thread");
   __shared__ __align__(16) T sA[NA][H][P];
   __shared__ __align__(16) T sB[kWgCols][P];
-  __shared__ float sred[256][8];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, h = lane >> 5, nn = lane & 31;
+  __shared__ float sred[256][2];
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, nn = lane & 31;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int cg = blockIdx.x, split = blockIdx.y;
   const bool is_w2 = cg == ncg1;
   const bool want_b1 = cg == 0 && !is_w2;
@@ -293,61 +298,84 @@ __global__ __launch_bounds__(256) void k_phi_wgrad(const T* __restrict__ x, cons
   f32x16 acc[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = zero16();
-  float bsum[8];
+  // the thread's operand columns: a pair of hidden units in token run ra, a
+  // pair of output columns in token run w
+  const int pa = tid % AP, ra = tid / AP;
+  const bool has_a = ra < NRUN;
+  const int colp = col0 + 2 * lane;
+  const int colb = colp < ncols ? colp : col0;   // columns past ncols are not stored
+  // (bh, i) of the first token of run w in the next chunk
+  int64_t bh = (ch0 * kWgTok + RUN * w) / n;
+  int64_t ti = ch0 * kWgTok + RUN * w - bh * n;
+  float asum[2] = {0.0f, 0.0f}, bsum[2] = {0.0f, 0.0f};
+  float av[RUN][2];
+  T bv[RUN][2];
+  // unconditional loads (a token past the last reads the last), zeroed when
+  // they are staged
+  auto fetch = [&](int64_t ch) {
+    const int64_t ga = ch * kWgTok + RUN * ra, gb = ch * kWgTok + RUN * w;
+    int64_t b2 = bh, i2 = ti;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) bsum[j] = 0.0f;
-
+    for (int j = 0; j < RUN; ++j) {
+      if (has_a) {
+        const float* p = asrc + (ga + j < M ? ga + j : M - 1) * H + 2 * pa;
+        av[j][0] = p[0];
+        av[j][1] = p[1];
+      }
+      typedef T Pair __attribute__((ext_vector_type(2)));
+      const int64_t row = gb + j >= M ? (is_w2 ? M - 1 : (BH - 1ll) * L + (n - 1ll) * d)
+                                      : (is_w2 ? gb + j : b2 * L + i2 * d);
+      const Pair v = *reinterpret_cast<const Pair*>((is_w2 ? dout : x) + row * D + colb);
+      bv[j][0] = v[0];
+      bv[j][1] = v[1];
+      if (++i2 == n) {
+        i2 = 0;
+        ++b2;
+      }
+    }
+    ti += kWgTok;   // the next chunk's run
+    while (ti >= n) {
+      ti -= n;
+      ++bh;
+    }
+  };
+  if (ch0 < ch1) fetch(ch0);
   for (int64_t ch = ch0; ch < ch1; ++ch) {
-    const int64_t g0 = ch * kWgTok;
-    // A: [32 tokens][H] float -> sA[.][u][token]
+    if (has_a) {
 #pragma unroll
-    for (int j = 0; j < kWgTok * A4 / 256; ++j) {
-      const int e = tid + 256 * j;
-      const int tk = e / A4, u4 = e % A4;
-      const int64_t g = g0 + tk;
-      f32x4 v = (f32x4){0.f, 0.f, 0.f, 0.f};
-      if (g < M) v = *reinterpret_cast<const f32x4*>(asrc + g * H + 4 * u4);
+      for (int c = 0; c < 2; ++c) {
+        float a[RUN];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float a = v[i];
-        if (is_w2) a = silu_f(a);
-        if (want_b1) bsum[i] += a;
+        for (int j = 0; j < RUN; ++j) {
+          a[j] = ch * kWgTok + RUN * ra + j < M ? av[j][c] : 0.0f;
+          if (is_w2) a[j] = silu_f(a[j]);   // silu(0) = 0
+          asum[c] += a[j];
+        }
+        Frag<T> f;
+        f.set(a);
+        f.store(&sA[0][2 * pa + c][RUN * ra]);
         if constexpr (NA == 2) {
-          const bf16 hi = (bf16)a;
-          sA[0][4 * u4 + i][tk] = hi;
-          sA[NA - 1][4 * u4 + i][tk] = (bf16)(a - (float)hi);
-        } else {
-          sA[0][4 * u4 + i][tk] = (T)a;
+#pragma unroll
+          for (int j = 0; j < RUN; ++j) a[j] -= to_f32(f.elem(j));
+          f.set(a);
+          f.store(&sA[NA - 1][2 * pa + c][RUN * ra]);
         }
       }
     }
-    // B: [32 tokens][128 columns] of the spans (dW1) or of dout (dW2) -> sB[column][token]
 #pragma unroll
-    for (int j = 0; j < kWgTok * BC / 256; ++j) {
-      const int e = tid + 256 * j;
-      const int tk = e / BC, cc = e % BC;
-      const int64_t g = g0 + tk;
-      const int col = col0 + cc * EPC;
-      alignas(16) T v[EPC];
+    for (int c = 0; c < 2; ++c) {
+      float b[RUN];
 #pragma unroll
-      for (int q = 0; q < EPC; ++q) v[q] = (T)0.0f;
-      if (g < M && col < ncols) {
-        const T* src;
-        if (is_w2) {
-          src = dout + g * D + col;
-        } else {
-          const int64_t bh = g / n, i = g % n;
-          src = x + (bh * L + i * d) * D + col;
-        }
-        *reinterpret_cast<int4*>(v) = *reinterpret_cast<const int4*>(src);
+      for (int j = 0; j < RUN; ++j) {
+        b[j] = ch * kWgTok + RUN * w + j < M ? to_f32(bv[j][c]) : 0.0f;
+        bsum[c] += b[j];
       }
-#pragma unroll
-      for (int q = 0; q < EPC; ++q) {
-        if (is_w2) bsum[q] += to_f32(v[q]);
-        sB[cc * EPC + q][tk] = v[q];
-      }
+      Frag<T> f;
+      f.set(b);
+      f.store(&sB[2 * lane + c][RUN * w]);
     }
     __syncthreads();
+    if (ch + 1 < ch1) fetch(ch + 1);   // in flight during this chunk's MFMAs
 #pragma unroll
     for (int s = 0; s < kWgTok / 16; ++s) {
       Frag<T> b;
@@ -373,25 +401,39 @@ __global__ __launch_bounds__(256) void k_phi_wgrad(const T* __restrict__ x, cons
       for (int r = 0; r < 16; ++r) dst[(int64_t)(32 * mt + acc_elem(h, r)) * ncols + col] = acc[mt][r];
   }
   if (want_b1 || is_w2) {   // uniform over the workgroup
-#pragma unroll
-    for (int j = 0; j < 8; ++j) sred[tid][j] = bsum[j];
+    sred[tid][0] = is_w2 ? bsum[0] : asum[0];
+    sred[tid][1] = is_w2 ? bsum[1] : asum[1];
     __syncthreads();
-    if (want_b1 && tid < H) {
-      // hidden unit u = 4 u4 + i: the threads with tid % A4 == u4, in thread order
+    // a column's runs, in run order
+    const int np = is_w2 ? 64 : AP;
+    if (tid < (is_w2 ? D : H)) {
       float s = 0.0f;
-      for (int t = tid / 4; t < 256; t += A4) s += sred[t][tid % 4];
-      bpart1[(int64_t)split * H + tid] = s;
-    }
-    if (is_w2 && tid < D) {
-      float s = 0.0f;
-      for (int t = tid / EPC; t < 256; t += BC) s += sred[t][tid % EPC];
-      bpart2[(int64_t)split * D + tid] = s;
+#pragma unroll
+      for (int r = 0; r < NRUN; ++r) s += sred[r * np + tid / 2][tid % 2];
+      (is_w2 ? bpart2 + (int64_t)split * D : bpart1 + (int64_t)split * H)[tid] = s;
     }
   }
 }
 
+// sum over the token ranges, in order, of p[sp * stride] (loads 8 at a time)
+template <typename V> __device__ __forceinline__ V sum_ranges(const float* p, int64_t stride, int nsplit, V s) {
+  typedef V __attribute__((aligned(4))) VU;   // the caller's workspace need only be float-aligned
+  int sp = 0;
+  for (; sp + 8 <= nsplit; sp += 8) {
+    V v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const VU*>(p + (sp + j) * stride);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s += v[j];
+  }
+  for (; sp < nsplit; ++sp) s += *reinterpret_cast<const VU*>(p + sp * stride);
+  return s;
+}
+
 // the token ranges of k_phi_wgrad's partials added in order; one thread per
-// output element of [dW1 | dpos | dW2 | db1 | db2]
+// run of 4 elements of dW1, then one per element of [dpos | dW2 | db1 | db2]
+// (bound by the latency of a thread's loads, which it therefore issues 8 or 16
+// at a time: 16 ranges of 128 x 4096, 27 -> 12 us)
 __global__ __launch_bounds__(256) void k_phi_wgrad_reduce(const float* __restrict__ part1,
                                                           const float* __restrict__ part2,
                                                           const float* __restrict__ bpart1,
@@ -401,34 +443,36 @@ __global__ __launch_bounds__(256) void k_phi_wgrad_reduce(const float* __restric
                                                           float* __restrict__ dw2, float* __restrict__ db1,
                                                           float* __restrict__ db2, int H, int D, int K, int nsplit) {
   __shared__ float sdb1[128];
-  for (int u = threadIdx.x; u < H; u += 256) {
-    float s = 0.0f;
-    for (int sp = 0; sp < nsplit; ++sp) s += bpart1[(int64_t)sp * H + u];
-    sdb1[u] = s;
-  }
+  for (int u = threadIdx.x; u < H; u += 256) sdb1[u] = sum_ranges(bpart1 + u, H, nsplit, 0.0f);
   __syncthreads();
   int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t HK = (int64_t)H * K;
-  if (e < HK) {
-    const int u = (int)(e / K), k = (int)(e % K);
-    float s = 0.0f;
-    for (int sp = 0; sp < nsplit; ++sp) s += part1[sp * HK + e];
-    dw1[e] = s + sdb1[u] * pos[k];
+  if (e < HK / 4) {   // K = l D is a multiple of 64
+    const int u = (int)(4 * e / K), k = (int)(4 * e % K);
+    const f32x4 s = sum_ranges(part1 + 4 * e, HK, nsplit, zero4());
+    float* o = dw1 + 4 * e;
+    const float b = sdb1[u];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = s[j] + b * pos[k + j];
     return;
   }
-  e -= HK;
+  e -= HK / 4;
   if (e < K) {
     float s = 0.0f;
-    for (int u = 0; u < H; ++u) s += sdb1[u] * w1[(int64_t)u * K + e];
+    for (int u0 = 0; u0 < H; u0 += 16) {   // H is a multiple of 32
+      float v[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) v[j] = w1[(int64_t)(u0 + j) * K + e];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) s += sdb1[u0 + j] * v[j];
+    }
     dpos[e] = s;
     return;
   }
   e -= K;
   if (e < (int64_t)D * H) {
     const int c = (int)(e / H), u = (int)(e % H);
-    float s = 0.0f;
-    for (int sp = 0; sp < nsplit; ++sp) s += part2[((int64_t)sp * H + u) * D + c];
-    dw2[e] = s;
+    dw2[e] = sum_ranges(part2 + (int64_t)u * D + c, (int64_t)H * D, nsplit, 0.0f);
     return;
   }
   e -= (int64_t)D * H;
@@ -437,11 +481,7 @@ __global__ __launch_bounds__(256) void k_phi_wgrad_reduce(const float* __restric
     return;
   }
   e -= H;
-  if (e < D) {
-    float s = 0.0f;
-    for (int sp = 0; sp < nsplit; ++sp) s += bpart2[(int64_t)sp * D + e];
-    db2[e] = s;
-  }
+  if (e < D) db2[e] = sum_ranges(bpart2 + e, D, nsplit, 0.0f);
 }
 
 // token ranges of k_phi_wgrad: about two workgroups per CU of a 256-CU part,
@@ -498,7 +538,7 @@ int nsa_phi_wgrad(const void* x, const void* dout, const float* dpre, const floa
     NSA_PHI_WGRAD(float, 32) NSA_PHI_WGRAD(float, 64) NSA_PHI_WGRAD(float, 128)
   }
 #undef NSA_PHI_WGRAD
-  const int64_t total = (int64_t)H * K + K + (int64_t)D * H + H + D;
+  const int64_t total = (int64_t)H * K / 4 + K + (int64_t)D * H + H + D;
   k_phi_wgrad_reduce<<<(unsigned)((total + 255) / 256), 256, 0, s>>>(part1, part2, bpart1, bpart2, pos, w1, dw1,
                                                                       dpos, dw2, db1, db2, H, D, K, ns);
   return nsa_launch_status();
