@@ -262,8 +262,8 @@ __global__ __launch_bounds__(256) void k_phi_fold8(const TI* __restrict__ dspan,
 // read in place.  bf16: dpre / silu(pre) enter as bf16 hi + lo (two MFMAs,
 // about 16 significant bits), the span / dout operand is exact; float: float
 // MFMAs.  The bias sums run per thread in token order beside the staging and
-// are combined in run order; k_phi_wgrad_reduce adds the token ranges in order, so every gradient
-// is the same bits on every run.
+// are combined in run order; k_phi_wgrad_reduce adds the token ranges in order,
+// so every gradient is the same bits on every run.
 constexpr int kWgCols = 128;   // output columns per workgroup
 constexpr int kWgTok = 32;     // tokens per staged chunk
 
