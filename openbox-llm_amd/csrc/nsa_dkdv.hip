@@ -1528,15 +1528,23 @@ __global__ __launch_bounds__(256) void k_sel_dkdv_reduce(const float* __restrict
 // per 4 floats of a key row, summed over the key block's parts (window) or
 // chunks (compression: chunk, then sub-chunk) in query order -- the logical
 // workgroup numbering of kv_work -- so the result does not depend on which
-// workgroup finished first.
-template <int D, int NW, typename TO>
+// workgroup finished first.  RG > 1: RG threads share the 4 floats, each the
+// parts i = g, g + RG, .. of a run, and their sums are added in thread order
+// through LDS: a short sequence's keys are few threads, each a chain of loads
+// over dozens of sub-chunk rows (T6011 Hkv4 D64, 93 keys of 60 rows: 19.2 us at
+// RG 1, 9.5 at 8).
+template <int D, int NW, int RG, typename TO>
 __global__ __launch_bounds__(256) void k_range_dkdv_reduce(const KvRange r, const float* __restrict__ part,
                                                            int64_t part_half, TO* __restrict__ dk,
                                                            TO* __restrict__ dv) {
   constexpr int KB = 32 * NW;
   constexpr int V4 = D / 4;   // float4 per key row
-  const int64_t f = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (f >= (int64_t)r.nbh * r.Lk * V4) return;
+  constexpr int FW = 256 / RG;   // runs of 4 floats per workgroup
+  const int g = threadIdx.x / FW;
+  const int64_t nf = (int64_t)r.nbh * r.Lk * V4;
+  const int64_t f0 = (int64_t)blockIdx.x * FW + threadIdx.x % FW;
+  if (RG == 1 && f0 >= nf) return;
+  const int64_t f = f0 < nf ? f0 : nf - 1;   // RG > 1: every thread reaches the barrier
   const int c = (int)(f % V4);
   const int key = (int)((f / V4) % r.Lk);
   const int bh = (int)(f / ((int64_t)V4 * r.Lk));
@@ -1556,12 +1564,12 @@ __global__ __launch_bounds__(256) void k_range_dkdv_reduce(const KvRange r, cons
     for (int u = 0; u < kRedBatch; ++u)
       if (wgi[u] >= 0) a += xa[u], b += xb[u];
   };
-  // n of them, `step` apart
+  // this thread's share of n of them, `step` apart
   auto add_run = [&](int64_t w0, int64_t step, int n) {
-    for (int i = 0; i < n; i += kRedBatch) {
+    for (int i = g; i < n; i += kRedBatch * RG) {
       int64_t wgi[kRedBatch];
 #pragma unroll
-      for (int u = 0; u < kRedBatch; ++u) wgi[u] = i + u < n ? w0 + (i + u) * step : -1;
+      for (int u = 0; u < kRedBatch; ++u) wgi[u] = i + u * RG < n ? w0 + (i + u * RG) * step : -1;
       add(wgi);
     }
   };
@@ -1577,7 +1585,7 @@ __global__ __launch_bounds__(256) void k_range_dkdv_reduce(const KvRange r, cons
 #pragma unroll
       for (int u = 0; u < kRedBatch; ++u) {
         const int na = c0 + u < r.chs ? cmp_active_blocks(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, c0 + u) : 0;
-        wgi[u] = kblk < na ? base + kblk : -1;
+        wgi[u] = kblk < na && g == 0 ? base + kblk : -1;
         base += na;
       }
       add(wgi);
@@ -1587,6 +1595,18 @@ __global__ __launch_bounds__(256) void k_range_dkdv_reduce(const KvRange r, cons
       const int na = cmp_active_blocks(r.T_, r.Lk, r.chunk, NW, r.cl, r.cd, ch);
       if (kblk < na) add_run(base + kblk, na, r.spl);
       base += (int64_t)na * r.spl;
+    }
+  }
+  if constexpr (RG > 1) {
+    __shared__ f32x4 sa[RG][FW], sb[RG][FW];
+    sa[g][threadIdx.x % FW] = a;
+    sb[g][threadIdx.x % FW] = b;
+    __syncthreads();
+    if (g != 0 || f0 >= nf) return;
+#pragma unroll
+    for (int j = 1; j < RG; ++j) {
+      a += sa[j][threadIdx.x];
+      b += sb[j][threadIdx.x];
     }
   }
   const int64_t orow = ((int64_t)bh * r.Lk + key) * D + 4 * c;
@@ -1612,6 +1632,8 @@ static inline int zero_out(void* x, int64_t n, int dtype, hipStream_t s) {
     default: return NSA_ERR_SHAPE;                              \
   }
 
+static constexpr int kReduceGroups = 8;           // threads of a run of 4 floats in k_range_dkdv_reduce
+static constexpr int64_t kReduceFew = 1ll << 16;  // runs below which a thread each leaves most of the chip idle
 static constexpr int kCmpChunk = 2048;   // queries per compression dK/dV work item
 static constexpr int kCmpSplit = 4;      // sub-chunks of the chunks that end a grid of several rounds
 
@@ -1784,11 +1806,21 @@ int nsa_range_dkdv_as(int mode, const void* q, const void* k, const void* v, con
     }
     if (partial) {
       if (hipGetLastError() != hipSuccess) return NSA_ERR_LAUNCH;
-      const unsigned rg = (unsigned)(((int64_t)r.nbh * Lk * (DD / 4) + 255) / 256);
-      if (out_dtype == NSA_F32)
-        k_range_dkdv_reduce<DD, NW, float><<<rg, 256, 0, s>>>(r, part, part_half, dk32, dv32);
-      else
-        k_range_dkdv_reduce<DD, NW, bf16><<<rg, 256, 0, s>>>(r, part, part_half, dk16, dv16);
+      const int64_t nf = (int64_t)r.nbh * Lk * (DD / 4);
+      auto reduce = [&](auto rgc, auto* o, auto* ov) {
+        constexpr int RG = decltype(rgc)::value;
+        k_range_dkdv_reduce<DD, NW, RG><<<(unsigned)((nf * RG + 255) / 256), 256, 0, s>>>(r, part, part_half, o, ov);
+      };
+      // few runs, each of eight parts or more (past 65536 runs the loads in flight
+      // are enough: T4096 B8 Hkv2 D64 7.5 us at one thread a run)
+      const bool few = nf < kReduceFew && r.spl >= kReduceGroups;
+      using One = std::integral_constant<int, 1>;
+      using Many = std::integral_constant<int, kReduceGroups>;
+      if (out_dtype == NSA_F32) {
+        if (few) reduce(Many{}, dk32, dv32); else reduce(One{}, dk32, dv32);
+      } else {
+        if (few) reduce(Many{}, dk16, dv16); else reduce(One{}, dk16, dv16);
+      }
     }
   });
   return nsa_launch_status();
