@@ -19,7 +19,7 @@
 // Tiles whose two queries see all 32 keys of a wave skip the per-element mask.
 //
 //   * window      : a workgroup owns 32*NW keys and walks queries [k0, k0 + 32 NW + w - 2], or a
-//                   part of them where the key blocks alone leave CUs idle (win_split).
+//                   part of them where the key blocks alone leave CUs idle (win_grid).
 //   * compression : same, over query chunks of kCmpChunk; the key blocks of one chunk share an XCD.
 //   Parts and chunks write partial rows that k_range_dkdv_reduce sums (or, without a
 //   partial buffer, the chunks merge with float atomics and the window is not split).
@@ -951,7 +951,7 @@ __device__ __forceinline__ void zero_rows(float* dkrow, float* dvrow, int h) {
 
 // ---------------------------------------------------------------------------
 // Work of a range dK/dV launch.  Window: ceil(Lk / (32 NW)) key blocks per bh,
-// the queries of each in `spl` equal parts (win_split).  Compression: every
+// the queries of each in `spl` equal parts (win_grid).  Compression: every
 // (query chunk, key block) pair takes about as long as any other, so a grid
 // of them would end in a partial round of workgroups on an otherwise idle GPU.
 // Chunks from `chs` on are split into `spl` sub-chunks and launched last,
