@@ -1013,9 +1013,8 @@ template <int NW> __device__ __forceinline__ KvWork kv_work(const KvRange& r) {
     x.k0 = (int)(kb % nkb) * 32 * NW;
     x.bh = (int)(kb / nkb);
     const int klast = x.k0 + 32 * NW - 1 < r.Lk - 1 ? x.k0 + 32 * NW - 1 : r.Lk - 1;
-    const int win = r.window < r.T_ ? r.window : r.T_;   // a longer window sees no more
-    const int last = klast + win - 1;
-    const int len = (32 * NW + win - 1 + r.spl - 1) / r.spl;
+    const int last = klast + r.window - 1;
+    const int len = (32 * NW + r.window - 1 + r.spl - 1) / r.spl;
     x.tlo = x.k0 + sub * len;
     x.thi = r.spl > 1 && x.tlo + len - 1 < last ? x.tlo + len - 1 : last;
   }
@@ -1663,6 +1662,21 @@ static int device_cu_count(hipStream_t s) {
 constexpr int kRangeNW = 2;        // key groups of 32 per range dK/dV workgroup
 constexpr int kMinPartQueries = 32;   // fewest queries of a window part or compression sub-chunk
 
+// A launch's KvRange.  A window of T or more sees every earlier key, a span
+// past T none, and from a stride of T on only key 0 is seen at all: the masks,
+// the grid and the partial sizes take them cut off there, where no product of
+// theirs leaves 32 bits.
+static KvRange kv_range(int mode, int T, int Lk, int window, int cl, int cd, int nbh) {
+  KvRange r{mode, T, Lk, T, 0, 1, 1, nbh, 0, 1};
+  if (mode == NSA_MODE_WINDOW) {
+    r.window = window < T ? window : T;
+  } else {
+    r.cl = cl <= T ? cl : T + 1;
+    r.cd = cd < T ? cd : T;
+  }
+  return r;
+}
+
 // Compression dK/dV grid: logical workgroups over (key block, query chunk),
 // the chunks from r.chs on in r.spl sub-chunks while their workgroups fit in
 // one round of the resident workgroups (two per CU of the stream's device).
@@ -1705,7 +1719,7 @@ static int64_t win_grid(KvRange& r, bool split, hipStream_t s) {
   r.spl = 1;
   if (split && g > 0) {
     int64_t most = 2 * (int64_t)device_cu_count(s) / g;
-    const int64_t room = (32 * kRangeNW + (int64_t)(r.window < r.T_ ? r.window : r.T_) - 1) / kMinPartQueries;
+    const int64_t room = (32 * kRangeNW + (int64_t)r.window - 1) / kMinPartQueries;
     if (most > room) most = room;
     if (most > 1) r.spl = (int)most;
   }
@@ -1723,7 +1737,7 @@ size_t nsa_range_dkdv_partial_bytes(int mode, int B, int Hkv, int T, int Lk, int
   if ((mode != NSA_MODE_COMPRESS && mode != NSA_MODE_WINDOW) || B <= 0 || Hkv <= 0 || T <= 0 || Lk <= 0 || D <= 0 ||
       cmp_block < 1 || cmp_stride < 1)
     return 0;
-  KvRange r{mode, T, Lk, 0, cmp_block, cmp_block, cmp_stride, B * Hkv, 0, 1};
+  KvRange r = kv_range(mode, T, Lk, cmp_block, cmp_block, cmp_stride, B * Hkv);
   if (mode == NSA_MODE_COMPRESS) return range_part_bytes(cmp_grid(r, (hipStream_t)stream), D);
   const int64_t grid = win_grid(r, true, (hipStream_t)stream);
   return r.spl > 1 ? range_part_bytes(grid, D) : 0;
@@ -1761,7 +1775,7 @@ int nsa_range_dkdv_as(int mode, const void* q, const void* k, const void* v, con
   // dK/dV from 2.03 / 3.89 ms to 1.72 / 3.18 ms, and unrolled over its
   // stages to 1.61 / 3.03 ms.
   constexpr int NW = kRangeNW;
-  KvRange r{mode, T, Lk, T, window, cmp_block, cmp_stride, B * Hkv, 0, 1};
+  KvRange r = kv_range(mode, T, Lk, window, cmp_block, cmp_stride, B * Hkv);
   int64_t grid = 0;
   if (T > 0 && Lk > 0) {
     if (mode == NSA_MODE_COMPRESS) {

@@ -267,10 +267,16 @@ static_assert(pair_rows(5, -1, 256).t0 == 5 && pair_rows(5, -1, 256).dB == 0, "n
 //   window (window > 0): key <= t < key + window  <=>  key G <= R < (key + window) G
 //   compression (window = 0): t >= key cd + cl - 1  <=>  R >= (key cd + cl - 1) G
 // (t = floor(R / G) >= m  <=>  R >= m G, and t < m  <=>  R < m G).
-// Returns bit r set for the tile rows r that see the key.
+// Returns bit r set for the tile rows r that see the key.  The products are 64
+// bits wide (a window of 2^31 / G no longer fits 32) and cut off past every
+// row: a launch has fewer than 2^27 of them.
+constexpr int kPastRows = 1 << 30;
+__host__ __device__ constexpr int flat_row_bound(int64_t t, int G) {
+  return t * G < kPastRows ? (int)(t * G) : kPastRows;
+}
 __host__ __device__ constexpr uint32_t flat_rows_seeing(int key, int R0, int G, int window, int cl, int cd) {
-  int lo = window > 0 ? key * G - R0 : (key * cd + cl - 1) * G - R0;
-  int hi = window > 0 ? (key + window) * G - R0 : 32;
+  int lo = flat_row_bound(window > 0 ? key : (int64_t)key * cd + cl - 1, G) - R0;
+  int hi = window > 0 ? flat_row_bound((int64_t)key + window, G) - R0 : 32;
   lo = lo < 0 ? 0 : (lo > 32 ? 32 : lo);
   hi = hi < 0 ? 0 : (hi > 32 ? 32 : hi);
   return lo < hi ? (uint32_t)(((1ull << hi) - 1ull) & ~((1ull << lo) - 1ull)) : 0u;
@@ -283,13 +289,20 @@ __host__ __device__ constexpr bool flat_tile_needs_mask(int kw, int R0, int rhi,
   const int tf = R0 / G;                                 // the tile's first query
   const int tl = (R0 + 31 < rhi ? R0 + 31 : rhi) / G;    // and its last present one
   const int wlast = kw + 31;
-  return window > 0 ? !(tf >= wlast && tl - window < kw) : !(wlast * cd + cl - 1 <= tf);
+  return window > 0 ? !(tf >= wlast && tl - window < kw) : !((int64_t)wlast * cd + cl - 1 <= tf);
 }
 static_assert(flat_rows_seeing(5, 0, 6, 512, 0, 0) == ~((1u << 30) - 1u), "window: rows of queries >= 5");
 static_assert(flat_rows_seeing(0, 0, 6, 3, 0, 0) == (1u << 18) - 1u, "window of 3: queries 0 .. 2");
 static_assert(flat_rows_seeing(1, 270, 6, 0, 32, 16) == ~((1u << 12) - 1u),
               "compression, l 32 / d 16: key 1 seen by queries >= 47, rows >= 282");
 static_assert(flat_rows_seeing(1, 60, 6, 0, 32, 16) == 0u, "compression: no row of queries 10 .. 15 sees key 1");
+static_assert(flat_rows_seeing(5, 0, 4, 1 << 29, 0, 0) == flat_rows_seeing(5, 0, 4, 64, 0, 0) &&
+                  flat_rows_seeing(5, 0, 15, 0x7fffffff, 0, 0) == 0u &&
+                  flat_rows_seeing(5, 64, 15, 0x7fffffff, 0, 0) == ~((1u << 11) - 1u),
+              "a window past the last query ends at no row");
+static_assert(flat_rows_seeing(63, 0, 15, 0, 0x7fffffff, 0x7fffffff) == 0u &&
+                  flat_tile_needs_mask(32, 0, 31, 15, 0, 0x7fffffff, 0x7fffffff),
+              "a span past the last query is seen by none");
 
 // Direct global -> LDS loads as volatile asm (lane i writes lds + SIZE i):
 // the compiler neither tracks them nor adds waits for them, so LDS reads of

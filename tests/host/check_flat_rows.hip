@@ -8,13 +8,14 @@
 
 #include "nsa_tile32.h"
 
-static bool sees(int key, int t, int window, int cl, int cd) {
+static bool sees(int64_t key, int t, int64_t window, int64_t cl, int64_t cd) {
   return window > 0 ? (key <= t && t < key + window) : (key * cd + cl - 1 <= t);
 }
 
 int main() {
-  const int windows[] = {0, 1, 3, 32, 512};
-  const int geo[][2] = {{32, 16}, {16, 16}, {48, 32}, {1, 1}};
+  // the last of each: bounds whose product with G does not fit 32 bits
+  const int windows[] = {0, 1, 3, 32, 512, 1 << 27, 1 << 29, 0x7fffffff};
+  const int geo[][2] = {{32, 16}, {16, 16}, {48, 32}, {1, 1}, {1 << 29, 1 << 29}, {1, 0x7fffffff}};
   long cases = 0, bad_bits = 0, bad_mask = 0, skipped_tiles = 0;
   for (int G = 1; G < 16; ++G)
     for (int window : windows)
