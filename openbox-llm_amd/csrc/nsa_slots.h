@@ -122,9 +122,11 @@ __device__ __forceinline__ void merge_slots(const P* __restrict__ opart, const f
     bool all = true;
 #pragma unroll
     for (int u = 0; u < SL::SPL; ++u) {
-      w[u] = fast_exp2(w[u] - bm);   // 0 where the slot does not count
+      // a weight that underflows to 0 still counts (0 times an infinite or NaN
+      // partial is NaN); negative: the slot does not, its l is 0
+      w[u] = p[u].y > 0.0f ? fast_exp2(w[u] - bm) : -1.0f;
       ls += w[u] * p[u].y;
-      all &= w[u] > 0.0f;
+      all &= p[u].y > 0.0f;
     }
     const float rs = M == -__builtin_inff() ? 0.0f : fast_exp2(M - bm);
     Ls = Ls * rs + SL::reduce(ls, [](float a, float b) { return a + b; });
@@ -137,7 +139,7 @@ __device__ __forceinline__ void merge_slots(const P* __restrict__ opart, const f
         load(k0);
       }
       if (!__all(all)) {
-        static_for<0, XB>([&](auto k) { x[k.value].keep_if(SL::template of<k0 + k.value>(w) > 0.0f); });
+        static_for<0, XB>([&](auto k) { x[k.value].keep_if(!(SL::template of<k0 + k.value>(w) < 0.0f)); });
       }
       static_for<0, XB>([&](auto k) {
         const float wk = SL::template of<k0 + k.value>(w);

@@ -43,3 +43,31 @@ def test_merge_and_dq_sum(S, bs, D, dtype):
     # float32 sums of S terms of size ~1, rounded to the dtype once
     eps = S * npass * 2.0 ** -23 + (2.0 ** -8 if dtype == BF else 0.0)
     assert float((got.double() - want).abs().max()) <= eps * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [F32, BF], ids=["f32", "bf16"])
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+def test_infinite_value_of_a_slot_without_weight(D, dtype):
+    """A selected block whose weight underflows to 0 beside the row's maximum
+    still passes an infinite or NaN value on (0 x inf is NaN, as in torch):
+    in the merge of its own and in the layer's window forward."""
+    import nsa_fused_kernel as nfk
+    import nsa_selection_backward as nsb
+    dev = require_gpu()
+    T, Hq, bs = 256, 4, 64
+    q, k = torch.ones(1, Hq, T, D), torch.zeros(1, 1, T, D)
+    k[:, :, :bs] = 400.0 / D ** 0.5      # scores of 400 in block 0, 0 elsewhere: exp(-400) is 0
+    v = randn((1, 1, T, D), 1, F32)
+    idx = torch.arange(T // bs).expand(1, 1, T, T // bs).clone().to(torch.int32)
+    idx[idx * bs > torch.arange(T)[:, None]] = -1
+    others = [randn((1, 1, T, D), 2 + i, F32) for i in range(4)]
+    gate = torch.zeros(1, Hq, T, 3)
+    for bad in (float("inf"), float("nan")):
+        vb = v.clone()
+        vb[:, :, 130] = bad              # block 2: the queries from 130 on see it
+        qd, kd, vd, *od, gd = (x.to(dev, dtype) for x in (q, k, vb, *others, gate))
+        o = nsb.selection_attn_triton(qd, kd, vd, idx.to(dev), bs)
+        layer = nfk.nsa_fused_forward(qd, od[0], od[1], kd, vd, od[2], od[3], gd, idx.to(dev), bs, 32)
+        for x, what in ((o, "selection"), (layer, "layer")):
+            assert x[:, :, :128].isfinite().all(), f"{what}: {bad} reached a query that has not selected it"
+            assert not x[:, :, 130:].isfinite().any(), f"{what}: {bad} lost"
