@@ -1801,8 +1801,15 @@ int nsa_range_dkdv_as(int mode, const void* q, const void* k, const void* v, con
   const float sl2 = scale * kLog2e;
   float* part = partial ? dkdv_part : nullptr;
   const int64_t part_half = grid * 32 * NW * D;
-  // groups of G < 16 heads: query tiles of 32 consecutive (query, head) rows
-  const bool flat = Hq / Hkv < 16;
+  // groups of G < 16 heads: query tiles of 32 consecutive (query, head) rows,
+  // G / 16 of the tiles of two queries.  A flat float tile at D = 128 costs
+  // twice the other (608 registers spilled against 388), so there the line lies
+  // at 8 heads: dK/dV, us, flat / pairs, window + compression at T8192 Hkv2: G 4
+  // 5384 / 9975, G 8 10659 / 10483, G 9 12045 / 10592, G 12 16006 / 10887, G 15
+  // 19998 / 11261; T512: G 8 569 / 614, G 12 820 / 637.  At D <= 64 flat takes
+  // 0.77 (G 12) to 0.97 (G 15) of the pairs' time.
+  const int flat_heads = dtype == NSA_F32 && D == 128 ? 8 : 15;
+  const bool flat = Hq / Hkv <= flat_heads;
   float* dk32 = out_dtype == NSA_F32 ? (float*)dk : nullptr;
   float* dv32 = out_dtype == NSA_F32 ? (float*)dv : nullptr;
   bf16* dk16 = out_dtype == NSA_F32 ? nullptr : (bf16*)dk;

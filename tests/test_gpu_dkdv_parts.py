@@ -5,7 +5,7 @@ the launch that takes each key block whole.
 Sizes put the parts' edges inside and past the key blocks' query ranges:
 windows of 3 (of 1, dK is 0) and past the sequence's end, lengths of one key block and one
 more, the last block nearly empty; groups with flat rows (G < 16, float32 and
-bf16) and with head chunks (G = 16, 20)."""
+bf16; up to G = 8 in float32 at D = 128) and with head chunks."""
 
 import pytest
 import torch
@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 
 # T, window, span l, stride d
 SIZES = [(64, 3, 16, 16), (65, 40, 16, 8), (257, 700, 32, 16), (1000, 100, 64, 64), (1301, 512, 32, 16)]
-HEADS = [(4, 1, 64), (12, 2, 32), (16, 1, 128), (20, 1, 64)]
+HEADS = [(4, 1, 64), (12, 2, 32), (16, 1, 128), (20, 1, 64), (8, 1, 128), (9, 1, 128), (15, 1, 128), (15, 1, 64)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
