@@ -148,3 +148,25 @@ def test_f16s_buffers_carry_their_row_scales():
     assert ops.kept_output((2, 3, 5, 64), torch.empty(0, dtype=torch.float32)).dtype == torch.float32
     with pytest.raises(AssertionError):
         mod.dtype_code(torch.empty(2, 3, 5, 64, dtype=torch.float16))
+
+
+@pytest.mark.parametrize("pooled", [0, 1])
+@pytest.mark.parametrize("dims", [(1, 16, 4, 4096, 128), (8, 8, 2, 256, 64), (1, 64, 4, 32768, 128)], ids=str)
+def test_backward_scratch_holds_one_branch_at_a_time(dims, pooled):
+    """The layer's backward scratch: what the last launches read, and the
+    largest branch's dK/dV buffers (the branches run one after the other)."""
+    mod, lib = _lib()
+    B, Hq, Hkv, T, D = dims
+    l, d, ls, S, w, es = 32, 16, 64, min(16, T // 64), 512, 2
+    n, rows = (T - l) // d + 1, B * Hq * T
+    kt = [B * Hkv * D * lib.nsa_padded_len(x) * es for x in (T, n)]
+    last = 9 * rows * 4 + rows * lib.nsa_sel_partial_slots(S, ls) * D * es + sum(kt)
+    last += 0 if pooled else 2 * B * Hkv * n * D * 4
+    chunk = lib.nsa_sel_dkdv_chunk(B, Hkv, T, S, ls)
+    sel = (rows * D * es + kt[0] + lib.nsa_sel_dkdv_workspace(B, Hkv, T, S, ls, chunk) +
+           lib.nsa_sel_dkdv_partial_bytes(B, Hkv, T, S, D, ls, chunk))
+    win = lib.nsa_range_dkdv_partial_bytes(0, B, Hkv, T, T, D, w, 1, None)
+    cmp = lib.nsa_range_dkdv_partial_bytes(1, B, Hkv, T, n, D, l, d, None)
+    got = lib.nsa_fused_bwd_scratch_bytes(B, Hq, Hkv, T, D, l, d, ls, 16, w, pooled, mod.NSA_BF16, None)
+    need = last + max(sel, win, cmp)
+    assert need <= got <= need + 16 * 256      # each buffer starts on 256 bytes
