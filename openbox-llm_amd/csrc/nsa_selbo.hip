@@ -471,11 +471,13 @@ static inline int grid_for(int64_t n) {
 
 // o[row] = sum_slots exp2(m - M) O_slot / sum exp2(m - M) l over the valid
 // slots, lse = (M + log2 L) ln 2, with a running maximum M across batches.
+// bf16: three waves per SIMD; held to three, D = 16 spilled 7 registers and took
+// 36.2 us at T8192 Hq16 B2, 33.4 at two (D = 32, 2 spilled: 54.5 and 56.2).
 template <typename T, int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 ? 3 : 2))) void k_sel_merge(const int32_t* __restrict__ idx, const PartT<T>* __restrict__ opart,
-                                                   const float2* __restrict__ mlpart, T* __restrict__ o,
-                                                   float* __restrict__ lse, int Hq, int Hkv, int T_, int S, int n_csr,
-                                                   int L, int nsub, int64_t total, float* __restrict__ o32) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 && D >= 32 ? 3 : 2)))
+void k_sel_merge(const int32_t* __restrict__ idx, const PartT<T>* __restrict__ opart,
+                 const float2* __restrict__ mlpart, T* __restrict__ o, float* __restrict__ lse, int Hq, int Hkv,
+                 int T_, int S, int n_csr, int L, int nsub, int64_t total, float* __restrict__ o32) {
   constexpr int NC = D / 8;
   const int G = Hq / Hkv;
   for (int64_t e = blockIdx.x * 256ll + threadIdx.x; e < total; e += (int64_t)gridDim.x * 256) {

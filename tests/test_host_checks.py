@@ -97,6 +97,27 @@ def test_m0_is_written_only_by_the_dma_helpers():
     assert checked > 0
 
 
+# kernel (mangled: f is float, DF16b bf16, Li64 D = 64) and the most registers a lane of it may spill
+SPILLS = [(r"k_sel_merge", 2), (r"k_sel_dq_reduce", 0)]
+
+
+def test_spilled_registers():
+    """The kernels that sum a row's selection slots beside its accumulators
+    keep them in registers (metadata of the device assembly)."""
+    if shutil.which("make") is None:
+        pytest.skip("needs make")
+    subprocess.run(["make", "-s", "-j8", "-C", PKG, "asm"], check=True, capture_output=True)
+    spilled = {}
+    for name in ("nsa_range.s", "nsa_selbo.s"):
+        text = open(os.path.join(PKG, "_build", name)).read()
+        entry = r"^\s*\.name:\s+(_Z\w+)\n(?:(?!\s*\.name:).*\n)*?\s*\.vgpr_spill_count:\s*(\d+)"
+        spilled.update(re.findall(entry, text, flags=re.M))
+    for pattern, most in SPILLS:
+        found = {k: int(v) for k, v in spilled.items() if re.search(pattern, k)}
+        assert found, f"no kernel {pattern}"
+        assert max(found.values()) <= most, f"{pattern}: {found}"
+
+
 def test_flat_row_visibility(tmp_path):
     """The range dK/dV's flat-row masks (groups of G < 16 heads, row R =
     query R / G) against brute force over every row of a tile, window and
