@@ -301,7 +301,7 @@ __device__ __forceinline__ void finish_rows(const FwdExtras<T, TO>& f, const f32
     }
     // selection: merge the slot partials
     float acc_s[8], M, Ls;
-    merge_slots<PartT<T>, D>(f.opart, f.ml, f.idx, bh * T_ + t, t, gl, G, f.S, nsub, n_csr, f.sel_L, c8, acc_s, M, Ls);
+    merge_slots<PartT<T>, D, true>(f.opart, f.ml, f.idx, bh * T_ + t, t, gl, G, f.S, nsub, n_csr, f.sel_L, c8, acc_s, M, Ls);
     const float inv_s = Ls > 0.0f ? 1.0f / Ls : 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc_s[i] *= inv_s;
@@ -849,7 +849,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] += u[i];
       }
-      add_slots<T, D>(sel_part, sel_idx, (int64_t)bh * T_ + t, t, gl, G, S, nsub, n_csr, sel_L, c8, lane, v);
+      add_slots<T, D, true>(sel_part, sel_idx, (int64_t)bh * T_ + t, t, gl, G, S, nsub, n_csr, sel_L, c8, lane, v);
       if (dq_out32 != nullptr)
         store8(dq_out32 + orow * D + 8 * c8, v);
       else

@@ -488,7 +488,7 @@ void k_sel_merge(const int32_t* __restrict__ idx, const PartT<T>* __restrict__ o
     const int t = (int)(r % T_);
     const int64_t bh = r / T_;
     float acc[8], M, Ls;
-    merge_slots<PartT<T>, D>(opart, mlpart, idx, bh * T_ + t, t, g, G, S, nsub, n_csr, L, c, acc, M, Ls);
+    merge_slots<PartT<T>, D, false>(opart, mlpart, idx, bh * T_ + t, t, g, G, S, nsub, n_csr, L, c, acc, M, Ls);
     const int64_t orow = (((bh / Hkv) * Hq + (bh % Hkv) * G + g) * T_ + t);
     const float inv = Ls > 0.0f ? 1.0f / Ls : 0.0f;
 #pragma unroll
@@ -523,7 +523,7 @@ __global__ __launch_bounds__(256) void k_sel_dq_reduce(const int32_t* __restrict
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
     }
-    add_slots<T, D>(dqpart, idx, bh * T_ + t, t, g, G, S, nsub, n_csr, L, c, threadIdx.x & 63, acc);
+    add_slots<T, D, false>(dqpart, idx, bh * T_ + t, t, g, G, S, nsub, n_csr, L, c, threadIdx.x & 63, acc);
     store8(dq_out + orow * D + 8 * c, acc);
   }
 }

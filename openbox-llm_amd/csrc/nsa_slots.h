@@ -66,16 +66,19 @@ __device__ __forceinline__ LaneAddr lane_addr(const void* p) {
   return r;
 }
 
-// slots whose row pieces are in flight together: a float piece is two loads,
-// and 16 of them (128 registers) made the float32 dQ spill
-template <typename P> constexpr int slot_loads() { return sizeof(P) == 4 ? 8 : 16; }
+// Slots whose row pieces are in flight together: a float piece is two loads and
+// eight registers.  TIGHT: in a range kernel, beside the row's accumulators and
+// operands; with eight pieces the float32 forward spilled 15 to 64 registers
+// and finishing a D = 64 window (T8192 Hq4 B2) took 161 us, with four it takes
+// 147.
+template <typename P> constexpr int slot_loads(bool tight) { return sizeof(P) == 4 ? (tight ? 4 : 8) : 16; }
 
 // Merge of the selection partials of one row (query t of pair row qs = (b Hkv
 // + hkv) T + t, head gl of the group): this lane's 8 elements (chunk c8) of
 // acc / Ls are o, M + log2(Ls) the row's log-sum-exp in log2 units.  Slots
 // that do not count were maybe never written: nothing of them is used.  A
 // running maximum over batches of 16 slots.  Whole rows of lanes call this.
-template <typename P, int D>
+template <typename P, int D, bool TIGHT>
 __device__ __forceinline__ void merge_slots(const P* __restrict__ opart, const float2* __restrict__ ml,
                                             const int32_t* __restrict__ idx, int64_t qs, int t, int gl, int G, int S,
                                             int nsub, int n_csr, int L, int c8, float (&acc)[8], float& M,
@@ -98,7 +101,7 @@ __device__ __forceinline__ void merge_slots(const P* __restrict__ opart, const f
       j[u] = irow[sl / nsub];
       p[u] = ml[(qs * NS + sl) * G + gl];
     }
-    constexpr int XB = slot_loads<P>();
+    constexpr int XB = slot_loads<P>(TIGHT);
     Raw8<P> x[XB];
     auto load = [&](int k0) {
 #pragma unroll
@@ -153,7 +156,7 @@ __device__ __forceinline__ void merge_slots(const P* __restrict__ opart, const f
 
 // v += the dQ partials of the row's valid slots, in slot order (arguments as
 // merge_slots).
-template <typename T, int D>
+template <typename T, int D, bool TIGHT>
 __device__ __forceinline__ void add_slots(const T* __restrict__ part, const int32_t* __restrict__ idx, int64_t qs,
                                           int t, int gl, int G, int S, int nsub, int n_csr, int L, int c8, int lane,
                                           float (&v)[8]) {
@@ -169,7 +172,7 @@ __device__ __forceinline__ void add_slots(const T* __restrict__ part, const int3
       const int sl = s0 + c8 + SL::CPR * u < NS ? s0 + c8 + SL::CPR * u : NS - 1;
       j[u] = irow[sl / nsub];
     }
-    constexpr int XB = slot_loads<T>();
+    constexpr int XB = slot_loads<T>(TIGHT);
     Raw8<T> x[XB];
     auto load = [&](int k0) {
 #pragma unroll

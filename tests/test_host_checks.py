@@ -98,7 +98,8 @@ def test_m0_is_written_only_by_the_dma_helpers():
 
 
 # kernel (mangled: f is float, DF16b bf16, Li64 D = 64) and the most registers a lane of it may spill
-SPILLS = [(r"k_sel_merge", 2), (r"k_sel_dq_reduce", 0)]
+SPILLS = [(r"k_range_fwd32I(DF16b|fLi16E|fLi128E)", 0), (r"k_range_fwd32IfLi32E", 8), (r"k_range_fwd32IfLi64E", 24),
+          (r"k_range_dq32I", 4), (r"k_sel_merge", 2), (r"k_sel_dq_reduce", 0)]
 
 
 def test_spilled_registers():
