@@ -155,7 +155,10 @@ __device__ __forceinline__ void merge_slots(const P* __restrict__ opart, const f
 }
 
 // v += the dQ partials of the row's valid slots, in slot order (arguments as
-// merge_slots).
+// merge_slots).  The partials are read once, past the caches, but for float
+// pieces in a launch of their own: their two loads share each line (T8192 Hq16
+// D64, us, cached / past the caches: B1 128 MiB 23.5 / 28.5, B4 2 GiB 403 / 451;
+// bf16 B4 1 GiB 219 / 191).
 template <typename T, int D, bool TIGHT>
 __device__ __forceinline__ void add_slots(const T* __restrict__ part, const int32_t* __restrict__ idx, int64_t qs,
                                           int t, int gl, int G, int S, int nsub, int n_csr, int L, int c8, int lane,
@@ -178,7 +181,11 @@ __device__ __forceinline__ void add_slots(const T* __restrict__ part, const int3
 #pragma unroll
       for (int k = 0; k < XB; ++k) {
         const int sl = s0 + k0 + k < NS ? s0 + k0 + k : NS - 1;
-        x[k].load_nt(reinterpret_cast<const T*>((const char*)(uintptr_t)(pa.base + (uint64_t)sl * pitch) + pa.off));
+        const T* src = reinterpret_cast<const T*>((const char*)(uintptr_t)(pa.base + (uint64_t)sl * pitch) + pa.off);
+        if constexpr (sizeof(T) == 2 || TIGHT)
+          x[k].load_nt(src);
+        else
+          x[k].load(src);
       }
     };
     load(0);
