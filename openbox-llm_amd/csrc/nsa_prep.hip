@@ -111,10 +111,42 @@ __global__ __launch_bounds__(256) void k_pool_fwd(const T* __restrict__ x, T* __
   }
 }
 
+// The rows of a span in ascending order, add(w[k], row) (unweighted: 1): batches
+// of up to 16 rows whose loads are all in flight.  Left to itself the compiler
+// moves loads to their sums (a weighted bf16 span then took up to four times as
+// long), so none of a long batch may pass the barrier.  bf16, us, before the
+// batches / with the last batch's loads clamped to the span / now: T1024 Hkv4
+// D128 spans of 32 3.5 / 4.5 / 3.8, of 128 7.4 / 11.9 / 7.5; B16 T8192 Hkv8 D128
+// spans of 32 77 / 72 / 70.
+template <bool WEIGHTED, typename T, typename Add>
+__device__ __forceinline__ void span_rows(const T* src, const float* w, int pl, int D, Add add) {
+  int k = 0;
+  auto batch = [&](auto count) {
+    constexpr int N = decltype(count)::value;
+    Frag<T> f[N];
+    float wk[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      f[u].load(src + (int64_t)u * D);
+      wk[u] = WEIGHTED ? w[k + u] : 1.0f;
+    }
+    if constexpr (N >= 8) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < N; ++u) add(wk[u], f[u]);
+    src += (int64_t)N * D;
+    k += N;
+  };
+  while (k + 16 <= pl) batch(std::integral_constant<int, 16>{});
+  if (pl - k >= 8) batch(std::integral_constant<int, 8>{});
+  if (pl - k >= 4) batch(std::integral_constant<int, 4>{});
+  if (pl - k >= 2) batch(std::integral_constant<int, 2>{});
+  if (pl - k >= 1) batch(std::integral_constant<int, 1>{});
+}
+
 // D % 8 == 0, 16-byte aligned rows: a lane sums 8 consecutive d (same order of
 // additions as k_pool_fwd).  Few lanes sum a short sequence: the rows' latency
-// is what it waits for, so 16 are in flight.  blockIdx.y = 1: a second tensor
-// of the same shape (keys and values in one launch).
+// is what it waits for.  blockIdx.y = 1: a second tensor of the same shape (keys
+// and values in one launch).
 template <typename T>
 __global__ __launch_bounds__(256) void k_pool_fwd8(const T* __restrict__ x0, T* __restrict__ out0,
                                                    const T* __restrict__ x1, T* __restrict__ out1, int BH, int L,
@@ -133,17 +165,10 @@ __global__ __launch_bounds__(256) void k_pool_fwd8(const T* __restrict__ x0, T* 
     float s[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) s[j] = 0.0f;
-    for (int k0 = 0; k0 < pl; k0 += 16) {
-      Frag<T> f[16];   // (left to itself the compiler waits for each row)
+    span_rows<false>(src, nullptr, pl, D, [&](float, const Frag<T>& f) {
 #pragma unroll
-      for (int u = 0; u < 16; ++u) f[u].load(src + (int64_t)(k0 + u < pl ? k0 + u : pl - 1) * D);
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (k0 + u < pl) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) s[j] += to_f32(f[u].elem(j));
-        }
-    }
+      for (int j = 0; j < 8; ++j) s[j] += to_f32(f.elem(j));
+    });
 #pragma unroll
     for (int j = 0; j < 8; ++j) s[j] *= inv;
     Frag<T> o;
@@ -232,18 +257,10 @@ __global__ __launch_bounds__(256) void k_wpool_fwd8(const T* __restrict__ x, con
     float s[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) s[j] = 0.0f;
-    for (int k0 = 0; k0 < pl; k0 += 16) {
-      Frag<T> f[16];   // 16 rows in flight, as k_pool_fwd8
+    span_rows<true>(src, w, pl, D, [&](float wk, const Frag<T>& f) {
 #pragma unroll
-      for (int u = 0; u < 16; ++u) f[u].load(src + (int64_t)(k0 + u < pl ? k0 + u : pl - 1) * D);
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (k0 + u < pl) {
-          const float wk = w[k0 + u];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) s[j] += wk * to_f32(f[u].elem(j));
-        }
-    }
+      for (int j = 0; j < 8; ++j) s[j] += wk * to_f32(f.elem(j));
+    });
 #pragma unroll
     for (int j = 0; j < 8; ++j) s[j] += cv[8 * c + j];
     float* o = out + r * D + 8 * c;

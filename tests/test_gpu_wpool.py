@@ -7,7 +7,7 @@ gradients of x, pool_logits, intra_pos and the projection weight."""
 import pytest
 import torch
 
-from nsa_testlib import assert_close, log, require_gpu
+from nsa_testlib import assert_close, log, randn, require_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +61,24 @@ def test_weighted_pool_matches_unfolded_module(geo, dtype):
         g = dict(mod.named_parameters())[name].grad.cpu()
         r = dict(ref_mod.named_parameters())[name].grad
         assert_close(g, r, torch.float32, f"d{name}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("l", [1, 2, 3, 7, 8, 15, 16, 17, 31, 47, 64])
+def test_span_lengths(l, dtype):
+    """Mean and weighted pooling of spans that fill the batches of 16, 8, 4, 2
+    and 1 rows and leave every remainder, against float64."""
+    import nsa_hip_ops as ops
+    dev = require_gpu()
+    x = randn((2, 3, 150, 32), l, dtype)
+    w = torch.softmax(randn((l,), 1, torch.float32), 0)
+    pos = randn((l, 32), 2, torch.float32)
+    spans = x.double().unfold(2, l, 5)                               # [B, H, n, D, l]
+    got = ops.pool_fwd(x.to(dev), l, 5)
+    ref = spans.mean(-1)
+    # l float32 additions of terms of size ~4, then one rounding to the dtype
+    eps = (l + 2) * 2.0 ** -24 * 4 + (2.0 ** -8 * 4 if dtype == torch.bfloat16 else 0.0)
+    assert got.shape == ref.shape and float((got.double().cpu() - ref).abs().max()) <= eps
+    got = ops.weighted_pool(x.to(dev), w.to(dev), pos.to(dev), l, 5)
+    ref = spans @ w.double() + w.double() @ pos.double()
+    assert float((got.double().cpu() - ref).abs().max()) <= (2 * l + 4) * 2.0 ** -24 * 4
