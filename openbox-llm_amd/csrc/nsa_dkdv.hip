@@ -27,7 +27,6 @@
 //   waves per 32 keys, two waves per SIMD; below).
 //   * selection   : work items (block, chunk of its CSR query list) built by
 //                   k_sel_items; a persistent grid drains them; chunks merge with atomics.
-#include <atomic>
 #include <mutex>
 
 #include "nsa_launch.h"
@@ -1635,29 +1634,6 @@ static constexpr int kReduceGroups = 8;           // threads of a run of 4 float
 static constexpr int64_t kReduceFew = 1ll << 16;  // runs below which a thread each leaves most of the chip idle
 static constexpr int kCmpChunk = 2048;   // queries per compression dK/dV work item
 static constexpr int kCmpSplit = 4;      // sub-chunks of the chunks that end a grid of several rounds
-
-// Device of a stream (the null stream: the current device), or -1.
-static int stream_device(hipStream_t s) {
-  hipDevice_t dev = -1;
-  if (hipStreamGetDevice(s, &dev) != hipSuccess) return -1;
-  return (int)dev;
-}
-
-// Compute units of the stream's device, cached per device.  The cache is
-// written with relaxed atomics: two threads that race on a first lookup store
-// the same value.
-static int device_cu_count(hipStream_t s) {
-  static std::atomic<int> cache[64];
-  const int dev = stream_device(s);
-  if (dev < 0 || dev >= 64) return 256;
-  int n = cache[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cache[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
-
 
 constexpr int kRangeNW = 2;        // key groups of 32 per range dK/dV workgroup
 constexpr int kMinPartQueries = 32;   // fewest queries of a window part or compression sub-chunk

@@ -143,9 +143,14 @@ __host__ __device__ inline int sel_item_chunk(int64_t pairs, int64_t slots, int 
   while (c < hi && pairs / slots >= 2 * c) c *= 2;
   return c;
 }
-static inline int sel_fwd_chunk(int64_t pairs) { return sel_item_chunk(pairs, 1024, 16, 128); }   // one wave per SIMD
-static inline int sel_dkdv_chunk(int64_t pairs) {                                                // two workgroups per CU
-  return pairs >= 512 * 2048 ? 512 : sel_item_chunk(pairs, 512, 32, 256);
+// The slots are those of 256 compute units, whatever the device has: the chunk
+// sizes workspaces too, and their queries are not told a stream.
+static inline int sel_fwd_chunk(int64_t pairs) {
+  return sel_item_chunk(pairs, 4 * 256, 16, 128);   // one wave per SIMD
+}
+static inline int sel_dkdv_chunk(int64_t pairs) {
+  constexpr int64_t kSlots = 2 * 256;   // two workgroups per CU
+  return pairs >= 4 * 512 * kSlots ? 512 : sel_item_chunk(pairs, kSlots, 32, 256);
 }
 
 // Most CSR entries in one selection work item (the kernels stage an item's

@@ -908,7 +908,8 @@ extern "C" {
 // Key parts of a launch: g1 workgroups of four row groups, lds[i] bytes of LDS
 // for KP = 1, 2, 4 (0: not built), at most `tiles` key tiles a workgroup.  KP
 // parts make KP times the workgroups of 1 / KP the walk; with s of them
-// resident the launch takes ceil(g1 KP / s) / KP of a whole walk.  Parts are
+// resident (on the stream's cus compute units) the launch takes ceil(g1 KP / s)
+// / KP of a whole walk.  Parts are
 // taken where that is at most `worth` of one part's and every part has two
 // tiles or more.  Measured, us of window and compression together, one part
 // -> parts: float32 T1024 Hq4 D64 (32 workgroups a branch) forward 82 -> 40 (4
@@ -916,7 +917,7 @@ extern "C" {
 // workgroups, where two parts take 0.75 of the rounds: forward T1301 Hq64 D128
 // 160 -> 142, T6011 Hq16 D64 99 -> 98, but the latter's dQ 74 -> 77.  So the
 // forward takes parts at 0.8 and the dQ, whose parts also sum dQ, at 0.7.
-static int key_parts(int64_t g1, const int (&lds)[3], int tiles, double worth) {
+static int key_parts(int64_t g1, const int (&lds)[3], int tiles, double worth, int cus) {
   int best = 1;
   double cost = 0.0;
   for (int i = 0; i < 3; ++i) {
@@ -925,7 +926,7 @@ static int key_parts(int64_t g1, const int (&lds)[3], int tiles, double worth) {
     int per = 160 * 1024 / lds[i];   // workgroups per CU: by LDS, and two by registers
     per = per > 2 ? 2 : per;
     if (per < 1) continue;
-    const int64_t s = 256 * (int64_t)per;
+    const int64_t s = (int64_t)cus * per;
     const double c = (double)((g1 * kp + s - 1) / s) / kp;
     if (kp == 1 || c <= worth * cost) {
       best = kp;
@@ -951,7 +952,8 @@ static int range_fwd_launch(int mode, const void* q, const void* k, const void* 
     constexpr int l2 = range_fwd_lds<E, DD, 2>();
     constexpr int l4 = range_fwd_lds<E, DD, 4>() <= 160 * 1024 ? range_fwd_lds<E, DD, 4>() : 0;
     const int lds[3] = {l1, l2, l4};
-    const int kp = key_parts((int64_t)B * Hkv * NHC * range_qtiles(flat, T, Hq / Hkv, NT, 4), lds, tiles, 0.8);
+    const int kp = key_parts((int64_t)B * Hkv * NHC * range_qtiles(flat, T, Hq / Hkv, NT, 4), lds, tiles, 0.8,
+                             device_cu_count(s));
     const int nqt = range_qtiles(flat, T, Hq / Hkv, NT, 4 / kp);
     const int64_t grid = (int64_t)B * Hkv * NHC * nqt;
     NSA_CHECK(grid < (1ll << 31), NSA_ERR_SHAPE);
@@ -985,7 +987,8 @@ static int range_dq_launch(int mode, const void* q, const void* k, const void* v
     constexpr int l2 = range_dq_lds<E, DD, 2>() <= 160 * 1024 ? range_dq_lds<E, DD, 2>() : 0;
     constexpr int l4 = range_dq_lds<E, DD, 4>() <= 160 * 1024 ? range_dq_lds<E, DD, 4>() : 0;
     const int lds[3] = {l1, l2, l4};
-    const int kp = key_parts((int64_t)B * Hkv * NHC * range_qtiles(flat, T, Hq / Hkv, NT, 4), lds, tiles, 0.7);
+    const int kp = key_parts((int64_t)B * Hkv * NHC * range_qtiles(flat, T, Hq / Hkv, NT, 4), lds, tiles, 0.7,
+                             device_cu_count(s));
     const int nqt = range_qtiles(flat, T, Hq / Hkv, NT, 4 / kp);
     const int64_t grid = (int64_t)B * Hkv * NHC * nqt;
     NSA_CHECK(grid < (1ll << 31), NSA_ERR_SHAPE);
