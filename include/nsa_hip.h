@@ -283,7 +283,6 @@ int nsa_sel_merge_both(const int32_t* block_idx, const void* o_part, const float
                        float* lse, int B, int Hq, int Hkv, int T, int D, int S, int block_size, int dtype,
                        void* stream);
 
-
 /* dq_out = dq_acc (float32, nullable) + sum of the dQ partials of the valid
  * slots, written in the input dtype (the dQ reduce of
  * nsa_selection_backward.py:322-334).  dtype is the partials' and dq_out's
@@ -309,6 +308,12 @@ int nsa_sel_dq_reduce(const int32_t* block_idx, const void* dq_part, const float
 int nsa_range_fwd(int mode, const void* q, const void* k, const void* vt, void* o, float* lse, int B, int Hq,
                   int Hkv, int T, int Lk, int D, int window, int cmp_block, int cmp_stride, void* q_packed, int dtype,
                   int o_dtype, void* stream);
+/* Key parts that a range launch's row groups share their keys in (1, 2 or 4, for
+ * the stream's device; a negative status for arguments that the launch
+ * refuses): pass 0 forward, 1 dQ, 2 the dQ of both branches in one launch
+ * (nsa_range_dq_cw: mode NSA_MODE_COMPRESS and the window). */
+int nsa_range_key_parts(int pass, int mode, int B, int Hq, int Hkv, int T, int Lk, int D, int window, int dtype,
+                        void* stream);
 
 /* nsa_range_fwd that also finishes the rows of the gated three-branch layer
  * (no reference counterpart as one call: nsa_sel_merge and nsa_gate_fwd

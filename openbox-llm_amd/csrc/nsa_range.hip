@@ -935,6 +935,24 @@ static int key_parts(int64_t g1, const int (&lds)[3], int tiles, double worth, i
   }
   return best;
 }
+constexpr int fits_lds(int bytes) { return bytes <= 160 * 1024 ? bytes : 0; }
+// most key tiles of a workgroup
+static int range_tiles(int mode, int T, int Lk, int window) {
+  return mode == NSA_MODE_WINDOW ? ((window < T ? window : T) + 31) / 32 + 1 : (Lk + 31) / 32;
+}
+// workgroups of a launch of one part
+template <int NT> static int64_t range_grid1(int B, int Hq, int Hkv, int T) {
+  const int G = Hq / Hkv;
+  return (int64_t)B * Hkv * ((G + 15) / 16) * range_qtiles(G < 16, T, G, NT, 4);
+}
+template <typename E, int D> static int fwd_parts(int B, int Hq, int Hkv, int T, int tiles, hipStream_t s) {
+  constexpr int lds[3] = {range_fwd_lds<E, D, 1>(), range_fwd_lds<E, D, 2>(), fits_lds(range_fwd_lds<E, D, 4>())};
+  return key_parts(range_grid1<RangeNT<E>::fwd>(B, Hq, Hkv, T), lds, tiles, 0.8, device_cu_count(s));
+}
+template <typename E, int D> static int dq_parts(int B, int Hq, int Hkv, int T, int tiles, hipStream_t s) {
+  constexpr int lds[3] = {range_dq_lds<E, D, 1>(), fits_lds(range_dq_lds<E, D, 2>()), fits_lds(range_dq_lds<E, D, 4>())};
+  return key_parts(range_grid1<RangeNT<E>::dq>(B, Hq, Hkv, T), lds, tiles, 0.7, device_cu_count(s));
+}
 
 template <typename E, typename TO>
 static int range_fwd_launch(int mode, const void* q, const void* k, const void* vt, void* o, float* lse, int B,
@@ -946,20 +964,15 @@ static int range_fwd_launch(int mode, const void* q, const void* k, const void* 
   constexpr int NT = RangeNT<E>::fwd;
   const bool flat = Hq / Hkv < 16;   // flat rows: no empty head slots
   NSA_CHECK((int64_t)T * (Hq / Hkv) < (1ll << 31), NSA_ERR_SHAPE);
-  const int tiles = mode == NSA_MODE_WINDOW ? ((window < T ? window : T) + 31) / 32 + 1 : (Lk + 31) / 32;
+  const int tiles = range_tiles(mode, T, Lk, window);
   NSA_DISPATCH_D(D, {
-    constexpr int l1 = range_fwd_lds<E, DD, 1>();
-    constexpr int l2 = range_fwd_lds<E, DD, 2>();
-    constexpr int l4 = range_fwd_lds<E, DD, 4>() <= 160 * 1024 ? range_fwd_lds<E, DD, 4>() : 0;
-    const int lds[3] = {l1, l2, l4};
-    const int kp = key_parts((int64_t)B * Hkv * NHC * range_qtiles(flat, T, Hq / Hkv, NT, 4), lds, tiles, 0.8,
-                             device_cu_count(s));
+    const int kp = fwd_parts<E, DD>(B, Hq, Hkv, T, tiles, s);
     const int nqt = range_qtiles(flat, T, Hq / Hkv, NT, 4 / kp);
     const int64_t grid = (int64_t)B * Hkv * NHC * nqt;
     NSA_CHECK(grid < (1ll << 31), NSA_ERR_SHAPE);
     auto kern = flat ? k_range_fwd32<E, DD, NT, TO, true, 1> : k_range_fwd32<E, DD, NT, TO, false, 1>;
     if (kp == 2) kern = flat ? k_range_fwd32<E, DD, NT, TO, true, 2> : k_range_fwd32<E, DD, NT, TO, false, 2>;
-    if constexpr (l4 > 0)
+    if constexpr (fits_lds(range_fwd_lds<E, DD, 4>()) > 0)
       if (kp == 4) kern = flat ? k_range_fwd32<E, DD, NT, TO, true, 4> : k_range_fwd32<E, DD, NT, TO, false, 4>;
     kern<<<(unsigned)grid, 256, 0, s>>>(mode, (const E*)q, (const E*)k, (const E*)vt, (TO*)o, lse, Hq, Hkv, T, Lk,
                                         Lp, nqt, window, cmp_block, cmp_stride, sl2, fin);
@@ -980,22 +993,17 @@ static int range_dq_launch(int mode, const void* q, const void* k, const void* v
   constexpr int NT = RangeNT<E>::dq;
   const bool flat = Hq / Hkv < 16;   // flat rows: no empty head slots
   NSA_CHECK((int64_t)T * (Hq / Hkv) < (1ll << 31), NSA_ERR_SHAPE);
-  int tiles = mode == NSA_MODE_WINDOW ? ((window < T ? window : T) + 31) / 32 + 1 : (Lk + 31) / 32;
-  if (w2.k != nullptr) tiles += ((window < T ? window : T) + 31) / 32 + 1;
+  int tiles = range_tiles(mode, T, Lk, window);
+  if (w2.k != nullptr) tiles += range_tiles(NSA_MODE_WINDOW, T, T, window);
   NSA_DISPATCH_D(D, {
-    constexpr int l1 = range_dq_lds<E, DD, 1>();
-    constexpr int l2 = range_dq_lds<E, DD, 2>() <= 160 * 1024 ? range_dq_lds<E, DD, 2>() : 0;
-    constexpr int l4 = range_dq_lds<E, DD, 4>() <= 160 * 1024 ? range_dq_lds<E, DD, 4>() : 0;
-    const int lds[3] = {l1, l2, l4};
-    const int kp = key_parts((int64_t)B * Hkv * NHC * range_qtiles(flat, T, Hq / Hkv, NT, 4), lds, tiles, 0.7,
-                             device_cu_count(s));
+    const int kp = dq_parts<E, DD>(B, Hq, Hkv, T, tiles, s);
     const int nqt = range_qtiles(flat, T, Hq / Hkv, NT, 4 / kp);
     const int64_t grid = (int64_t)B * Hkv * NHC * nqt;
     NSA_CHECK(grid < (1ll << 31), NSA_ERR_SHAPE);
     auto kern = flat ? k_range_dq32<E, DD, NT, true, 1> : k_range_dq32<E, DD, NT, false, 1>;
-    if constexpr (l2 > 0)
+    if constexpr (fits_lds(range_dq_lds<E, DD, 2>()) > 0)
       if (kp == 2) kern = flat ? k_range_dq32<E, DD, NT, true, 2> : k_range_dq32<E, DD, NT, false, 2>;
-    if constexpr (l4 > 0)
+    if constexpr (fits_lds(range_dq_lds<E, DD, 4>()) > 0)
       if (kp == 4) kern = flat ? k_range_dq32<E, DD, NT, true, 4> : k_range_dq32<E, DD, NT, false, 4>;
     kern<<<(unsigned)grid, 256, 0, s>>>(mode, (const E*)q, (const E*)k, (const E*)v, (const E*)kt, (const E*)dout,
                                         lse, dot, rowscale, dq, accumulate, Hq, Hkv, T, Lk, Lp, nqt, window,
@@ -1007,6 +1015,25 @@ static int range_dq_launch(int mode, const void* q, const void* k, const void* v
 }
 
 extern "C" {
+
+int nsa_range_key_parts(int pass, int mode, int B, int Hq, int Hkv, int T, int Lk, int D, int window, int dtype,
+                        void* stream) {
+  NSA_CHECK(pass >= 0 && pass <= 2 && (mode == NSA_MODE_WINDOW || mode == NSA_MODE_COMPRESS), NSA_ERR_ARG);
+  NSA_CHECK(B > 0 && Hkv > 0 && Hq > 0 && Hq % Hkv == 0 && T > 0 && Lk >= 0, NSA_ERR_SHAPE);
+  NSA_CHECK((int64_t)T * (Hq / Hkv) < (1ll << 31) && (mode == NSA_MODE_COMPRESS || window >= 1), NSA_ERR_SHAPE);
+  NSA_CHECK(dtype == NSA_F32 || dtype == NSA_BF16, NSA_ERR_DTYPE);
+  hipStream_t s = (hipStream_t)stream;
+  int tiles = range_tiles(mode, T, Lk, window);
+  if (pass == 2) tiles += range_tiles(NSA_MODE_WINDOW, T, T, window);
+  NSA_DISPATCH_D(D, {
+    if (pass == 0)
+      return dtype == NSA_BF16 ? fwd_parts<bf16, DD>(B, Hq, Hkv, T, tiles, s)
+                               : fwd_parts<float, DD>(B, Hq, Hkv, T, tiles, s);
+    return dtype == NSA_BF16 ? dq_parts<bf16, DD>(B, Hq, Hkv, T, tiles, s)
+                             : dq_parts<float, DD>(B, Hq, Hkv, T, tiles, s);
+  });
+  return NSA_ERR_SHAPE;
+}
 
 int nsa_range_fwd(int mode, const void* q, const void* k, const void* vt, void* o, float* lse, int B, int Hq,
                   int Hkv, int T, int Lk, int D, int window, int cmp_block, int cmp_stride, void* q_packed, int dtype,
