@@ -226,8 +226,9 @@ __host__ __device__ inline int64_t csr_place_lds_ints(int n_blk, int S) {
 // The chunk's first slot in each list is the list's start + pos; the starts of
 // bh's lists are the sum of all totals before bh and a scan of its own (or,
 // with own_scan = 0, read from k_csr_base's).  The first chunk's wave writes
-// bh's row of offsets (the last bh's also *count).  Lane q takes query t0 + q: its S indices are staged in LDS and its bit set in the
-// 64-bit query mask of each of its blocks.  A pair of query q on block j then
+// bh's row of offsets (the last bh's also *count).  Lane q takes query t0 + q:
+// its S indices are staged in LDS and its bit set in the 64-bit query mask of
+// each of its blocks.  A pair of query q on block j then
 // lands at run[j] + popcount(mask[j] & bits below q): the pairs of block j
 // from earlier queries of the chunk come first.  A row holding one block
 // twice (an atomicOr that finds its bit already set) makes the chunk take the

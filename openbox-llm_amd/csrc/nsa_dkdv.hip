@@ -1657,9 +1657,9 @@ static KvRange kv_range(int mode, int T, int Lk, int window, int cl, int cd, int
 // the chunks from r.chs on in r.spl sub-chunks while their workgroups fit in
 // one round of the resident workgroups (two per CU of the stream's device).
 // A sequence whose chunks all fit takes as many sub-chunks as fill that
-// round.  With it, the window's parts and flat float tiles, a float32 layer
-// step at B1 T1024 Hq4 Hkv1 D64 takes 892 us instead of 3267: the compression
-// ran on 4 workgroups and the window on 16, three of four tile rows empty.
+// round: with them and flat float tiles the compression of a float32 layer at
+// B1 T1024 Hq4 Hkv1 D64 takes 29 us instead of 1143 (4 workgroups, three of four
+// tile rows empty), with the window's parts the window 41 instead of 1299 (16).
 static int64_t cmp_grid(KvRange& r, hipStream_t s) {
   constexpr int NW = kRangeNW;
   r.chunk = r.T_ < kCmpChunk ? r.T_ : kCmpChunk;

@@ -301,7 +301,8 @@ __device__ __forceinline__ void finish_rows(const FwdExtras<T, TO>& f, const f32
     }
     // selection: merge the slot partials
     float acc_s[8], M, Ls;
-    merge_slots<PartT<T>, D, true>(f.opart, f.ml, f.idx, bh * T_ + t, t, gl, G, f.S, nsub, n_csr, f.sel_L, c8, acc_s, M, Ls);
+    merge_slots<PartT<T>, D, true>(f.opart, f.ml, f.idx, bh * T_ + t, t, gl, G, f.S, nsub, n_csr, f.sel_L, c8, acc_s, M,
+                                   Ls);
     const float inv_s = Ls > 0.0f ? 1.0f / Ls : 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc_s[i] *= inv_s;
@@ -950,7 +951,8 @@ template <typename E, int D> static int fwd_parts(int B, int Hq, int Hkv, int T,
   return key_parts(range_grid1<RangeNT<E>::fwd>(B, Hq, Hkv, T), lds, tiles, 0.8, device_cu_count(s));
 }
 template <typename E, int D> static int dq_parts(int B, int Hq, int Hkv, int T, int tiles, hipStream_t s) {
-  constexpr int lds[3] = {range_dq_lds<E, D, 1>(), fits_lds(range_dq_lds<E, D, 2>()), fits_lds(range_dq_lds<E, D, 4>())};
+  constexpr int lds[3] = {range_dq_lds<E, D, 1>(), fits_lds(range_dq_lds<E, D, 2>()),
+                          fits_lds(range_dq_lds<E, D, 4>())};
   return key_parts(range_grid1<RangeNT<E>::dq>(B, Hq, Hkv, T), lds, tiles, 0.7, device_cu_count(s));
 }
 

@@ -575,7 +575,8 @@ int nsa_sel_fwd_bo(const void* q, const void* k, const void* vt, const int32_t* 
   const size_t cap = sel_items_cap(B, Hkv, T, S, block_size, chunk);
   int4* items = (int4*)workspace;
   int32_t* n_items = (int32_t*)((char*)workspace + cap * sizeof(int4));
-  k_sel_items<<<sel_items_grid(B * Hkv * n_blk), 256, 0, s>>>(block_offsets, B * Hkv * n_blk, n_blk, chunk, items, n_items);
+  const int nb = B * Hkv * n_blk;
+  k_sel_items<<<sel_items_grid(nb), 256, 0, s>>>(block_offsets, nb, n_blk, chunk, items, n_items);
   if (hipGetLastError() != hipSuccess) return NSA_ERR_LAUNCH;
   const int nsub = sel_passes(block_size);
   const size_t grid = cap * nsub < 8192 ? cap * nsub : 8192;

@@ -29,8 +29,8 @@ def _csr(idx, bs, n_blk, packed):
 
 
 # B, Hkv, T, block, S
-SIZES = [(1, 1, 1, 16, 1), (5, 64, 600, 16, 2), (1, 2, 64, 16, 4), (2, 3, 65, 16, 5), (1, 4, 1025, 16, 16), (3, 2, 1040, 16, 3),
-         (1, 1, 16500, 64, 2), (1, 3, 17000, 256, 4), (2, 32, 1100, 16, 2), (70, 2, 500, 16, 2)]
+SIZES = [(1, 1, 1, 16, 1), (5, 64, 600, 16, 2), (1, 2, 64, 16, 4), (2, 3, 65, 16, 5), (1, 4, 1025, 16, 16),
+         (3, 2, 1040, 16, 3), (1, 1, 16500, 64, 2), (1, 3, 17000, 256, 4), (2, 32, 1100, 16, 2), (70, 2, 500, 16, 2)]
 
 
 @pytest.mark.parametrize("c", SIZES, ids=str)

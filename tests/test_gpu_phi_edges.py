@@ -26,7 +26,11 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{str(c[0])[6:]}-B{c[1]}H{c[2]}T{c[3]}D{c[4]}h{c[5]}l{c[6]}d{c[7]}")
+def case_id(c):
+    return f"{str(c[0])[6:]}-B{c[1]}H{c[2]}T{c[3]}D{c[4]}h{c[5]}l{c[6]}d{c[7]}"
+
+
+@pytest.mark.parametrize("case", CASES, ids=case_id)
 def test_phi_edges(case):
     import nsa_hip_ops as ops
     dev = require_gpu()
