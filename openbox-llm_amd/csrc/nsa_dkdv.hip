@@ -761,16 +761,15 @@ template <typename T, int D, int NTH> struct FlatTiles {
     int it;
   };
   FlatReq<T, D, NTH> rq;
-  int rlo, rhi, key, kw, window, cl, cd, h;
-  bool key_ok;
+  int rlo, rhi, kw, window, cl, cd, h;
+  FlatRun run;   // of the lane's key
   __device__ __forceinline__ void prepare(int, int) {}
   __device__ __forceinline__ void issue(KvStage<T, D>& s, int, int) { rq.request(s); }
   __device__ __forceinline__ Info info(const KvStage<T, D>&, int ti) const { return Info{ti}; }
   __device__ __forceinline__ VisBits vis(const Info& i, bool& mask) const {
     const int R0 = rlo + 32 * i.it;
     mask = flat_tile_needs_mask(kw, R0, rhi, rq.G, window, cl, cd);
-    const uint32_t bits = key_ok ? flat_rows_seeing(key, R0, rq.G, window, cl, cd) : 0u;
-    return VisBits{bits >> (8 * h)};
+    return VisBits{flat_run_bits(run, R0) >> (8 * h)};
   }
 };
 
@@ -1059,13 +1058,12 @@ void k_range_dkdv32(const KvRange r, const T* __restrict__ q, const T* __restric
     tiles.rlo = wk.tlo * x.G;
     tiles.rhi = wk.thi * x.G + x.G - 1;
     tiles.rq.init(x, b, hkv, tiles.rlo, wk.thi, tid);
-    tiles.key = key;
     tiles.kw = kw;
     tiles.window = r.mode == NSA_MODE_WINDOW ? r.window : 0;
     tiles.cl = r.cl;
     tiles.cd = r.cd;
     tiles.h = h;
-    tiles.key_ok = key_ok;
+    tiles.run = key_ok ? flat_run(key, x.G, tiles.window, r.cl, r.cd) : FlatRun{0, 0};
     kv_walk<false, 0, T, D, NTH>(acc, stg, tiles, 1, (tiles.rhi - tiles.rlo) / 32 + 1, no_pre, no_post, sl2, tid);
   } else {
     const int ntile = (wk.thi - wk.tlo) / 2 + 1;
@@ -1199,7 +1197,7 @@ void k_range_dkdv_split(const KvRange r, const T* __restrict__ q, const T* __res
   };
   if constexpr (FLAT) {
     // rows tlo G .. thi G + G - 1 of the group; the rows that see a key are
-    // one run (flat_rows_seeing)
+    // one run (flat_run)
     const int G = x.G;
     const int rlo = tlo * G, rhi = thi * G + G - 1;
     auto make_rq = [&]() {
@@ -1208,11 +1206,11 @@ void k_range_dkdv_split(const KvRange r, const T* __restrict__ q, const T* __res
       return rq;
     };
     const int wmode = r.mode == NSA_MODE_WINDOW ? window : 0;
+    const FlatRun seen = key_ok ? flat_run(key, G, wmode, cl, cd) : FlatRun{0, 0};
     auto vis = [&](const KvStage<T, D>&, int it, bool& mask) {
       const int R0 = rlo + 32 * it;
       mask = flat_tile_needs_mask(kw, R0, rhi, G, wmode, cl, cd);
-      const uint32_t bits = key_ok ? flat_rows_seeing(key, R0, G, wmode, cl, cd) : 0u;
-      return VisBits{bits >> (8 * h)};
+      return VisBits{flat_run_bits(seen, R0) >> (8 * h)};
     };
     run(make_rq, (rhi - rlo) / 32 + 1, vis);
   } else {

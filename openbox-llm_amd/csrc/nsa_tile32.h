@@ -267,19 +267,29 @@ static_assert(pair_rows(5, -1, 256).t0 == 5 && pair_rows(5, -1, 256).dB == 0, "n
 //   window (window > 0): key <= t < key + window  <=>  key G <= R < (key + window) G
 //   compression (window = 0): t >= key cd + cl - 1  <=>  R >= (key cd + cl - 1) G
 // (t = floor(R / G) >= m  <=>  R >= m G, and t < m  <=>  R < m G).
-// Returns bit r set for the tile rows r that see the key.  The products are 64
-// bits wide (a window of 2^31 / G no longer fits 32) and cut off past every
-// row: a launch has fewer than 2^27 of them.
+// The products are 64 bits wide (a window of 2^31 / G no longer fits 32) and
+// cut off past every row, of which a launch has fewer than 2^27; a walk forms
+// them once.
 constexpr int kPastRows = 1 << 30;
 __host__ __device__ constexpr int flat_row_bound(int64_t t, int G) {
   return t * G < kPastRows ? (int)(t * G) : kPastRows;
 }
-__host__ __device__ constexpr uint32_t flat_rows_seeing(int key, int R0, int G, int window, int cl, int cd) {
-  int lo = flat_row_bound(window > 0 ? key : (int64_t)key * cd + cl - 1, G) - R0;
-  int hi = window > 0 ? flat_row_bound((int64_t)key + window, G) - R0 : 32;
+struct FlatRun {
+  int lo, hi;   // rows lo .. hi - 1 of the group see the key
+};
+__host__ __device__ constexpr FlatRun flat_run(int key, int G, int window, int cl, int cd) {
+  return FlatRun{flat_row_bound(window > 0 ? key : (int64_t)key * cd + cl - 1, G),
+                 window > 0 ? flat_row_bound((int64_t)key + window, G) : kPastRows};
+}
+// bit r set for the rows r of the tile at R0 that are in the run
+__host__ __device__ constexpr uint32_t flat_run_bits(FlatRun run, int R0) {
+  int lo = run.lo - R0, hi = run.hi - R0;
   lo = lo < 0 ? 0 : (lo > 32 ? 32 : lo);
   hi = hi < 0 ? 0 : (hi > 32 ? 32 : hi);
   return lo < hi ? (uint32_t)(((1ull << hi) - 1ull) & ~((1ull << lo) - 1ull)) : 0u;
+}
+__host__ __device__ constexpr uint32_t flat_rows_seeing(int key, int R0, int G, int window, int cl, int cd) {
+  return flat_run_bits(flat_run(key, G, window, cl, cd), R0);
 }
 // Whether a flat tile needs the per-element test for the 32 keys kw ..
 // kw + 31: false only when every one of them is seen by every row of the
