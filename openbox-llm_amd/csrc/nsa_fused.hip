@@ -143,8 +143,15 @@ BwdScratch carve_bwd(const Dims& m, void* base, size_t* bytes, hipStream_t s) {
   x.sel_part_bytes = nsa_sel_dkdv_partial_bytes(m.B, m.Hkv, m.T, S, m.D, m.ls, m.dkdv_chunk());
   x.sel_part = (float*)c.take(x.sel_part_bytes);
   size_t end = c.off;
-  c.off = branch;   // the window's parts (0 bytes where it is not split)
+  // The window's parts (0 bytes where it is not split).  They are written right
+  // after the selection's parts are read; over the same memory that costs a
+  // short bf16 layer, forward and backward, 3 to 6 us (T512: D128 Hkv2 186 ->
+  // 190, 8 sequences 243 -> 249, D64 G6 200 -> 204), so up to 24 MiB are laid out
+  // apart.  Float32 is level either way (266 us at T512 D64 G4), and so is bf16
+  // from 26.7 MB on (355 us at T1500 D128 G16).
   x.win_part_bytes = nsa_range_dkdv_partial_bytes(NSA_MODE_WINDOW, m.B, m.Hkv, m.T, m.T, m.D, m.window, 1, s);
+  const bool apart = m.dtype == NSA_BF16 && x.win_part_bytes <= ((size_t)24 << 20);
+  c.off = apart ? end : branch;
   x.win_part = x.win_part_bytes > 0 ? (float*)c.take(x.win_part_bytes) : nullptr;
   end = c.off > end ? c.off : end;
   c.off = branch;
